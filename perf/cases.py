@@ -156,6 +156,7 @@ def prepare(case, seed):
     else:
         cfg = dict(qwen3_0p6b(max_seq=1024), num_layers=case["layers"])
         s["model"] = Qwen(cfg, seed=int(seed) % 1000003 + 1)
+        s["model"].set_decode_mode(1)
     return s
 
 
