@@ -11,7 +11,6 @@ constexpr int LM_THREADS = 256;
 constexpr int LM_ROWS_PER_WAVE = 64;
 constexpr int LM_KC = 64;                 // k-values staged per step
 constexpr int LM_ROW_STRIDE = LM_KC * 2 + 16;  // bytes per staged row (+16 pad)
-constexpr int LM_MR = 4;                  // activation rows per pass
 constexpr int LM_MAX_K = 8192;
 
 __device__ __forceinline__ h2v as_h2(uint32_t u) { return __builtin_bit_cast(h2v, u); }

@@ -272,6 +272,24 @@ def test_matmul_f16(dev, orc, M, K, N):
     assert_bits(dev.get(c, np.uint16, (M, N)), orc.matmul_f16(a, b), "matmul_f16")
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (1, 8, 15), (2, 264, 17), (4, 8192, 129), (3, 512, 64),            # rows kernel: stage and tile edges, largest K
+    (5, 8, 1), (9, 136, 63), (33, 1160, 65), (31, 128, 130),           # tile kernel, 2 rows per wave
+    (16, 264, 16385), (70, 120, 8200),                                 # 4 rows per wave
+    (65, 72, 33000), (2049, 16, 1030)])                                # 8 rows per wave
+def test_matmul_f16_tiles(dev, orc, M, K, N):
+    """Edges of the row counts, column tiles and k stages of the FP16 matmul."""
+    say("matmul_f16 tiles", M, K, N)
+    rng = np.random.default_rng(M * 7 + K + N)
+    a = f16(rng.normal(0, 1, (M, K)))
+    b = f16(rng.normal(0, 0.05, (N, K)))
+    c = dev.put(np.full((M, N), 0x7E01, np.uint16))
+    dev.cm.call("cactus_hip_matmul_f16", dev.put(a), dev.put(b), c, M, K, N, None)
+    got = np.empty((M, N), np.uint16)
+    dev.cm.call("cactus_hip_memcpy_d2h", got.ctypes.data, c, got.nbytes, None)
+    assert_bits(got, orc.matmul_f16(a, b), "matmul_f16")
+
+
 def test_lm_head_argmax_qwen_vocab(dev, orc):
     say("lm_head_argmax K=1024 N=151936")
     rng = np.random.default_rng(6)
