@@ -19,6 +19,9 @@
 //      expf, an order-preserving compaction, then thread 0 sums, normalises
 //      and walks the running sum to the first value >= u, and appends the
 //      token to the device-resident history.
+// With a top-k small against the vocabulary the passes over the vocabulary run
+// in many workgroups instead (sample_filter_kernel) and one workgroup
+// finishes over their few candidates (sample_finish).
 // The sequential float sums run by one thread over the survivors only
 // (probabilities of removed tokens are exactly 0 and add nothing), so with
 // top-k they are short; without any filter they cover the vocabulary.
@@ -91,6 +94,9 @@ struct SampleArgs {
     uint16_t inv_t;     // fp16(1/T)
     uint16_t pen_inv, pen;
     int scale;          // temperature > 0
+    unsigned long long* blk;   // [nblk][SF_TOK] candidates of each filter workgroup (nblk = 0: not run)
+    uint32_t* blk_n;           // [nblk] their counts
+    int nblk;
 };
 
 // order-preserving key of an fp16 value (non-NaN; -0 folded onto +0)
@@ -275,6 +281,263 @@ __device__ void topp_large(const Ops& ops, size_t V, float top_p, uint32_t* sk, 
     __syncthreads();
 }
 
+// ---------------------------------------------------------------- small top-k
+// Phases 1 and 2 over the vocabulary, spread over the chip: a workgroup takes
+// SF_TOK tokens, applies temperature and repetition penalty and keeps the
+// values at or above its own k-th largest: a superset of the vocabulary's top
+// k (ties included), since no part's k-th largest exceeds the whole's.  The
+// threshold is found bit by bit on the 16-bit order keys with ballot counts;
+// an LDS histogram serialises on the few bins that logits share.
+// 151936 logits, top_k 20, top_p 0.95: 302-329 us in one workgroup before
+// (eight passes over the vocabulary at one CU's load latency), 6 us here and
+// 21 us in the finishing workgroup.
+constexpr int SF_T = 512;
+constexpr int SF_TOK = 2048;           // tokens per workgroup
+constexpr int SF_CAND = SP_CAND * 3 / 4;   // candidates expected at most: the rest of the LDS takes the survivors
+
+// candidates sort ascending by (descending value, ascending token)
+__device__ __forceinline__ unsigned long long cand_entry(uint32_t key, uint32_t token) {
+    return ((unsigned long long)(0xFFFFu - key) << 32) | token;
+}
+__device__ __forceinline__ uint32_t cand_key(unsigned long long e) { return 0xFFFFu - (uint32_t)(e >> 32); }
+
+// The largest 16-bit threshold that at least k of the workgroup's keys reach.
+// count(t): how many of this wave's keys are >= t (uniform over the wave).
+template <int NWAVE, class Count>
+__device__ __forceinline__ uint32_t kth_key(uint32_t k, uint32_t (*part)[NWAVE], Count count) {
+    const int wid = threadIdx.x >> 6;
+    uint32_t t = 0;
+    for (int bit = 15; bit >= 0; bit--) {
+        const uint32_t c = t | (1u << bit);
+        const uint32_t n = count(c);
+        if ((threadIdx.x & 63) == 0) part[bit & 1][wid] = n;   // two buffers: one barrier per bit
+        __syncthreads();
+        uint32_t sum = 0;
+#pragma unroll
+        for (int w = 0; w < NWAVE; w++) sum += part[bit & 1][w];
+        if (sum >= k) t = c;
+    }
+    return t;
+}
+
+__global__ void __launch_bounds__(SF_T) sample_filter_kernel(SampleArgs a) {
+    constexpr int PER = SF_TOK / SF_T;
+    __shared__ uint16_t val[SF_TOK];
+    __shared__ uint32_t hist[SP_HIST];
+    __shared__ uint32_t part[2][SF_T / 64];
+    __shared__ uint32_t kept;
+    const int tid = threadIdx.x;
+    const size_t base = (size_t)blockIdx.x * SF_TOK;
+    const int ntok = (int)(a.V - base < (size_t)SF_TOK ? a.V - base : (size_t)SF_TOK);
+    const int nh = (int)a.hist[0];
+    uint16_t h[PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++) h[i] = a.logits[base + min(tid + i * SF_T, ntok - 1)];
+    if (tid < nh) hist[tid] = a.hist[1 + tid];
+#pragma unroll
+    for (int i = 0; i < PER; i++) val[tid + i * SF_T] = a.scale ? hmul(h[i], a.inv_t) : h[i];
+    if (tid == 0) kept = 0;
+    __syncthreads();
+    // the penalty is applied once per history entry of the token; its repeats
+    // compute the same product again, so the first entry's thread does them all
+    if (tid < nh && (size_t)hist[tid] >= base && (size_t)hist[tid] < base + ntok) {
+        const uint32_t t = hist[tid];
+        uint16_t v = val[t - base];
+        bool first = true;
+        for (int j = 0; j < tid; j++) first = first && hist[j] != t;
+        if (first) {
+            for (int j = tid; j < nh; j++)
+                if (hist[j] == t) v = h2f(v) > 0.0f ? hmul(v, a.pen_inv) : hmul(v, a.pen);
+            val[t - base] = v;
+        }
+    }
+    __syncthreads();
+    uint32_t key[PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        h[i] = val[tid + i * SF_T];
+        key[i] = okey(h[i]);
+    }
+    const uint32_t t = kth_key<SF_T / 64>((uint32_t)a.top_k, part, [&](uint32_t c) {
+        uint32_t n = 0;
+#pragma unroll
+        for (int i = 0; i < PER; i++) n += __popcll(__ballot(tid + i * SF_T < ntok && key[i] >= c));
+        return n;
+    });
+    unsigned long long* out = a.blk + (size_t)blockIdx.x * SF_TOK;
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+        if (tid + i * SF_T < ntok && key[i] >= t)
+            out[atomicAdd(&kept, 1u)] = ((unsigned long long)(h[i] == SP_NEG_INF) << 63) |
+                                        cand_entry(key[i], (uint32_t)(base + tid + i * SF_T));
+    __syncthreads();
+    if (tid == 0) a.blk_n[blockIdx.x] = kept;
+}
+
+// ascending bitonic sort of x[0, n2) in LDS, n2 a power of two
+__device__ __forceinline__ void bitonic_sort_lds(unsigned long long* x, uint32_t n2) {
+    for (uint32_t size = 2; size <= n2; size <<= 1) {
+        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+            for (uint32_t p = threadIdx.x; p < n2 / 2; p += blockDim.x) {
+                const uint32_t lo = 2 * p - (p & (stride - 1)), hi = lo + stride;
+                const bool up = (lo & size) == 0;
+                const unsigned long long u = x[lo], v = x[hi];
+                if ((u > v) == up) {
+                    x[lo] = v;
+                    x[hi] = u;
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// Phases 2 to 4 over the filter's candidates, all in LDS: the vocabulary's
+// k-th largest key among them, the survivors sorted for the top-p cut, then
+// sorted by token for the draw.  Every exponential and quotient is computed
+// in parallel; thread 0 only adds, in the reference's order.  Returns false,
+// having written nothing, when ties leave more candidates than the LDS holds.
+__device__ bool sample_finish(const SampleArgs& a, unsigned long long* cand, uint32_t* scan, float* red,
+                              uint32_t* sh_u32) {
+    const uint32_t tid = threadIdx.x;
+    uint32_t(*part)[SP_T / 64] = reinterpret_cast<uint32_t(*)[SP_T / 64]>(scan);
+    if (tid == 0) sh_u32[0] = sh_u32[1] = 0;
+    __syncthreads();
+    uint32_t E = 1;
+    while (E < a.top_k && E < (uint32_t)SF_TOK) E <<= 1;
+    const uint32_t slots = (uint32_t)a.nblk * E;
+    for (uint32_t s = tid; s < slots; s += SP_T) {
+        const uint32_t b = s / E, n = a.blk_n[b];
+        unsigned long long v = a.blk[(size_t)b * SF_TOK + (s & (E - 1))];
+        for (uint32_t e = s & (E - 1); e < n; e += E) {   // past E: values tied with the workgroup's k-th
+            if (e >= E) v = a.blk[(size_t)b * SF_TOK + e];
+            const uint32_t o = atomicAdd(&sh_u32[0], 1u);
+            if (o < (uint32_t)SP_CAND) cand[o] = v;
+        }
+    }
+    __syncthreads();
+    const uint32_t nc = sh_u32[0];
+    if (nc > (uint32_t)SP_CAND) return false;
+    const uint32_t kth = kth_key<SP_T / 64>((uint32_t)a.top_k, part, [&](uint32_t c) {
+        uint32_t n = 0;
+        for (uint32_t i0 = 0; i0 < nc; i0 += SP_T) {
+            const uint32_t i = i0 + tid;
+            n += __popcll(__ballot(i < nc && cand_key(cand[min(i, nc - 1)] & ~(1ull << 63)) >= c));
+        }
+        return n;
+    });
+    // survivors behind the candidates (values of -inf count towards the top k
+    // and are gone here)
+    for (uint32_t i = tid; i < nc; i += SP_T) {
+        const unsigned long long v = cand[i];
+        if (!(v >> 63) && cand_key(v) >= kth) {
+            const uint32_t o = nc + atomicAdd(&sh_u32[1], 1u);
+            if (o < (uint32_t)SP_CAND) cand[o] = v;
+        }
+    }
+    __syncthreads();
+    uint32_t n = sh_u32[1], n2 = 1;
+    while (n2 < n) n2 <<= 1;
+    // the sort's padding and two floats per survivor follow them
+    if (n == 0) {
+        if (tid == 0) *a.out = 0;
+        return true;
+    }
+    if (nc + 2 * n2 > (uint32_t)SP_CAND) return false;
+    unsigned long long* sv = cand + nc;
+    float* pv = reinterpret_cast<float*>(sv + n2);
+    for (uint32_t j = n + tid; j < n2; j += SP_T) sv[j] = ~0ull;
+    __syncthreads();
+    if (a.top_p > 0.0f && a.top_p < 1.0f) {
+        bitonic_sort_lds(sv, n2);
+        const float mx = h2f(ukey(cand_key(sv[0])));
+        for (uint32_t j = tid; j < n; j += SP_T) pv[j] = cactus_expf(h2f(ukey(cand_key(sv[j]))) - mx);
+        __syncthreads();
+        if (tid == 0) {
+            float sum = 0.0f;
+            for (uint32_t j = 0; j < n; j++) sum += pv[j];
+            red[0] = sum;
+        }
+        __syncthreads();
+        const float sum = red[0];
+        for (uint32_t j = tid; j < n; j += SP_T) pv[j] = pv[j] / sum;
+        __syncthreads();
+        if (tid == 0) {
+            uint32_t cut = n;
+            float cum = 0.0f;
+            for (uint32_t j = 0; j < n; j++) {
+                cum += pv[j];
+                if (cum > a.top_p && j > 0) {
+                    cut = j;
+                    break;
+                }
+            }
+            sh_u32[2] = cut;
+        }
+        __syncthreads();
+        n = sh_u32[2];
+    }
+    // the draw, in token order
+    float m = -__builtin_inff();
+    for (uint32_t j = tid; j < n2; j += SP_T) {
+        if (j < n) {
+            const uint32_t key = cand_key(sv[j]);
+            m = __builtin_fmaxf(m, h2f(ukey(key)));
+            sv[j] = ((sv[j] & 0xFFFFFFFFull) << 32) | key;
+        } else {
+            sv[j] = ~0ull;
+        }
+    }
+    m = wave_max(m);
+    if ((tid & 63) == 0) red[tid >> 6] = m;
+    __syncthreads();
+    float mx = red[0];
+    for (int w = 1; w < SP_T / 64; w++) mx = __builtin_fmaxf(mx, red[w]);
+    if (mx == -__builtin_inff()) {
+        if (tid == 0) *a.out = 0;
+        return true;
+    }
+    bitonic_sort_lds(sv, n2);
+    for (uint32_t j = tid; j < n; j += SP_T) pv[j] = cactus_expf(h2f(ukey((uint32_t)sv[j] & 0xFFFFu)) - mx);
+    const uint32_t nh = a.hist[0];
+    const uint32_t next = tid + 2 <= (uint32_t)SP_HIST ? a.hist[tid + 2] : 0u;
+    __syncthreads();
+    if (tid == 0) {
+        float sum = 0.0f;
+        for (uint32_t j = 0; j < n; j++) sum += pv[j];
+        red[0] = sum;
+    }
+    __syncthreads();
+    const float sum = red[0];
+    if (sum == 0.0f) {
+        if (tid == 0) *a.out = 0;
+        return true;
+    }
+    for (uint32_t j = tid; j < n; j += SP_T) pv[j] = pv[j] / sum;
+    __syncthreads();
+    if (nh == (uint32_t)SP_HIST && tid + 2 <= (uint32_t)SP_HIST) a.hist[tid + 1] = next;   // every read is done
+    if (tid != 0) return true;
+    uint32_t tok = 0;
+    bool found = false;
+    if (a.u <= 0.0f) {
+        found = true;   // the running sum is >= u already at token 0
+    } else {
+        float cum = 0.0f;
+        for (uint32_t j = 0; j < n && !found; j++) {
+            cum += pv[j];
+            if (cum >= a.u) { tok = (uint32_t)(sv[j] >> 32); found = true; }
+        }
+        for (uint32_t j = n; j > 0 && !found; j--)
+            if (pv[j - 1] > 0.0f) { tok = (uint32_t)(sv[j - 1] >> 32); found = true; }
+    }
+    // history (:633-650)
+    const uint32_t at = nh == (uint32_t)SP_HIST ? (uint32_t)SP_HIST - 1 : nh;
+    a.hist[1 + at] = tok;
+    a.hist[0] = at + 1;
+    *a.out = tok;
+    return true;
+}
+
 __global__ void __launch_bounds__(SP_T) sample_kernel(SampleArgs a) {
     extern __shared__ unsigned long long cand[];   // [SP_CAND], dynamic: 128 KB
     __shared__ uint32_t hbin[256];
@@ -283,6 +546,8 @@ __global__ void __launch_bounds__(SP_T) sample_kernel(SampleArgs a) {
     __shared__ uint32_t sh_u32[4];
     const int tid = threadIdx.x;
     const size_t V = a.V;
+    if (a.nblk > 0 && sample_finish(a, cand, scan, red, sh_u32)) return;
+    __syncthreads();
 
     // 1. temperature, then the repetition penalty (kernel_nn.cpp:501-529)
     for (size_t i = tid; i < V; i += SP_T) a.f[i] = a.scale ? hmul(a.logits[i], a.inv_t) : a.logits[i];
@@ -741,6 +1006,8 @@ struct SampleState {
     float* pv = nullptr;
     uint32_t* surv = nullptr;
     uint32_t* sk = nullptr;
+    unsigned long long* blk = nullptr;
+    uint32_t* blk_n = nullptr;
     size_t cap = 0;
     uint32_t* hist = nullptr;
 };
@@ -764,7 +1031,10 @@ static int sample_state(size_t V, SampleState** out) {
         if (s.surv) CH_HIP(hipFree(s.surv));
         if (s.f32) CH_HIP(hipFree(s.f32));
         if (s.sk) CH_HIP(hipFree(s.sk));
+        if (s.blk) CH_HIP(hipFree(s.blk));
+        if (s.blk_n) CH_HIP(hipFree(s.blk_n));
         s.f = nullptr; s.pv = nullptr; s.surv = nullptr; s.f32 = nullptr; s.sk = nullptr; s.cap = 0;
+        s.blk = nullptr; s.blk_n = nullptr;
         CH_HIP(hipMalloc(&s.f, V * sizeof(uint16_t)));
         CH_HIP(hipMalloc(&s.pv, V * sizeof(float)));
         CH_HIP(hipMalloc(&s.surv, V * sizeof(uint32_t)));
@@ -772,6 +1042,9 @@ static int sample_state(size_t V, SampleState** out) {
         size_t n2 = 1;
         while (n2 < V) n2 <<= 1;
         CH_HIP(hipMalloc(&s.sk, n2 * sizeof(uint32_t)));
+        const size_t nblk = ceil_div(V, SF_TOK);
+        CH_HIP(hipMalloc(&s.blk, nblk * SF_TOK * sizeof(unsigned long long)));
+        CH_HIP(hipMalloc(&s.blk_n, nblk * sizeof(uint32_t)));
         s.cap = V;
     }
     *out = &s;
@@ -824,6 +1097,18 @@ int cactus_hip_sample_f16(const uint16_t* logits, uint32_t* out, size_t vocab, f
     static const hipError_t attr =
         hipFuncSetAttribute((const void*)sample_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     CH_REQUIRE(attr == hipSuccess, "sample: cannot reserve the candidate LDS");
+    // a top-k whose candidates (k of each workgroup) are few enough for the
+    // finishing workgroup's LDS is filtered by many workgroups first (the
+    // limit: 163 at 151936 logits)
+    const size_t nblk = ceil_div(vocab, SF_TOK);
+    if (top_k > 0 && top_k < vocab && top_k <= (size_t)SF_CAND / nblk) {
+        a.blk = s->blk;
+        a.blk_n = s->blk_n;
+        a.nblk = (int)nblk;
+        hipLaunchKernelGGL(sample_filter_kernel, dim3((unsigned)nblk), dim3(SF_T), 0, as_stream(stream), a);
+        rc = check_launch("sample (filter)");
+        if (rc) return rc;
+    }
     hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(SP_T), lds, as_stream(stream), a);
     return check_launch("sample");
 }

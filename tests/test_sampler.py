@@ -190,6 +190,38 @@ def test_sampler_ties(hip_ready, orc):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("vocab,cfg", [
+    (2048, (0.7, 0.9, 1)), (2049, (0.7, 0.0, 2048)), (4097, (0.9, 0.95, 4096)),   # tile edges, whole tiles kept
+    (151936, (0.8, 0.9, 163)), (151936, (0.8, 0.9, 164)),                         # both sides of the candidate limit
+    (6000, (0.0, 0.8, 50))])
+def test_sampler_filtered_top_k(hip_ready, orc, vocab, cfg):
+    """The top-k filter over many workgroups: a history longer than its 128
+    entries with repeats, masked logits, ties and more masked than kept."""
+    cm = hip_ready
+    run, history = _gpu_sampler(cm)
+    cm.call("cactus_hip_sample_history_reset", None)
+    s = orc.OracleSampler()
+    rng = np.random.default_rng(vocab + cfg[2])
+    say("sampler filtered top-k", vocab, cfg)
+    peak = rng.integers(0, vocab, 12)
+    for step in range(140):
+        x = np.round(rng.normal(0, 2, vocab) * 8) / 8
+        x[peak] += 9.0                         # the same few tokens over and over: repeated penalties
+        x[rng.integers(0, vocab, vocab // 3)] = -np.inf
+        if step % 20 == 7:
+            x[:] = -np.inf
+            x[rng.integers(0, vocab, 3)] = 1.0   # fewer live logits than top_k
+        if step == 27:
+            x[:] = -np.inf
+        x = f16(x)
+        seed = int(rng.integers(1, 2**31))
+        rc, got = run(x, *cfg, seed)
+        assert rc == 0
+        assert got == s.sample(x, *cfg, seed), step
+    assert (history() == s.history()).all() and len(history()) == 128
+
+
+@pytest.mark.gpu
 def test_sampler_large_top_p(hip_ready, orc):
     """More top-p candidates than the LDS sort holds (16384): top-p with
     top_k 0 on 151936 logits, a flat row of 20000 ties (top-k 10 keeps every
