@@ -2,6 +2,7 @@
 // fp16 add/multiply (a12) and the embedding gather (a13).
 #include "decode_device.h"
 #include "hip_common.h"
+#include "pointwise_device.h"
 
 #include <cmath>
 #include <map>
@@ -13,10 +14,11 @@ namespace cactus_hip {
 
 // ---------------------------------------------------------------- RMSNorm
 // One wave per row.  The row is staged in LDS; lanes 0..15 each run one of
-// the reference's 16 fp32 FMA chains (element i -> chain i mod 16, i.e.
-// accumulator (i%16)/4, lane i%4, kernel_attention.cpp:500-523), which are
-// combined as ((v0+v1)+v2)+v3 per lane and then (l0+l1)+(l2+l3) (:525-530).
-// Output: y = fp16(fp16(x * fp16(1/rms)) * w) on the 8-aligned prefix.
+// the reference's 16 fp32 FMA chains (rms_stats_wave, kernel_attention.cpp:
+// 500-538).  Output: y = fp16(fp16(x * fp16(1/rms)) * w) on the 8-aligned
+// prefix.  Rows of 8-value chunks at 16-byte addresses move as 16-byte loads
+// and stores, all of a lane's loads of a row in flight together: the chains
+// bound the row then, not the two-byte loads in front of them.
 constexpr int RMS_MAX_DIMS = 8192;
 
 __global__ void __launch_bounds__(256) rms_norm_kernel(const uint16_t* __restrict__ X,
@@ -26,47 +28,46 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const uint16_t* __restric
     extern __shared__ __align__(16) uint16_t srow[];
     const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const size_t row = (size_t)blockIdx.x * 4 + wid;
-    uint16_t* xs = srow + wid * dims;
-    const bool active = row < rows;
+    if (row >= rows) return;   // the whole wave: no workgroup barrier below
+    uint16_t* xs = srow + wid * ((dims + 7) & ~7);
     const uint16_t* x = X + row * dims;
-    if (active)
-        for (int i = lane; i < dims; i += 64) xs[i] = x[i];
-    __syncthreads();
-    float ss = 0.0f;
-    float chain = 0.0f;
-    const int n16 = dims / 16;
+    uint16_t* y = Y + row * dims;
+    float inv;
+    uint16_t hinv;
+    if ((dims & 7) == 0 && (((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) & 15) == 0) {
+        const int nch = dims / 8;
+        const i32x4* x4 = reinterpret_cast<const i32x4*>(x);
+        const i32x4* w4 = reinterpret_cast<const i32x4*>(W);
+        i32x4* xs4 = reinterpret_cast<i32x4*>(xs);
+        for (int c0 = 0; c0 < nch; c0 += 256) {
+            i32x4 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = x4[min(c0 + 64 * j + lane, nch - 1)];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (c0 + 64 * j + lane < nch) xs4[c0 + 64 * j + lane] = v[j];
+        }
+        wave_lds_order();
+        rms_stats_wave(xs, dims, eps, inv, hinv);
+        for (int c = lane; c < nch; c += 64) {
+            const i32x4 v = xs4[c], w = w4[c];
+            i32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t xv = (uint32_t)v[e], wv = (uint32_t)w[e];
+                const uint32_t lo = hmul(hmul((uint16_t)(xv & 0xFFFFu), hinv), (uint16_t)(wv & 0xFFFFu));
+                const uint32_t hi = hmul(hmul((uint16_t)(xv >> 16), hinv), (uint16_t)(wv >> 16));
+                o[e] = (int)(lo | (hi << 16));
+            }
+            reinterpret_cast<i32x4*>(y)[c] = o;
+        }
+        return;
+    }
+    for (int i = lane; i < dims; i += 64) xs[i] = x[i];
+    wave_lds_order();
+    rms_stats_wave(xs, dims, eps, inv, hinv);
     const int end8 = (dims / 8) * 8;
-    if (active && lane < 16) {
-        for (int i = 0; i < n16; i++) {
-            const float a = h2f(xs[i * 16 + lane]);
-            chain = __builtin_fmaf(a, a, chain);
-        }
-        if (lane < 8 && n16 * 16 + 8 <= dims) {
-            const float a = h2f(xs[n16 * 16 + lane]);
-            chain = __builtin_fmaf(a, a, chain);
-        }
-    }
-    const float c4 = __shfl(chain, (lane + 4) & 63, 64);
-    const float c8 = __shfl(chain, (lane + 8) & 63, 64);
-    const float c12 = __shfl(chain, (lane + 12) & 63, 64);
-    const float t = ((chain + c4) + c8) + c12;
-    const float t1 = __shfl(t, 1, 64), t2 = __shfl(t, 2, 64), t3 = __shfl(t, 3, 64);
-    const float t0 = __shfl(t, 0, 64);
-    ss = (t0 + t1) + (t2 + t3);
-    for (int k = end8; k < dims; k++) {
-        const float a = h2f(xs[k]);
-        ss = __builtin_fmaf(a, a, ss);
-    }
-    const float rms = __builtin_sqrtf(ss / (float)dims + eps);
-    const float inv = 1.0f / rms;
-    const uint16_t hinv = f2h(inv);
-    if (active) {
-        uint16_t* y = Y + row * dims;
-        for (int i = lane; i < dims; i += 64) {
-            if (i < end8) y[i] = hmul(hmul(xs[i], hinv), W[i]);
-            else y[i] = f2h((h2f(xs[i]) * inv) * h2f(W[i]));
-        }
-    }
+    for (int i = lane; i < dims; i += 64) y[i] = rms_apply(xs[i], W[i], i, end8, inv, hinv);
 }
 
 // ---------------------------------------------------------------- RoPE
@@ -261,30 +262,20 @@ __global__ void __launch_bounds__(256) rms_rope_rows_kernel(RopeRowsArgs a) {
     }
 }
 
-__global__ void silu_kernel(const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, size_t n) {
-    const size_t body = (n / 8) * 8;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const float x = h2f(X[i]);
-        const float e = (i < body) ? fast_exp(-x) : cactus_expf(-x);
+struct SiluOp {
+    __device__ uint16_t operator()(uint16_t a, uint16_t, bool body) const {
+        const float x = h2f(a);
+        const float e = body ? fast_exp(-x) : cactus_expf(-x);
         const float sig = 1.0f / (1.0f + e);
-        Y[i] = f2h(x * sig);
+        return f2h(x * sig);
     }
-}
-
-__global__ void add_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
-                           uint16_t* __restrict__ Y, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x)
-        Y[i] = hadd(A[i], B[i]);
-}
-
-__global__ void mul_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
-                           uint16_t* __restrict__ Y, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x)
-        Y[i] = hmul(A[i], B[i]);
-}
+};
+struct AddOp {
+    __device__ uint16_t operator()(uint16_t a, uint16_t b, bool) const { return hadd(a, b); }
+};
+struct MulOp {
+    __device__ uint16_t operator()(uint16_t a, uint16_t b, bool) const { return hmul(a, b); }
+};
 
 // ---------------------------------------------------------------- transpose
 __global__ void transpose_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
@@ -339,7 +330,7 @@ int cactus_hip_rms_norm_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, s
     CH_REQUIRE(x && w && y, "rms_norm: null pointer");
     CH_REQUIRE(dims <= (size_t)RMS_MAX_DIMS, "rms_norm: dims > 8192 not supported");
     CH_REQUIRE(rows < (1ull << 33), "rms_norm: too many rows");
-    const size_t smem = 4 * dims * sizeof(uint16_t);
+    const size_t smem = 4 * ((dims + 7) & ~(size_t)7) * sizeof(uint16_t);
     hipLaunchKernelGGL(rms_norm_kernel, dim3(ceil_div(rows, 4)), dim3(256), smem, as_stream(stream),
                        x, w, y, rows, (int)dims, eps);
     return check_launch("rms_norm");
@@ -417,23 +408,20 @@ int cactus_hip_softmax_f16(const uint16_t* x, uint16_t* y, size_t batch, size_t 
 int cactus_hip_silu_f16(const uint16_t* x, uint16_t* y, size_t n, void* stream) {
     if (n == 0) return CACTUS_HIP_OK;
     CH_REQUIRE(x && y, "silu: null pointer");
-    hipLaunchKernelGGL(silu_kernel, dim3(grid_for(n, 256)), dim3(256), 0, as_stream(stream), x, y, n);
-    return check_launch("silu");
+    return launch_pointwise<false>("silu", x, nullptr, y, n, stream, SiluOp{});
 }
 
 int cactus_hip_add_f16(const uint16_t* a, const uint16_t* b, uint16_t* y, size_t n, void* stream) {
     if (n == 0) return CACTUS_HIP_OK;
     CH_REQUIRE(a && b && y, "add: null pointer");
-    hipLaunchKernelGGL(add_kernel, dim3(grid_for(n, 256)), dim3(256), 0, as_stream(stream), a, b, y, n);
-    return check_launch("add");
+    return launch_pointwise<true>("add", a, b, y, n, stream, AddOp{});
 }
 
 int cactus_hip_multiply_f16(const uint16_t* a, const uint16_t* b, uint16_t* y, size_t n,
                             void* stream) {
     if (n == 0) return CACTUS_HIP_OK;
     CH_REQUIRE(a && b && y, "multiply: null pointer");
-    hipLaunchKernelGGL(mul_kernel, dim3(grid_for(n, 256)), dim3(256), 0, as_stream(stream), a, b, y, n);
-    return check_launch("multiply");
+    return launch_pointwise<true>("multiply", a, b, y, n, stream, MulOp{});
 }
 
 int cactus_hip_transpose_2d_f16(const uint16_t* src, uint16_t* dst, size_t rows, size_t cols,

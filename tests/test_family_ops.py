@@ -133,7 +133,25 @@ def test_gelu_matches_oracle(hip_ready, orc, n):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,F", [(1, 1280), (37, 384), (1500, 1280), (3, 7)])
+def test_gelu_erf_every_input(hip_ready, orc):
+    """Every fp16 value, at an aligned and at an odd address."""
+    cm = hip_ready
+    x = np.arange(65536, dtype=np.uint16)
+    want = orc.gelu_erf(x)
+    nan = np.isnan(want.view(np.float16))
+    say("gelu_erf every input")
+    for off in (0, 1):
+        d = _dev(cm, np.concatenate([np.zeros(off, np.uint16), x]))
+        o = cm.DeviceBuffer(x.nbytes)
+        cm.call("cactus_hip_gelu_erf_f16", d.ptr + 2 * off, o.ptr, x.size, None)
+        got = _get(cm, o, want)
+        assert (got[~nan] == want[~nan]).all()
+        assert np.isnan(got[nan].view(np.float16)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,F", [(1, 1280), (37, 384), (1500, 1280), (3, 7), (5, 15), (4, 16), (9, 2056),
+                                    (2, 4084), (3, 4085), (1, 1)])
 def test_layer_norm_matches_oracle(hip_ready, orc, rows, F):
     cm = hip_ready
     rng = np.random.default_rng(rows + F)

@@ -256,6 +256,34 @@ def test_unpack_int4(dev, orc):
 
 
 # ------------------------------------------------------------------ a4
+@pytest.mark.parametrize("n,off", [(1, 0), (8, 0), (2055, 0), (2055, 1), (70000, 3)])
+def test_pointwise_edges(dev, orc, n, off):
+    """add, multiply and silu at chunk remainders and off 16-byte addresses."""
+    say("pointwise", n, off)
+    rng = np.random.default_rng(n + off)
+    a, b = (f16(rng.normal(0, 2, n)) for _ in range(2))
+    pad = np.zeros(off, np.uint16)
+    pa, pb = dev.put(np.concatenate([pad, a])) + 2 * off, dev.put(np.concatenate([pad, b])) + 2 * off
+    out = dev.put(np.zeros(n + off + 1, np.uint16))
+    for name, args, want in (("add", (pa, pb), orc.add(a, b)), ("multiply", (pa, pb), orc.multiply(a, b)),
+                             ("silu", (pa,), orc.silu(a))):
+        dev.cm.call("cactus_hip_%s_f16" % name, *args, out + 2 * off, n, None)
+        got = dev.get_ptr(out, np.uint16, n + off + 1)
+        assert_bits(got[off:off + n], want, name)
+        assert got[off + n] == 0
+
+
+@pytest.mark.parametrize("rows,dims,off", [(1, 8, 0), (5, 24, 0), (3, 2056, 0), (2, 8192, 0), (4, 129, 0), (3, 1024, 1)])
+def test_rms_norm_edges(dev, orc, rows, dims, off):
+    say("rms_norm edges", rows, dims, off)
+    rng = np.random.default_rng(rows + dims)
+    x, w = f16(rng.normal(0, 2, (rows, dims))), f16(1 + rng.normal(0, 0.1, dims))
+    px = dev.put(np.concatenate([np.zeros(off, np.uint16), x.ravel()])) + 2 * off
+    y = dev.empty(x.nbytes)
+    dev.cm.call("cactus_hip_rms_norm_f16", px, dev.put(w), y.ptr, rows, dims, 1e-6, None)
+    assert_bits(dev.get(y, np.uint16, x.shape), orc.rms_norm(x, w, 1e-6), "rms_norm")
+
+
 @pytest.mark.parametrize("M,K,N", [(1, 1024, 4096), (2, 3, 2), (3, 1024, 1000), (5, 520, 77), (1, 24, 9)])
 def test_matmul_f16(dev, orc, M, K, N):
     say("matmul_f16", M, K, N)
