@@ -45,6 +45,8 @@ CXX_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-Wall", "-ffp-contract=off"]
 # rescale) needs no v_accvgpr_read / v_accvgpr_write copies
 HIP_FILE_FLAGS = {
     "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    # the exact prefill attention reads its chain accumulators on the VALU
+    "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     # the prefill attention scales its output accumulators every key tile
     "attention_fast.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     # the decode value chains: the next block's scalar weight loads must stay

@@ -224,22 +224,19 @@ __global__ void __launch_bounds__(256) attn_scores_kernel(AttnArgs a_in) {
     }
 }
 
-// ------------------------------------------------ kernel A, many query rows
-// Prefill form of the scores.  A lane still owns one key, but a wave scores
-// it against SQ_NQ query vectors (SQ_NQ/gq consecutive query rows times the
-// gq heads of the kv head): the key row is loaded and converted once per 16
-// dims for all of them.  A query vector enters the FMA through DPP
-// row_newbcast from a register that holds 16 of its dims replicated over the
-// four 16-lane rows, so a score step is one VALU op.  The reference's
-// per-score order is kept: accumulator c of query q takes dims 8i+c in
-// increasing i, then ((c0+c4)+(c1+c5)) + ((c2+c6)+(c3+c7)), times scale.
-// The INT8 key value (float)code * scale is formed as
+// ------------------------------------------------ kernel A, decode row
+// One query row of up to two heads per kv head: a one-wave workgroup per 64
+// keys and query head.  A lane owns one key, whose whole INT8 row is loaded
+// before the query, so the two memory round trips overlap.  The query vector
+// enters the FMA through DPP row_newbcast from a register that holds 16 of
+// its dims replicated over the four 16-lane rows, so a score step is one VALU
+// op.  The reference's per-score order is kept: accumulator c takes dims
+// 8i+c in increasing i, then ((c0+c4)+(c1+c5)) + ((c2+c6)+(c3+c7)), times
+// scale.  The INT8 key value (float)code * scale is formed as
 // fma((float)(code + 128), scale, -128 * scale): the exact product rounded
 // once, the same float as the reference's rounded multiply.  Block sums run
 // in the reference's sequential order in one lane per (query, block), from
 // the wave's weights in LDS.
-constexpr int SQ_NQ = 8;
-
 template <int NQ, int K>
 __device__ __forceinline__ void sq_step(float (&acc)[NQ][8], const float (&qv)[NQ], float k) {
 #pragma unroll
@@ -252,21 +249,16 @@ __device__ __forceinline__ void sq_group16(float (&acc)[NQ][8], const float (&qv
     (sq_step<NQ, K>(acc, qv, kk[K]), ...);
 }
 
-// NQ query vectors per wave, NW waves (64-key chunks) per workgroup.  The
-// prefill form is NQ = 8, NW = 4; the decode form (one query row) is
-// NQ = 1, NW = 1, the gq heads of a kv head in gq workgroups per chunk
-// (hsplit), with the lane's whole INT8 key row loaded before the query, so
-// the two memory round trips overlap.
-template <bool HYBRID, int D, int NQ, int NW>
-__global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in) {
-    constexpr bool PRE = NQ <= 2;                      // key row preloaded
+// the gq heads of a kv head in gq workgroups per chunk (hsplit)
+template <bool HYBRID, int D>
+__global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
+    constexpr int NQ = 1;                              // query vectors per wave
     const AttnArgs a = resolve(a_in);
     __shared__ float qsh[NQ][D];
-    __shared__ __align__(16) float wsh[NW][NQ][64];
-    __shared__ float msh[NW][NQ][2];
-    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-    // gq: the query heads of the kv head this workgroup takes (all of them,
-    // or 1 / hsplit of them in the decode form)
+    __shared__ __align__(16) float wsh[NQ][64];
+    __shared__ float msh[NQ][2];
+    const int lane = threadIdx.x;
+    // gq: the query heads of the kv head this workgroup takes (1 / hsplit of them)
     const int hsp = a.hsplit > 1 ? a.hsplit : 1;
     const int gq = a.gq / hsp, qr = NQ / gq;
     const int ngrp = (a.S + qr - 1) / qr;
@@ -300,8 +292,7 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
         kv_range<HYBRID>(a, (size_t)(qp0 + r), s0, e, bl);
         if (e > kv_end_max) kv_end_max = e;
     }
-    const size_t chunk = (size_t)bx * NW + wid;
-    const size_t wbase = chunk * 64;                   // first key of the wave
+    const size_t wbase = (size_t)bx * 64;              // first key of the wave
     const int jl = lane & 31;
     const size_t bs0 = wbase + (lane & 32);
     const size_t kp = wbase + lane;
@@ -318,34 +309,32 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
         const size_t klen = HYBRID ? a.new_len : a.Skv;
         krow16 = a.k + ((b * klen + kpos) * a.Hkv + kvh) * (size_t)d;
     }
-    // decode form: the lane's INT8 key row, loaded branch-free (a lane
+    // the lane's INT8 key row, loaded branch-free (a lane
     // without a cached key reads a stand-in row, its values unused) so no
     // wait is forced at the load; issued after the head preparation's own
     // loads when that runs here
-    uint4 pre[PRE ? D / 16 : 1];
+    uint4 pre[D / 16];
     float pres = 0.0f;
     auto preload = [&]() {
-        if constexpr (PRE) {
-            const bool own = kload && kint8;
-            const void* stand_in = a.prep.q_raw ? (const void*)a.prep.q_raw : (const void*)a.q;
-            const int8_t* src = own ? krow8 : reinterpret_cast<const int8_t*>(stand_in);
-            const float* ssrc = own ? ksr : reinterpret_cast<const float*>(stand_in);
+        const bool own = kload && kint8;
+        const void* stand_in = a.prep.q_raw ? (const void*)a.prep.q_raw : (const void*)a.q;
+        const int8_t* src = own ? krow8 : reinterpret_cast<const int8_t*>(stand_in);
+        const float* ssrc = own ? ksr : reinterpret_cast<const float*>(stand_in);
 #pragma unroll
-            for (int m = 0; m < D / 16; m++) pre[m] = *reinterpret_cast<const uint4*>(src + 16 * m);
-            pres = ssrc[0];
-        }
+        for (int m = 0; m < D / 16; m++) pre[m] = *reinterpret_cast<const uint4*>(src + 16 * m);
+        pres = ssrc[0];
     };
-    // decode form with the head preparation fused in (one wave, one row):
+    // with the head preparation fused in (one wave, one row):
     // q of the group's heads and, in the chunk holding it, the new key row
     // get the reference's head RMSNorm and RoPE here (the step's attn_prep
     // arithmetic, kernel_attention.cpp:484-676); that chunk also appends the
     // new key and value to the INT8 cache (and the value's product tiles)
-    __shared__ uint16_t prow[PRE ? NQ + 1 : 1][PRE ? D : 1];
-    __shared__ uint16_t pys[PRE ? NQ + 1 : 1][PRE ? D : 1];
-    __shared__ uint16_t krot[PRE ? D : 1];
-    __shared__ __align__(16) float nk_acc[PRE ? NQ : 1][8];
+    __shared__ uint16_t prow[NQ + 1][D];
+    __shared__ uint16_t pys[NQ + 1][D];
+    __shared__ uint16_t krot[D];
+    __shared__ __align__(16) float nk_acc[NQ][8];
     bool nk_lane = false;                               // the new key's accumulators come from nk_acc
-    if constexpr (PRE && NW == 1) {
+    {
         if (a.prep.q_raw) {
             const bool appender = bx == nbx - 1;
             if (appender && hs != 0) return;               // one appender per kv head
@@ -444,9 +433,9 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
             }
         }
     }
-    if (!(PRE && NW == 1) || !a.prep.q_raw) {
+    if (!a.prep.q_raw) {
         preload();
-        for (int i = threadIdx.x; i < NQ * D; i += 64 * NW) {
+        for (int i = threadIdx.x; i < NQ * D; i += 64) {
             const int v = i / D, dim = i % D;
             const int qp = qp0 + v / gq;
             qsh[v][dim] = qp < a.S ? h2f(a.q[((b * a.S + qp) * a.Hq + h0 + v % gq) * (size_t)d + dim]) : 0.0f;
@@ -462,52 +451,14 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
 #pragma unroll
         for (int c = 0; c < 8; c++) acc[q][c] = 0.0f;
     const int lr = lane & 15;
-    // prefill form: the next 16 dims of the key (codes and scale, or fp16
-    // values) are loaded while the current 16 feed the FMAs, so a step's
-    // global round trip overlaps the previous step's 128 FMAs
-    // The loads take no branch: a lane past the last key reads the row of
-    // the wave's last live key instead (its values are never used), an INT8
-    // row is read through both pointers, an fp16 row as two halves.
-    uint4 nx0[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
-    uint4 nx1[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
-    float nxs[2] = {0.0f, 0.0f};   // two buffers, alternating by step
-    const bool one_scale = a.qgs >= D;
-    float s_row = 0.0f;
-    const uint8_t* ld0 = nullptr;
-    const uint8_t* ld1 = nullptr;
-    int ldstep = 0;
-    if constexpr (!PRE) {
-        if (kload && kint8 && one_scale) s_row = ksr[0];
-        const size_t kpl = kload ? kp : kv_end_max - 1;   // kv_end_max > wbase here
-        if (HYBRID && kpl < a.cache_len) {
-            ld0 = reinterpret_cast<const uint8_t*>(a.kc + ((b * a.cache_len + kpl) * a.Hkv + kvh) * (size_t)d);
-            ld1 = ld0;
-            ldstep = 16;
-        } else {
-            const size_t kpos = HYBRID ? kpl - a.cache_len : kpl;
-            const size_t klen = HYBRID ? a.new_len : a.Skv;
-            ld0 = reinterpret_cast<const uint8_t*>(a.k + ((b * klen + kpos) * a.Hkv + kvh) * (size_t)d);
-            ld1 = ld0 + 16;
-            ldstep = 32;
-        }
-    }
-    auto fetch = [&](int m) {
-        if constexpr (!PRE) {
-            nx0[m & 1] = *reinterpret_cast<const uint4*>(ld0 + (size_t)ldstep * m);
-            nx1[m & 1] = *reinterpret_cast<const uint4*>(ld1 + (size_t)ldstep * m);
-            if (!one_scale) nxs[m & 1] = (kload && kint8) ? ksr[(16 * m) / a.qgs] : 0.0f;
-        }
-    };
-    // decode form: every step's query values in registers before the loop
+    // every step's query values in registers before the loop
     // (a read from LDS right before its step's FMAs would wait out the LDS
     // latency at each of the D/16 steps)
-    float qall[PRE ? D / 16 : 1][NQ];
-    if constexpr (PRE) {
+    float qall[D / 16][NQ];
 #pragma unroll
-        for (int m = 0; m < D / 16; m++)
+    for (int m = 0; m < D / 16; m++)
 #pragma unroll
-            for (int q = 0; q < NQ; q++) qall[m][q] = qsh[q][16 * m + lr];
-    }
+        for (int q = 0; q < NQ; q++) qall[m][q] = qsh[q][16 * m + lr];
     auto conv_i8 = [](float (&kk)[16], const uint4 raw, const float s) {
         const float ns = -128.0f * s;
         const uint32_t w4[4] = {raw.x ^ 0x80808080u, raw.y ^ 0x80808080u, raw.z ^ 0x80808080u,
@@ -530,9 +481,9 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
     // lane its own, unused: their scores are not computed, or replaced below)
     auto step = [&](int m, auto all_i8) {
         float kk[16];
-        if constexpr (PRE && decltype(all_i8)::value) {
+        if constexpr (decltype(all_i8)::value) {
             conv_i8(kk, pre[m], pres);
-        } else if constexpr (PRE) {
+        } else {
             if (kload && kint8) {
                 conv_i8(kk, pre[m], (a.qgs >= D) ? pres : ksr[(16 * m) / a.qgs]);
             } else if (kload && !nk_lane) {
@@ -542,21 +493,14 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
 #pragma unroll
                 for (int e = 0; e < 16; e++) kk[e] = 0.0f;
             }
-        } else {
-            if (m + 1 < D / 16) fetch(m + 1);
-            // a lane past the last key converts the row it loaded; its
-            // scores are never used (not computed, or masked to -inf)
-            if (ldstep == 16) conv_i8(kk, nx0[m & 1], one_scale ? s_row : nxs[m & 1]);
-            else conv_f16(kk, nx0[m & 1], nx1[m & 1]);
         }
         float qv[NQ];
 #pragma unroll
-        for (int q = 0; q < NQ; q++) qv[q] = PRE ? qall[m][q] : qsh[q][16 * m + lr];
+        for (int q = 0; q < NQ; q++) qv[q] = qall[m][q];
         sq_group16<NQ>(acc, qv, kk, std::make_integer_sequence<int, 16>{});
     };
-    fetch(0);
     bool all_i8 = false;
-    if constexpr (PRE && NW == 1 && HYBRID) all_i8 = a.prep.q_raw != nullptr && a.qgs >= D;
+    if constexpr (HYBRID) all_i8 = a.prep.q_raw != nullptr && a.qgs >= D;
     if (all_i8) {
 #pragma unroll
         for (int m = 0; m < D / 16; m++) step(m, std::true_type{});
@@ -564,7 +508,7 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
 #pragma unroll
         for (int m = 0; m < D / 16; m++) step(m, std::false_type{});
     }
-    if constexpr (PRE && NW == 1) {
+    {
         if (__builtin_amdgcn_readfirstlane(__ballot(nk_lane) != 0ull ? 1 : 0)) {   // the new key's chunk only
             typedef float f4v __attribute__((ext_vector_type(4)));
 #pragma unroll
@@ -616,8 +560,8 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
         const bool wlane = block_live && jl < bsz;
         const size_t row = (b * a.S + (row_ok ? qp : 0)) * a.Hq + h0 + q % gq;
         if (wlane) a.w[row * a.wstride + kp] = w;
-        wsh[wid][q][lane] = w;
-        if (jl == 0) msh[wid][q][lane >> 5] = mx;
+        wsh[q][lane] = w;
+        if (jl == 0) msh[q][lane >> 5] = mx;
     }
     wave_lds_order();
     // ---- block sums, one lane per (query vector, block), reference order
@@ -638,7 +582,7 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
                 // past bsz hold other keys' weights or stale values; they are
                 // selected out), then the fold in the reference's order
                 typedef float f4v __attribute__((ext_vector_type(4)));
-                const f4v* x4 = reinterpret_cast<const f4v*>(&wsh[wid][q][32 * half]);
+                const f4v* x4 = reinterpret_cast<const f4v*>(&wsh[q][32 * half]);
                 float x[32];
 #pragma unroll
                 for (int t = 0; t < 8; t++) {
@@ -661,11 +605,265 @@ __global__ void __launch_bounds__(64 * NW) attn_scores_rows_kernel(AttnArgs a_in
                 }
                 const size_t row = (b * a.S + qp) * a.Hq + h0 + q % gq;
                 const int blk = (int)(bs / ATT_BLOCK);
+                a.bmax[row * a.nbstride + blk] = block_skipped ? NEG_INF : msh[q][half];
+                const float bsv = block_skipped ? 0.0f : sum;
+                a.bsum[row * a.nbstride + blk] = has_zero ? set_sign(bsv) : bsv;
+            }
+        }
+    }
+}
+
+// ------------------------------------------------ kernel A, prefill rows
+// A score is eight fp32 FMA chains in a fixed order, and
+// v_mfma_f32_4x4x1_16b_f32 is a chain step: every output takes one product,
+// fused and rounded once as fmaf (compared bit for bit on the device over
+// normal, denormal and infinite operands).  With lane = key as operand B
+// and four query vectors as operand A -- one register holds 16 dims x 4
+// vectors, the dim picked by the instruction's A-block broadcast -- an
+// instruction advances 256 chains in 8 cycles, against 64 in ~4.5 for a
+// v_fmac_f32 with a DPP operand, and leaves the VALU to the conversions and
+// the weights.  A wave converts its 64 keys once into registers (D values per
+// lane) and runs them against SM_Q query vectors, four at a time; the eight
+// accumulators of a step are independent, so the matrix pipe stays full from
+// one wave.  What bounds it now is the VALU work per weight (the block
+// maximum and a double-precision expf), four vectors side by side so that
+// their dependent steps alternate.  The weights of all SM_Q vectors stay in
+// LDS, so that the sequential block sums run on all 64 lanes at once (lane =
+// query vector and block).  256 rows x 16 heads over 1920 keys on average,
+// 128 dims: 83 us with the DPP form, 48 us.
+constexpr int SM_Q = 32;                           // query vectors staged together
+constexpr int SM_WS = 68;                          // weights of a vector in LDS (bank skew)
+
+template <int... T>
+__device__ __forceinline__ void sm_step16(f32x4 (&acc)[8], float a, const float* k, std::integer_sequence<int, T...>) {
+    ((acc[T & 7] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, k[T], acc[T & 7], 4, T, 0)), ...);
+}
+
+template <bool HYBRID, int D>
+__global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in, int nsub) {
+    const AttnArgs a = resolve(a_in);
+    // lane 4 t + i of a register: dim t of vector i (rows 4 banks apart: the
+    // staging writes of a wave fall on 64 banks)
+    __shared__ float qsh[SM_Q / 4][D / 16][SM_WS];
+    __shared__ __align__(16) float wsh[4][SM_Q][SM_WS];
+    __shared__ float msh[4][SM_Q][2];
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const float NEG_INF = -__builtin_inff();
+    const int gq = a.gq, qr = SM_Q / gq;                 // query rows of a sub-tile
+    const int ngrp = (a.S + qr * nsub - 1) / (qr * nsub);
+    size_t gy = blockIdx.y;
+    const int kvh = (int)(gy % a.Hkv);
+    gy /= a.Hkv;
+    const int qp_wg = (int)(gy % ngrp) * qr * nsub, qp_end = min(qp_wg + qr * nsub, a.S);
+    const size_t b = gy / ngrp;
+    const int h0 = kvh * gq;
+    // kv_range of a row on this path (no window, at most 32768 keys, so ints)
+    const int pos = (int)(a.pos_off < (1u << 30) ? a.pos_off : (1u << 30)), Skv = (int)a.Skv;
+    auto row_end = [&](int qp, int& limit) {
+        const int e = a.causal ? min(pos + qp + 1, Skv) : Skv;
+        limit = HYBRID ? e : Skv;
+        return e;
+    };
+    int lim_last;
+    const int kv_end_max = row_end(qp_end - 1, lim_last);   // the last row reaches furthest
+    if ((int)blockIdx.x * 256 >= kv_end_max) return;     // the whole workgroup
+    const int wbase = (int)blockIdx.x * 256 + wid * 64;
+
+    // ---- every global load first: this lane's key row (a lane past the last
+    // key reads the row of the last one; its scores are not used) ...
+    const int kp = wbase + lane;
+    const int kpl = min(kp, kv_end_max - 1);
+    const bool own8 = HYBRID && (size_t)kpl < a.cache_len;
+    const int8_t* k8 = nullptr;
+    const uint16_t* k16 = nullptr;
+    const float* ksr = nullptr;
+    if (own8) {
+        k8 = a.kc + ((b * a.cache_len + kpl) * a.Hkv + kvh) * (size_t)D;
+        ksr = a.ks + ((size_t)kpl * a.Hkv + kvh) * (size_t)a.nqg;   // no batch offset (kernel_attention.cpp:353)
+    } else {
+        const size_t kpos = HYBRID ? kpl - a.cache_len : (size_t)kpl;
+        const size_t klen = HYBRID ? a.new_len : a.Skv;
+        k16 = a.k + ((b * klen + kpos) * a.Hkv + kvh) * (size_t)D;
+    }
+    // a wave whose keys are all cached (the common one) reads INT8 rows only
+    const bool all8 = HYBRID && (size_t)min(wbase + 63, kv_end_max - 1) < a.cache_len;
+    i32x4 raw[D / 16];
+    float sc8[D / 16];
+    if (all8) {
+#pragma unroll
+        for (int m = 0; m < D / 16; m++) raw[m] = *reinterpret_cast<const i32x4*>(k8 + 16 * m);
+#pragma unroll
+        for (int m = 0; m < D / 16; m++) sc8[m] = ksr[a.qgs >= D ? 0 : 16 * m / a.qgs];
+    }
+    // ... and the first sub-tile's query vectors, 8 dims per thread and step
+    // (rows past S repeat the last one; their weights are not stored)
+    const bool qvec = ((uintptr_t)a.q & 15) == 0;
+    constexpr int QU = SM_Q * D / 8 / 256;
+    i32x4 qw[QU];
+    auto load_q = [&](int qp0) {
+#pragma unroll
+        for (int j = 0; j < QU; j++) {
+            const int u = threadIdx.x + 256 * j;
+            const int v = u / (D / 8), c = u % (D / 8);
+            const int qp = min(qp0 + v / gq, a.S - 1);
+            const uint16_t* src = a.q + ((b * a.S + qp) * a.Hq + h0 + v % gq) * (size_t)D + 8 * c;
+            if (qvec) {
+                qw[j] = *reinterpret_cast<const i32x4*>(src);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) qw[j][e] = (int)((uint32_t)src[2 * e] | ((uint32_t)src[2 * e + 1] << 16));
+            }
+        }
+    };
+    auto store_q = [&]() {
+#pragma unroll
+        for (int j = 0; j < QU; j++) {
+            const int u = threadIdx.x + 256 * j;
+            const int v = u / (D / 8), c = u % (D / 8);
+            float* dst = &qsh[v >> 2][c >> 1][32 * (c & 1) + (v & 3)];
+#pragma unroll
+            for (int e = 0; e < 8; e++) dst[4 * e] = h2f((uint16_t)((uint32_t)qw[j][e >> 1] >> (16 * (e & 1))));
+        }
+    };
+    load_q(qp_wg);
+    float kk[D];                                         // the key row as fp32
+    // (float)code * scale as fma(code + 128, scale, -128 scale): the exact
+    // product rounded once
+    auto conv8 = [&](int m, const i32x4 w4, float sc) {
+        const float ns = -128.0f * sc;
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const uint32_t w = (uint32_t)w4[e >> 2] ^ 0x80808080u;
+            kk[16 * m + e] = __builtin_fmaf((float)((w >> (8 * (e & 3))) & 0xFFu), sc, ns);
+        }
+    };
+    if (all8) {
+#pragma unroll
+        for (int m = 0; m < D / 16; m++) conv8(m, raw[m], sc8[m]);
+    } else {
+#pragma unroll
+        for (int m = 0; m < D / 16; m++) {
+            if (own8) {
+                conv8(m, *reinterpret_cast<const i32x4*>(k8 + 16 * m), ksr[16 * m / a.qgs]);
+            } else {
+                const i32x4 x0 = *reinterpret_cast<const i32x4*>(k16 + 16 * m);
+                const i32x4 x1 = *reinterpret_cast<const i32x4*>(k16 + 16 * m + 8);
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const uint32_t w = (uint32_t)(e < 8 ? x0[e >> 1] : x1[(e - 8) >> 1]);
+                    kk[16 * m + e] = h2f((uint16_t)(e & 1 ? w >> 16 : w & 0xFFFFu));
+                }
+            }
+        }
+    }
+    const int jl = lane & 31;
+    const int bs0 = wbase + (lane & 32);
+    const int lgq = __builtin_ctz((unsigned)gq);         // gq divides SM_Q: a power of two
+    for (int qp0 = qp_wg; qp0 < qp_end; qp0 += qr) {
+        if (qp0 > qp_wg) __syncthreads();                    // every wave is done with the last sub-tile
+        store_q();
+        __syncthreads();
+        if (qp0 + qr < qp_end) load_q(qp0 + qr);             // in flight while this one is used
+        for (int g = 0; g < SM_Q / 4; g++) {
+            if (qp0 + (4 * g >> lgq) >= a.S) break;
+            int lim_g;
+            if (wbase >= row_end(min(qp0 + ((4 * g + 3) >> lgq), a.S - 1), lim_g)) continue;
+            // accumulator c of the four vectors: dims 8 i + c in increasing i
+            f32x4 acc[8];
+#pragma unroll
+            for (int c = 0; c < 8; c++) acc[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+            float qa[D / 16];
+#pragma unroll
+            for (int m = 0; m < D / 16; m++) qa[m] = qsh[g][m][lane];
+#pragma unroll
+            for (int m = 0; m < D / 16; m++) sm_step16(acc, qa[m], kk + 16 * m, std::make_integer_sequence<int, 16>{});
+            // the four vectors' weights side by side, without branches (a row
+            // past S repeats the last one and is not stored)
+            float sc[4], mx[4], w[4];
+            bool wlane[4];
+            const f32x4 dot = (((acc[0] + acc[4]) + (acc[1] + acc[5])) + ((acc[2] + acc[6]) + (acc[3] + acc[7]))) * a.scale;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int qp = min(qp0 + ((4 * g + r) >> lgq), a.S - 1);
+                int blk_limit;
+                const int kv_end = row_end(qp, blk_limit);
+                if constexpr (HYBRID) {
+                    wlane[r] = kp < kv_end;
+                    sc[r] = wlane[r] ? dot[r] : NEG_INF;
+                } else {
+                    const bool block_live = bs0 < kv_end;
+                    const int bsz = block_live ? min(ATT_BLOCK, blk_limit - bs0) : 0;
+                    wlane[r] = jl < bsz;
+                    const int aq = (int)a.pos_off + qp;
+                    const bool is_decode = qp == a.S - 1 && a.S > 1;
+                    bool ok = wlane[r] && !(a.causal && (kp > aq || (!is_decode && bs0 > aq)));
+                    if (a.mask && ok) ok = h2f(a.mask[(b * a.S + qp) * a.Skv + kp]) != 0.0f;
+                    sc[r] = ok ? dot[r] : NEG_INF;
+                }
+                mx[r] = sc[r];
+            }
+            half_wave_max4(mx);
+#pragma unroll
+            for (int r = 0; r < 4; r++) w[r] = sc[r] - mx[r];
+            cactus_expf_n<4>(w, w);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if constexpr (!HYBRID) {
+                    const int qp = min(qp0 + ((4 * g + r) >> lgq), a.S - 1);
+                    int blk_limit;
+                    const int kv_end = row_end(qp, blk_limit);
+                    const int bsz = bs0 < kv_end ? min(ATT_BLOCK, blk_limit - bs0) : 0;
+                    if (jl < (bsz / 4) * 4) w[r] = poly_exp_weight(sc[r], mx[r]);
+                }
+                w[r] = sc[r] != NEG_INF ? w[r] : 0.0f;       // -inf also from masks and score overflow
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int q = 4 * g + r, qp = qp0 + (q >> lgq);
+                const size_t row = (b * a.S + qp) * a.Hq + h0 + (q & (gq - 1));
+                if (wlane[r] && qp < a.S) (a.w + row * a.wstride + wbase)[lane] = w[r];
+                wsh[wid][q][lane] = w[r];
+                if (jl == 0) msh[wid][q][lane >> 5] = mx[r];
+            }
+        }
+        wave_lds_order();
+        // ---- block sums, one lane per (query vector, block), reference order
+        const int q = lane >> 1, half = lane & 1;
+        const int qp = qp0 + q / gq;
+        const int bs = wbase + 32 * half;
+        if (qp < a.S) {
+            int blk_limit;
+            const int kv_end = row_end(qp, blk_limit);
+            if (bs < kv_end) {
+                const int bsz = min(ATT_BLOCK, blk_limit - bs);
+                const bool is_decode = (!HYBRID) && (qp == a.S - 1) && a.S > 1;
+                const bool block_skipped = !HYBRID && !is_decode && a.causal && bs > (int)a.pos_off + qp;
+                // slots past bsz hold other keys' weights or stale values; they
+                // are selected out
+                const f32x4* x4 = reinterpret_cast<const f32x4*>(&wsh[wid][q][32 * half]);
+                const int v4 = HYBRID ? 0 : (bsz / 4) * 4;
+                float sum = 0.0f;
+                bool has_zero = false;
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    const f32x4 x = x4[t];
+                    if (!HYBRID && 4 * t < v4) {
+                        sum = sum + ((x[0] + x[1]) + (x[2] + x[3]));
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 4; u++) sum = 4 * t + u < bsz ? sum + x[u] : sum;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; u++) has_zero |= 4 * t + u < bsz && !(x[u] != 0.0f);
+                }
+                const size_t row = (b * a.S + qp) * a.Hq + h0 + q % gq;
+                const int blk = bs / ATT_BLOCK;
                 a.bmax[row * a.nbstride + blk] = block_skipped ? NEG_INF : msh[wid][q][half];
                 const float bsv = block_skipped ? 0.0f : sum;
                 a.bsum[row * a.nbstride + blk] = has_zero ? set_sign(bsv) : bsv;
             }
         }
+        wave_lds_order();                                // the sums are read before the next weights
     }
 }
 
@@ -933,7 +1131,9 @@ struct CdCfg {
 // (the running max is the last finite block max), else NEG_INF (the block
 // leaves the accumulators unscaled); bsum[blk] is the block's flagged sum.
 // One whole wave.
-__device__ __forceinline__ void chain_corr_scan(int nb, float* corr);
+// ST: floats between a row's blocks in LDS; none: what an unscaled block holds.
+template <int ST = 1>
+__device__ __forceinline__ void chain_corr_scan(int nb, float* corr, float none = -__builtin_inff());
 __device__ __forceinline__ void chain_corr(const AttnArgs& a, size_t row, int nb, float* corr, float* bsum) {
     const int lane = threadIdx.x & 63;
     const float* bm = a.bmax + row * a.nbstride;
@@ -946,13 +1146,14 @@ __device__ __forceinline__ void chain_corr(const AttnArgs& a, size_t row, int nb
     chain_corr_scan(nb, corr);
 }
 // block maxima in corr[0, nb) -> the corrections, in place (one wave)
-__device__ __forceinline__ void chain_corr_scan(int nb, float* corr) {
+template <int ST>
+__device__ __forceinline__ void chain_corr_scan(int nb, float* corr, float none) {
     const int lane = threadIdx.x & 63;
     const float NEG_INF = -__builtin_inff();
     float carry = NEG_INF;
     for (int c0 = 0; c0 < nb; c0 += 64) {
         const int i = c0 + lane;
-        const float m = i < nb ? corr[i] : NEG_INF;
+        const float m = i < nb ? corr[i * ST] : NEG_INF;
         const bool fin = m > NEG_INF;
         int idx = fin ? lane : -1;
 #pragma unroll
@@ -964,7 +1165,7 @@ __device__ __forceinline__ void chain_corr_scan(int nb, float* corr) {
         if (lane == 0) ex = -1;
         const float pm = __shfl(m, ex < 0 ? 0 : ex, 64);
         const float prev = ex >= 0 ? pm : carry;
-        if (i < nb) corr[i] = fin ? cactus_expf(prev - m) : NEG_INF;
+        if (i < nb) corr[i * ST] = fin ? cactus_expf(prev - m) : none;
         const int last = __shfl(idx, 63, 64);
         if (last >= 0) carry = __shfl(m, last, 64);
     }
@@ -1344,61 +1545,50 @@ __global__ void __launch_bounds__(64 * (ATT_MAX_GQ + CD_NP)) attn_chain_dma_kern
 // ------------------------------------------------ kernel B, many query rows
 // Prefill form of the value chains.  A workgroup owns RW_CH chains -- RW_CH/gq
 // consecutive query rows times the gq heads of one kv head -- on one 64-dim
-// slice.  Each chain wave runs RW_CPW chains per lane (lane = dimension), so
-// one LDS read of a value row feeds RW_CPW FMAs, and the chains of a lane
-// interleave instead of waiting on each other's FMA latency.  Weights enter
-// the FMA through DPP row_newbcast (a 16-key weight vector replicated per
-// 16-lane row), so a step reads no weight from LDS.  The stage waves fetch
-// the next tile's value rows into registers a whole step ahead and store the
-// reference's fp32 operands (INT8 code * per-key group scale for the cache,
-// fp16 -> fp32 for new rows and the FP16 path) as [dim][key] rows, plus the
-// chains' weights.  Blocks that are partial or hold a zero weight run key by
+// slice.  The chain step is the matrix instruction of the prefill scores,
+// v_mfma_f32_4x4x1_16b_f32 (one fused product per output, rounded as fmaf):
+// lane = dim as operand B, the weights of four chains and 16 keys in one A
+// register, so a chain wave advances its RW_CPW = 8 chains of 64 dims by one
+// key with two instructions of 8 cycles whose results alternate (a dependent
+// pair needs 16).  The stage waves fetch the next tile's value rows into
+// registers a whole step ahead and store the reference's fp32 operands (INT8
+// code * per-key group scale for the cache, fp16 -> fp32 for new rows and the
+// FP16 path) as [dim][key] rows, plus the chains' weights as [4 chains][key].
+// Where the chains' key ranges end, the keys that all of them have run as
+// before and the rest key by key; blocks that hold a zero weight run key by
 // key with the reference's zero skip (kernel_attention.cpp:200-201).
+// 256 rows x 16 heads over 1920 keys on average, 128 dims: 74 us with DPP
+// chains, 57 us (the matrix steps alone take 14: the chain waves' LDS reads
+// and the stage waves' issue share the rest).
 constexpr int RW_T = 64;                          // keys per tile
 constexpr int RW_PS = RW_T + 4;                   // floats per dim row (bank skew)
 constexpr int RW_CH = 32;                         // chains per workgroup
-constexpr int RW_CPW = 4;                         // chains per lane of a chain wave
+constexpr int RW_CPW = 8;                         // chains per chain wave
+constexpr int RW_CS = RW_CH + 4;                  // floats per block of factors (bank skew)
 constexpr int RW_NCW = RW_CH / RW_CPW;            // chain waves
 constexpr int RW_NSW = 4;                         // stage waves
+constexpr int RW_PF = 3;                           // tiles of loads in flight per stage wave
 constexpr int RW_THREADS = 64 * (RW_NCW + RW_NSW);
-constexpr int RW_PROD_B = 2 * 64 * RW_PS * 4;
-constexpr int RW_W_B = 2 * RW_CH * RW_T * 4;
+constexpr int RW_NB = 3;                           // tiles in LDS: two ahead of the stage waves' writes
+constexpr int RW_PROD_B = RW_NB * 64 * RW_PS * 4;
+constexpr int RW_W_B = RW_NB * RW_CH * RW_T * 4;
 
-template <int K>
-__device__ __forceinline__ void rw_step(float (&acc)[RW_CPW], const float (&wv)[RW_CPW], float p) {
-#pragma unroll
-    for (int c = 0; c < RW_CPW; c++) fmac_row_bcast<K>(acc[c], wv[c], p);
-}
-template <int... K>
-__device__ __forceinline__ void rw_chain16(float (&acc)[RW_CPW], const float* p, const float (&wv)[RW_CPW],
-                                           std::integer_sequence<int, K...>) {
-    asm volatile("s_nop 1");   // DPP source read after a possible VALU write of wv
-    (rw_step<K>(acc, wv, p[K]), ...);
-}
-
-// weight k of a 16-lane row, broadcast over the row (DPP row_newbcast:k)
-template <int K>
-__device__ __forceinline__ float row_bcast(float w) {
-    return __builtin_bit_cast(float,
-                              __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, w), 0x150 + K, 0xF, 0xF, false));
-}
-// 16 chain steps of one chain, key k taken only where bit k of the
-// wave-uniform mask nz is set
-template <int... K>
-__device__ __forceinline__ void rw_masked16(float& acc, const float* p, float wv, uint32_t nz,
-                                            std::integer_sequence<int, K...>) {
-    ((((nz >> K) & 1u) ? (void)(acc = __builtin_fmaf(p[K], row_bcast<K>(wv), acc)) : (void)0), ...);
+// N keys (A blocks K0..) of the two four-chain groups: products p[k] (lane =
+// dim), weights of key k in A block k of w0 / w1
+template <int K0, int... K>
+__device__ __forceinline__ void rw_chain(f32x4 (&acc)[2], const f32x4* v, float w0, float w1,
+                                         std::integer_sequence<int, K...>) {
+    ((acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(w0, v[K >> 2][K & 3], acc[0], 4, K0 + K, 0),
+      acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(w1, v[K >> 2][K & 3], acc[1], 4, K0 + K, 0)), ...);
 }
 
 template <bool HYBRID>
 __global__ void __launch_bounds__(RW_THREADS) attn_rows_kernel(AttnArgs a_in, int nbmax) {
     const AttnArgs a = resolve(a_in);
     extern __shared__ __align__(16) unsigned char smem[];
-    float* prod = reinterpret_cast<float*>(smem);                        // [2][64][RW_PS]
-    float* wts = reinterpret_cast<float*>(smem + RW_PROD_B);             // [2][RW_CH][RW_T]
-    float* corr_s = reinterpret_cast<float*>(smem + RW_PROD_B + RW_W_B); // [RW_CH][nbmax]
-    float* bsum_s = corr_s + (size_t)RW_CH * nbmax;                      // [RW_CH][nbmax]
-    const float NEG_INF = -__builtin_inff();
+    float* prod = reinterpret_cast<float*>(smem);                        // [RW_NB][64][RW_PS]
+    float* wts = reinterpret_cast<float*>(smem + RW_PROD_B);             // [RW_NB][RW_CH / 4][RW_T][4]
+    float* corr_s = reinterpret_cast<float*>(smem + RW_PROD_B + RW_W_B); // [nbmax][RW_CS]
 
     const int d = a.d, da = (d / 8) * 8, gq = a.gq;
     const int qr = RW_CH / gq;                     // query rows of the workgroup
@@ -1429,201 +1619,308 @@ __global__ void __launch_bounds__(RW_THREADS) attn_rows_kernel(AttnArgs a_in, in
     const int nst = (int)((kneed - ks + RW_T - 1) / RW_T);
     const bool is_chain = wv < RW_NCW;
 
-    // ---- stage waves: item (dq, kq) = 4 dims x 4 keys of a tile
+    // ---- stage waves: item (dq, kq) = 4 dims x 4 keys of a tile.  RW_PF
+    // tiles of loads are in flight: a tile's chain steps are shorter than a
+    // memory round trip.  A tile of one kind (all cached, or all fp16) is read
+    // at fixed per-lane offsets from a scalar base, so it takes no address
+    // arithmetic; only tiles across a boundary pick each key's source.
     const int pl = (int)threadIdx.x - RW_NCW * 64;
-    const int dq = pl & 15, kq = pl >> 4;
-    const int dim0 = sl * 64 + dq * 4;
-    uint32_t r8[4];
-    uint2 r16[4];
-    float rsc[4];
-    float4 wr[2];
-    auto load_raw = [&](int t) {
-        const size_t tb = ks + (size_t)t * RW_T;
+    const int dq = pl & 15, kq = (pl >> 4) & 15;
+    const int dim0 = sl * 64 + dq * 4 < d ? sl * 64 + dq * 4 : 0;
+    struct Raw {
+        uint32_t lo[4], hi[4];   // 4 INT8 values in lo, or 4 fp16 values
+        float sc[4];
+        f32x4 w[2];
+    };
+    // 0: all keys cached, 1: all fp16, 2: both, or past the last key
+    auto kind = [&](int t) {
+        const size_t k0 = ks + (size_t)t * RW_T, k1 = k0 + RW_T;
+        if (k1 > kneed) return 2;
+        if (!HYBRID || k0 >= a.cache_len) return 1;
+        return k1 <= a.cache_len ? 0 : 2;
+    };
+    const uint32_t krow = (uint32_t)(a.Hkv * d);          // values from a key to the next
+    uint32_t off8[4], offs[4], offw[2];                   // from the tile's first key / column
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const size_t kp = tb + kq * 4 + e;
-            r8[e] = 0;
-            r16[e] = make_uint2(0, 0);
-            rsc[e] = 0.0f;
-            if (kp >= kneed || dim0 >= da) continue;
-            if (HYBRID && kp < a.cache_len) {
-                const size_t off = (b * a.cache_len + kp) * a.Hkv + kvh;
-                r8[e] = *reinterpret_cast<const uint32_t*>(a.vc + off * d + dim0);
-                rsc[e] = a.vs[(kp * a.Hkv + kvh) * a.nqg + dim0 / a.qgs];   // no batch offset (:424)
-            } else {
-                const size_t vpos = HYBRID ? kp - a.cache_len : kp;
-                const size_t vlen = HYBRID ? a.new_len : a.Skv;
-                r16[e] = *reinterpret_cast<const uint2*>(a.v + ((b * vlen + vpos) * a.Hkv + kvh) * (size_t)d + dim0);
+    for (int e = 0; e < 4; e++) {
+        off8[e] = (uint32_t)(kq * 4 + e) * krow + (uint32_t)dim0;
+        offs[e] = (uint32_t)((kq * 4 + e) * a.Hkv * a.nqg + dim0 / a.qgs);
+    }
+    const size_t wrow0 = (b * a.S + qp0) * a.Hq + kvh * gq;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int i = (pl & 255) + 256 * j, c = i >> 4;
+        const int dr = min(qp0 + c / gq, a.S - 1) - qp0;   // rows past S read the last one's (unused)
+        offw[j] = (uint32_t)((size_t)(dr * a.Hq + c % gq) * a.wstride) + (uint32_t)((i & 15) * 4);
+    }
+    const float* wbase = a.w + wrow0 * a.wstride;
+    auto load_raw = [&](int t, Raw& r) {
+        if (t >= nst) return;
+        const size_t k0 = ks + (size_t)t * RW_T;
+        const int kd = kind(t);
+        if (kd == 0) {
+            const int8_t* p = a.vc + ((b * a.cache_len + k0) * a.Hkv + kvh) * (size_t)d;
+            const float* ps = a.vs + (k0 * a.Hkv + kvh) * (size_t)a.nqg;   // no batch offset (:424)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                r.lo[e] = *reinterpret_cast<const uint32_t*>(p + off8[e]);
+                r.sc[e] = ps[offs[e]];
+            }
+        } else if (kd == 1) {
+            const size_t vpos = HYBRID ? k0 - a.cache_len : k0;
+            const size_t vlen = HYBRID ? a.new_len : a.Skv;
+            const uint16_t* p = a.v + ((b * vlen + vpos) * a.Hkv + kvh) * (size_t)d;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint2 u = *reinterpret_cast<const uint2*>(p + off8[e]);
+                r.lo[e] = u.x;
+                r.hi[e] = u.y;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const size_t kp = min(k0 + kq * 4 + e, kneed - 1);   // past the end: the last key (unused)
+                if (HYBRID && kp < a.cache_len) {
+                    const size_t off = (b * a.cache_len + kp) * a.Hkv + kvh;
+                    r.lo[e] = *reinterpret_cast<const uint32_t*>(a.vc + off * d + dim0);
+                    r.sc[e] = a.vs[(kp * a.Hkv + kvh) * a.nqg + dim0 / a.qgs];
+                } else {
+                    const size_t vpos = HYBRID ? kp - a.cache_len : kp;
+                    const size_t vlen = HYBRID ? a.new_len : a.Skv;
+                    const uint2 u = *reinterpret_cast<const uint2*>(a.v + ((b * vlen + vpos) * a.Hkv + kvh) * (size_t)d + dim0);
+                    r.lo[e] = u.x;
+                    r.hi[e] = u.y;
+                }
             }
         }
         // weights of the chains for this tile: 32 rows x 64 keys, 8 per thread
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int i = pl + 256 * j;
-            const int c = i >> 4, j4 = (i & 15) * 4;
-            const int qp = qp0 + c / gq;
-            wr[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            const size_t col = (size_t)t * RW_T + j4;
-            if (qp < a.S && col + 4 <= a.wstride) {
-                const size_t row = (b * a.S + qp) * a.Hq + kvh * gq + (c % gq);
-                wr[j] = *reinterpret_cast<const float4*>(a.w + row * a.wstride + col);
-            }
-        }
+        for (int j = 0; j < 2; j++) r.w[j] = *reinterpret_cast<const f32x4*>(wbase + (size_t)t * RW_T + offw[j]);
     };
-    auto store_tile = [&](int t) {
-        const size_t tb = ks + (size_t)t * RW_T;
-        float* pb = prod + (t & 1) * 64 * RW_PS;
+    auto store_tile = [&](int t, const Raw& r) {
+        if (t >= nst) return;
+        float* pb = prod + (t % RW_NB) * 64 * RW_PS;
+        const int kd = kind(t);
         float pr[4][4];
+        auto as_i8 = [&](int e) {
+            // (float)code * scale as fma(code + 128, scale, -128 scale): the
+            // exact product rounded once
+            const uint32_t u = r.lo[e] ^ 0x80808080u;
+            const float ns = -128.0f * r.sc[e];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const size_t kp = tb + kq * 4 + e;
-            if (HYBRID && kp < a.cache_len) {
+            for (int c = 0; c < 4; c++) pr[e][c] = __builtin_fmaf((float)((u >> (8 * c)) & 0xFFu), r.sc[e], ns);
+        };
+        auto as_f16 = [&](int e) {
+            pr[e][0] = h2f((uint16_t)(r.lo[e] & 0xFFFF));
+            pr[e][1] = h2f((uint16_t)(r.lo[e] >> 16));
+            pr[e][2] = h2f((uint16_t)(r.hi[e] & 0xFFFF));
+            pr[e][3] = h2f((uint16_t)(r.hi[e] >> 16));
+        };
+        if (kd == 0) {
 #pragma unroll
-                for (int c = 0; c < 4; c++) pr[e][c] = (float)(int8_t)((r8[e] >> (8 * c)) & 0xFF) * rsc[e];
-            } else {
-                pr[e][0] = h2f((uint16_t)(r16[e].x & 0xFFFF));
-                pr[e][1] = h2f((uint16_t)(r16[e].x >> 16));
-                pr[e][2] = h2f((uint16_t)(r16[e].y & 0xFFFF));
-                pr[e][3] = h2f((uint16_t)(r16[e].y >> 16));
+            for (int e = 0; e < 4; e++) as_i8(e);
+        } else if (kd == 1) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) as_f16(e);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if (HYBRID && min(ks + (size_t)t * RW_T + kq * 4 + e, kneed - 1) < a.cache_len) as_i8(e);
+                else as_f16(e);
             }
         }
 #pragma unroll
         for (int c = 0; c < 4; c++)
-            *reinterpret_cast<float4*>(pb + (dq * 4 + c) * RW_PS + kq * 4) =
-                make_float4(pr[0][c], pr[1][c], pr[2][c], pr[3][c]);
-        float* wb = wts + (t & 1) * RW_CH * RW_T;
+            *reinterpret_cast<f32x4*>(pb + (dq * 4 + c) * RW_PS + kq * 4) = (f32x4){pr[0][c], pr[1][c], pr[2][c], pr[3][c]};
+        float* wb = wts + (t % RW_NB) * RW_CH * RW_T;
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const int i = pl + 256 * j;
-            *reinterpret_cast<float4*>(wb + (i >> 4) * RW_T + (i & 15) * 4) = wr[j];
+            const int c = i >> 4, j4 = (i & 15) * 4;
+            float* wd = wb + ((c >> 2) * RW_T + j4) * 4 + (c & 3);
+#pragma unroll
+            for (int e = 0; e < 4; e++) wd[4 * e] = r.w[j][e];
         }
     };
 
-    // ---- chain waves: chains c0..c0+3 of the workgroup
-    const int c0 = wv * RW_CPW;
-    size_t crow[RW_CPW];
-    size_t crbl[RW_CPW];
-    int cnb[RW_CPW];
+    // ---- every wave prepares four chains' rescale factors; blocks that
+    // leave a chain as it is hold 1 (x * 1 is exact)
+    Raw raw[RW_PF];
+    if (!is_chain && nst > 0) {
 #pragma unroll
-    for (int c = 0; c < RW_CPW; c++) {
-        const int ch = c0 + c;
-        const int qp = qp0 + ch / gq;
-        crow[c] = 0;
-        crbl[c] = 0;
-        cnb[c] = 0;
-        if (is_chain && qp < a.S) {
+        for (int i = 0; i < RW_PF; i++) load_raw(i, raw[i]);
+    }
+    const int nbt = (int)((kneed - ks + ATT_BLOCK - 1) / ATT_BLOCK);
+    constexpr int CPW = RW_CH / (RW_NCW + RW_NSW);
+    int cnb[CPW];
+#pragma unroll
+    for (int i = 0; i < CPW; i++) {
+        const int qp = qp0 + (wv * CPW + i) / gq;
+        cnb[i] = 0;
+        if (qp < a.S) {
             size_t rks, rke, rbl;
             kv_range<HYBRID>(a, (size_t)qp, rks, rke, rbl);
-            crow[c] = (b * a.S + qp) * a.Hq + kvh * gq + ch % gq;
-            crbl[c] = rbl;
-            cnb[c] = rke > rks ? (int)((rke - rks + ATT_BLOCK - 1) / ATT_BLOCK) : 0;
-            chain_corr(a, crow[c], cnb[c], corr_s + (size_t)ch * nbmax, bsum_s + (size_t)ch * nbmax);
+            cnb[i] = rke > rks ? (int)((rke - rks + ATT_BLOCK - 1) / ATT_BLOCK) : 0;
         }
     }
-    if (!is_chain && nst > 0) {
-        load_raw(0);
-        store_tile(0);
-        if (nst > 1) load_raw(1);
+    // the four chains' block maxima are loaded together, then scanned in turn
+    for (int blk = lane; blk < nbt; blk += 64) {
+        float m[CPW];
+#pragma unroll
+        for (int i = 0; i < CPW; i++) {
+            const int ch = wv * CPW + i;
+            const size_t row = (b * a.S + min(qp0 + ch / gq, a.S - 1)) * a.Hq + kvh * gq + ch % gq;
+            m[i] = a.bmax[row * a.nbstride + blk];
+        }
+#pragma unroll
+        for (int i = 0; i < CPW; i++) corr_s[blk * RW_CS + wv * CPW + i] = blk < cnb[i] ? m[i] : 1.0f;
+    }
+    wave_lds_order();
+#pragma unroll
+    for (int i = 0; i < CPW; i++) chain_corr_scan<RW_CS>(cnb[i], corr_s + wv * CPW + i, 1.0f);
+    if (!is_chain) {
+        // tiles 0 and 1 before the first barrier; after barrier t the tile
+        // t + 2 goes to the buffer that tile t - 1 left
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            store_tile(i, raw[i]);
+            load_raw(i + RW_PF, raw[i]);
+        }
+        for (int t0 = 0; t0 < nst; t0 += RW_PF) {
+#pragma unroll
+            for (int i = 0; i < RW_PF; i++) {
+                const int t = t0 + i;
+                if (t >= nst) break;
+                __syncthreads();
+                store_tile(t + 2, raw[(i + 2) % RW_PF]);
+                load_raw(t + 2 + RW_PF, raw[(i + 2) % RW_PF]);
+            }
+        }
+        return;
     }
 
-    float acc[RW_CPW], rs[RW_CPW];
+    // ---- chain waves: chains c0..c0+7 of the workgroup; klen: the keys a
+    // chain accumulates (kmin / kmax over the wave's chains)
+    const int c0 = wv * RW_CPW;
+    int klen[RW_CPW], kmin = INT32_MAX, kmax = 0;
 #pragma unroll
     for (int c = 0; c < RW_CPW; c++) {
-        acc[c] = 0.0f;
-        rs[c] = 0.0f;
-    }
-    const int lr = lane & 15;
-    for (int t = 0; t < nst; t++) {
-        __syncthreads();
-        if (!is_chain) {
-            // buffer (t+1)&1 last held tile t-1, finished before this barrier
-            if (t + 1 < nst) {
-                store_tile(t + 1);
-                if (t + 2 < nst) load_raw(t + 2);
+        klen[c] = 0;
+        const int qp = qp0 + (c0 + c) / gq;
+        if (qp < a.S) {
+            size_t rks, rke, rbl;
+            kv_range<HYBRID>(a, (size_t)qp, rks, rke, rbl);
+            if (rke > rks) {
+                const size_t full = (rke - rks + ATT_BLOCK - 1) / ATT_BLOCK * ATT_BLOCK;
+                klen[c] = (int)(rks + full < rbl ? full : rbl - rks);
             }
-            continue;
+            kmin = min(kmin, klen[c]);
+            kmax = max(kmax, klen[c]);
         }
-        const float* pt = prod + (t & 1) * 64 * RW_PS + lane * RW_PS;
-        const float* wt = wts + (t & 1) * RW_CH * RW_T + (size_t)c0 * RW_T;
+    }
+    f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+    float rs = 0.0f;                               // lane c: the running sum of chain c0 + c
+    const int lc = lane & 7;
+    // this lane's chain's block sums (global) and how many it has
+    const int qpl = min(qp0 + (c0 + lc) / gq, a.S - 1);
+    const float* bsum_l = a.bsum + ((b * a.S + qpl) * a.Hq + kvh * gq + (c0 + lc) % gq) * (size_t)a.nbstride;
+    int nbl = 0;
+    if (qp0 + (c0 + lc) / gq < a.S) {
+        size_t rks, rke, rbl;
+        kv_range<HYBRID>(a, (size_t)qpl, rks, rke, rbl);
+        nbl = rke > rks ? (int)((rke - rks + ATT_BLOCK - 1) / ATT_BLOCK) : 0;
+    }
+    // a block's operands, read from LDS one block ahead of its chain steps
+    struct Blk {
+        f32x4 v[8], cr[2];
+        float w[2][2], bs, crl;
+    };
+    auto read = [&](int blk, Blk& o) {
+        const int buf = (blk >> 1) % RW_NB, jo = (blk & 1) * ATT_BLOCK;
+        const float* pt = prod + buf * 64 * RW_PS + lane * RW_PS + jo;
+        const float* wt = wts + buf * RW_CH * RW_T + ((c0 / 4) * RW_T + jo) * 4 + lane;
+        const int bc = min(blk, nbt - 1) * RW_CS + c0;
+        const f32x4* cr4 = reinterpret_cast<const f32x4*>(corr_s + bc);
+        const float bs = bsum_l[max(min(blk, nbl - 1), 0)];
+        o.bs = blk < nbl ? bs : 0.0f;
+        o.cr[0] = cr4[0];
+        o.cr[1] = cr4[1];
+        o.crl = corr_s[bc + lc];
 #pragma unroll
-        for (int h = 0; h < RW_T / ATT_BLOCK; h++) {
-            const int blk = t * (RW_T / ATT_BLOCK) + h;
-            const int jo = h * ATT_BLOCK;
-            const size_t bs0 = ks + (size_t)blk * ATT_BLOCK;
-            bool all_fast = true;
-            float bse[RW_CPW];
-            int bsz[RW_CPW];
+        for (int q = 0; q < 8; q++) o.v[q] = *reinterpret_cast<const f32x4*>(pt + 4 * q);
 #pragma unroll
-            for (int c = 0; c < RW_CPW; c++) {
-                bse[c] = 0.0f;
-                bsz[c] = 0;
-                if (blk < cnb[c]) {
-                    const float cr = corr_s[(size_t)(c0 + c) * nbmax + blk];
-                    bse[c] = bsum_s[(size_t)(c0 + c) * nbmax + blk];
-                    if (cr != NEG_INF) {
-                        acc[c] = acc[c] * cr;
-                        rs[c] = rs[c] * cr;
-                    }
-                    bsz[c] = (int)((bs0 + ATT_BLOCK < crbl[c] ? bs0 + ATT_BLOCK : crbl[c]) - bs0);
-                    if (bsz[c] != ATT_BLOCK || __builtin_signbit(bse[c])) all_fast = false;
-                } else {
-                    all_fast = false;
-                }
-            }
-            if (blk >= cnb[0] && blk >= cnb[1] && blk >= cnb[2] && blk >= cnb[3]) continue;
-            float pv[ATT_BLOCK];
+        for (int hh = 0; hh < 2; hh++)
 #pragma unroll
-            for (int q = 0; q < ATT_BLOCK / 4; q++) {
-                const float4 v = *reinterpret_cast<const float4*>(pt + jo + 4 * q);
-                pv[4 * q] = v.x;
-                pv[4 * q + 1] = v.y;
-                pv[4 * q + 2] = v.z;
-                pv[4 * q + 3] = v.w;
-            }
-            if (all_fast) {
+            for (int gg = 0; gg < 2; gg++) o.w[hh][gg] = wt[(gg * RW_T + 16 * hh) * 4];
+    };
+    auto run = [&](int blk, const Blk& o) {
+        const int k0 = blk * ATT_BLOCK;
+        if (k0 >= kmax) return;
+        acc[0] = acc[0] * o.cr[0];
+        acc[1] = acc[1] * o.cr[1];
+        rs = rs * o.crl;
+        rs = rs + __builtin_fabsf(o.bs);
+        const bool zeros = __ballot(__builtin_signbit(o.bs)) != 0;
+        int done = zeros ? 0 : min(kmin - k0, ATT_BLOCK);   // keys that all the chains take
+        if (done == ATT_BLOCK) {
+            rw_chain<0>(acc, o.v, o.w[0][0], o.w[0][1], std::make_integer_sequence<int, 16>{});
+            rw_chain<0>(acc, o.v + 4, o.w[1][0], o.w[1][1], std::make_integer_sequence<int, 16>{});
+            return;
+        }
+        done = max(done, 0) & ~3;
+        using four = std::make_integer_sequence<int, 4>;
+        if (done > 0) rw_chain<0>(acc, o.v, o.w[0][0], o.w[0][1], four{});
+        if (done > 4) rw_chain<4>(acc, o.v + 1, o.w[0][0], o.w[0][1], four{});
+        if (done > 8) rw_chain<8>(acc, o.v + 2, o.w[0][0], o.w[0][1], four{});
+        if (done > 12) rw_chain<12>(acc, o.v + 3, o.w[0][0], o.w[0][1], four{});
+        if (done > 16) rw_chain<0>(acc, o.v + 4, o.w[1][0], o.w[1][1], four{});
+        if (done > 20) rw_chain<4>(acc, o.v + 5, o.w[1][0], o.w[1][1], four{});
+        if (done > 24) rw_chain<8>(acc, o.v + 6, o.w[1][0], o.w[1][1], four{});
+        // the rest key by key, from LDS: keys past a chain's end and zero
+        // weights are skipped (an FMA with a zero weight could turn an
+        // accumulator of -0 into +0)
+        const int buf = (blk >> 1) % RW_NB, jo = (blk & 1) * ATT_BLOCK;
+        const float* pt = prod + buf * 64 * RW_PS + lane * RW_PS + jo;
+        const f32x4* wt = reinterpret_cast<const f32x4*>(wts + buf * RW_CH * RW_T) + (c0 / 4) * RW_T + jo;
+        const int end = min(kmax - k0, ATT_BLOCK);
+#pragma unroll 1
+        for (int k = done; k < end; k += 4) {
+            const f32x4 p = *reinterpret_cast<const f32x4*>(pt + k);
+            f32x4 w[4][2];
 #pragma unroll
-                for (int hh = 0; hh < 2; hh++) {
-                    float wvv[RW_CPW];
+            for (int e = 0; e < 4; e++)
 #pragma unroll
-                    for (int c = 0; c < RW_CPW; c++) wvv[c] = wt[c * RW_T + jo + 16 * hh + lr];
-                    rw_chain16(acc, pv + 16 * hh, wvv, std::make_integer_sequence<int, 16>{});
-                }
-            } else {
+                for (int gg = 0; gg < 2; gg++) w[e][gg] = wt[gg * RW_T + k + e];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
 #pragma unroll
                 for (int c = 0; c < RW_CPW; c++) {
-                    if (blk >= cnb[c]) continue;
-                    // keys of a partial block's end, and zero weights, are
-                    // skipped: an FMA with a zero weight could turn an
-                    // accumulator of -0 into +0
-#pragma unroll
-                    for (int hh = 0; hh < 2; hh++) {
-                        const int lim = bsz[c] - 16 * hh;
-                        if (lim <= 0) break;
-                        const float wvv = wt[c * RW_T + jo + 16 * hh + lr];
-                        uint32_t nz = (uint32_t)__ballot(wvv != 0.0f) & 0xFFFFu;   // lanes 0-15: keys
-                        if (lim < 16) nz &= (1u << lim) - 1u;
-                        rw_masked16(acc[c], pv + 16 * hh, wvv, nz, std::make_integer_sequence<int, 16>{});
-                    }
+                    const float x = w[e][c >> 2][c & 3], y = acc[c >> 2][c & 3];
+                    acc[c >> 2][c & 3] = (k0 + k + e < klen[c] && x != 0.0f) ? __builtin_fmaf(p[e], x, y) : y;
                 }
-            }
-#pragma unroll
-            for (int c = 0; c < RW_CPW; c++)
-                if (blk < cnb[c]) rs[c] = rs[c] + __builtin_fabsf(bse[c]);
         }
+    };
+    Blk cur, nxt;
+    for (int t = 0; t < nst; t++) {
+        __syncthreads();                           // tiles t and t + 1 are in LDS
+        if (t == 0) read(0, cur);
+        read(2 * t + 1, nxt);
+        run(2 * t, cur);
+        if (t + 1 < nst) read(2 * t + 2, cur);
+        run(2 * t + 1, nxt);
     }
-    if (!is_chain) return;
     const int dim = sl * 64 + lane;
-    if (dim >= d) return;
 #pragma unroll
     for (int c = 0; c < RW_CPW; c++) {
-        if (qp0 + (c0 + c) / gq >= a.S) continue;
-        uint16_t* ov = a.o + crow[c] * (size_t)d;
-        if (!(rs[c] > 0.0f) || dim >= da) ov[dim] = 0;
-        else ov[dim] = f2h(acc[c] * (1.0f / rs[c]));
+        const float rsc_ = lane_f(rs, c);          // before the lanes past the row leave
+        if (dim >= d || qp0 + (c0 + c) / gq >= a.S) continue;
+        uint16_t* ov = a.o + ((b * a.S + qp0 + (c0 + c) / gq) * a.Hq + kvh * gq + (c0 + c) % gq) * (size_t)d;
+        if (!(rsc_ > 0.0f) || dim >= da) ov[dim] = 0;
+        else ov[dim] = f2h(acc[c >> 2][c & 3] * (1.0f / rsc_));
     }
 }
 
-static size_t rows_smem(int nbmax) { return (size_t)RW_PROD_B + RW_W_B + 2 * (size_t)RW_CH * nbmax * sizeof(float); }
+static size_t rows_smem(int nbmax) { return (size_t)RW_PROD_B + RW_W_B + (size_t)RW_CS * nbmax * sizeof(float); }
 
 // ------------------------------------------------ per-(device, stream) scratch
 static int attn_scratch(void* stream, size_t bytes, void** out) {
@@ -1667,21 +1964,26 @@ static int launch_attention(AttnArgs a, void* stream) {
     a.bsum = a.bmax + rows * a.nbstride;
     const size_t chunks = (maxr + 63) / 64;
     const bool windowed = !HYBRID && a.window > 0 && a.window < a.Skv;
-    // prefill scores: several query rows per wave (16-dim DPP groups, one
-    // scale per 16 dims, 16-byte key rows)
+    // scores of prefill rows and of a decode row: 16-byte key rows, one scale
+    // per 16 dims, whole groups of query heads
     const bool k16 = HYBRID ? ((uintptr_t)a.kc % 16 == 0 && (uintptr_t)a.ks % 4 == 0 && a.qgs % 16 == 0) : true;
-    const bool rows_ok = chunks > 0 && !windowed && (a.d == 64 || a.d == 128) && a.gq <= SQ_NQ &&
-                         SQ_NQ % a.gq == 0 && k16 && (uintptr_t)a.k % 16 == 0;
+    const bool rows_ok = chunks > 0 && !windowed && (a.d == 64 || a.d == 128) && a.gq <= ATT_MAX_GQ &&
+                         ATT_MAX_GQ % a.gq == 0 && k16 && (uintptr_t)a.k % 16 == 0;
     CH_REQUIRE(!a.prep.q_raw || (rows_ok && (size_t)a.B * a.S <= 2 && (a.gq == 1 || a.gq == 2)),
                "decode attention with fused head preparation: needs head_dim 64 or 128, 1 or 2 query heads "
                "per KV head and 16-byte aligned rows");
     if (rows_ok && (size_t)a.B * a.S > 2) {
-        const int qr = SQ_NQ / a.gq;
-        dim3 ga((unsigned)((chunks + 3) / 4), (unsigned)((size_t)a.B * ((a.S + qr - 1) / qr) * a.Hkv));
+        // sub-tiles of query vectors per workgroup: the keys are converted
+        // once for all of them, as long as two workgroups per CU remain
+        const int qr = SM_Q / a.gq;
+        auto grid_y = [&](int n) { return (size_t)a.B * (((size_t)a.S + (size_t)qr * n - 1) / ((size_t)qr * n)) * a.Hkv; };
+        int nsub = 1;
+        while (nsub < 8 && (size_t)qr * nsub < (size_t)a.S && (chunks + 3) / 4 * grid_y(2 * nsub) >= 512) nsub *= 2;
+        dim3 ga((unsigned)((chunks + 3) / 4), (unsigned)grid_y(nsub));
         if (a.d == 64)
-            hipLaunchKernelGGL((attn_scores_rows_kernel<HYBRID, 64, SQ_NQ, 4>), ga, dim3(256), 0, as_stream(stream), a);
+            hipLaunchKernelGGL((attn_scores_mfma_kernel<HYBRID, 64>), ga, dim3(256), 0, as_stream(stream), a, nsub);
         else
-            hipLaunchKernelGGL((attn_scores_rows_kernel<HYBRID, 128, SQ_NQ, 4>), ga, dim3(256), 0, as_stream(stream), a);
+            hipLaunchKernelGGL((attn_scores_mfma_kernel<HYBRID, 128>), ga, dim3(256), 0, as_stream(stream), a, nsub);
         rc = check_launch("attention scores (rows)");
         if (rc) return rc;
     } else if (rows_ok && (a.gq == 1 || a.gq == 2)) {
@@ -1699,8 +2001,8 @@ static int launch_attention(AttnArgs a, void* stream) {
         CH_REQUIRE(nwg < (1u << 31), "attention: decode key range too long");
         dim3 ga((unsigned)nwg);
         auto go = [&](auto kern) { hipLaunchKernelGGL(kern, ga, dim3(64), 0, as_stream(stream), a); };
-        if (a.d == 64) go(attn_scores_rows_kernel<HYBRID, 64, 1, 1>);
-        else go(attn_scores_rows_kernel<HYBRID, 128, 1, 1>);
+        if (a.d == 64) go(attn_scores_row_kernel<HYBRID, 64>);
+        else go(attn_scores_row_kernel<HYBRID, 128>);
         rc = check_launch("attention scores (decode)");
         if (rc) return rc;
     } else if (chunks > 0) {

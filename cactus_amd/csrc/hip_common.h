@@ -158,31 +158,57 @@ __device__ __forceinline__ float exp2_bits(int32_t zi) {
 // fused), one rounding to float.  Relative error of the double result is a
 // few 1e-16, so the float result is the correctly rounded e^x except when
 // e^x lies within ~1e-15 (relative) of a float rounding boundary.
-__device__ __forceinline__ float cactus_expf(float xf) {
-    if (xf != xf) return xf;
-    if (xf > 100.0f) return __builtin_inff();
-    if (xf < -110.0f) return 0.0f;
+// Branch-free, so that independent calls interleave: beyond the clamps e^x
+// rounds to 0 or overflows to infinity by itself, and 2^k is applied by
+// v_ldexp_f64 (exact: the double stays normal).  The polynomial's constants
+// come from scalar registers (the compiler otherwise copies each into the
+// FMA's destination first, an instruction per step).
+__device__ __forceinline__ double fma_sc(double a, double b, double c) {
+    double o;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(o) : "v"(a), "v"(b), "s"(c));
+    return o;
+}
+// N values side by side: their steps alternate, so a step does not wait for
+// the one before it
+template <int N>
+__device__ __forceinline__ void cactus_expf_n(const float (&xf)[N], float (&out)[N]) {
     const double LN2_HI = 6.93147180369123816490e-01;
     const double LN2_LO = 1.90821492927058770002e-10;
-    double x = (double)xf;
-    double k = __builtin_rint(x * 1.44269504088896338700e+00);
-    double r = __builtin_fma(-k, LN2_HI, x);
-    r = __builtin_fma(-k, LN2_LO, r);
-    double p = 1.0 / 479001600.0;
-    p = __builtin_fma(p, r, 1.0 / 39916800.0);
-    p = __builtin_fma(p, r, 1.0 / 3628800.0);
-    p = __builtin_fma(p, r, 1.0 / 362880.0);
-    p = __builtin_fma(p, r, 1.0 / 40320.0);
-    p = __builtin_fma(p, r, 1.0 / 5040.0);
-    p = __builtin_fma(p, r, 1.0 / 720.0);
-    p = __builtin_fma(p, r, 1.0 / 120.0);
-    p = __builtin_fma(p, r, 1.0 / 24.0);
-    p = __builtin_fma(p, r, 1.0 / 6.0);
-    p = __builtin_fma(p, r, 0.5);
-    p = __builtin_fma(p, r, 1.0);
-    p = __builtin_fma(p, r, 1.0);
-    uint64_t sb = (uint64_t)((int64_t)k + 1023) << 52;
-    return (float)(p * __builtin_bit_cast(double, sb));
+    double r[N], k[N], p[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) r[i] = (double)__builtin_fminf(__builtin_fmaxf(xf[i], -110.0f), 100.0f);
+#pragma unroll
+    for (int i = 0; i < N; i++) k[i] = __builtin_rint(r[i] * 1.44269504088896338700e+00);
+#pragma unroll
+    for (int i = 0; i < N; i++) r[i] = __builtin_fma(-k[i], LN2_HI, r[i]);
+#pragma unroll
+    for (int i = 0; i < N; i++) r[i] = __builtin_fma(-k[i], LN2_LO, r[i]);
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = 1.0 / 479001600.0;
+    constexpr double C[9] = {1.0 / 39916800.0, 1.0 / 3628800.0, 1.0 / 362880.0, 1.0 / 40320.0, 1.0 / 5040.0,
+                             1.0 / 720.0,      1.0 / 120.0,     1.0 / 24.0,     1.0 / 6.0};
+#pragma unroll
+    for (int j = 0; j < 9; j++)
+#pragma unroll
+        for (int i = 0; i < N; i++) p[i] = fma_sc(p[i], r[i], C[j]);
+    // 0.5 and 1.0 are inline constants
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = __builtin_fma(p[i], r[i], 0.5);
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = __builtin_fma(p[i], r[i], 1.0);
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = __builtin_fma(p[i], r[i], 1.0);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const float e = (float)__builtin_ldexp(p[i], (int)k[i]);
+        out[i] = xf[i] != xf[i] ? xf[i] : e;
+    }
+}
+__device__ __forceinline__ float cactus_expf(float xf) {
+    const float x[1] = {xf};
+    float o[1];
+    cactus_expf_n<1>(x, o);
+    return o[0];
 }
 
 // fast_exp_f32x4 lane (reference kernel_utils.h:108-141)
@@ -283,6 +309,28 @@ __device__ __forceinline__ float half_wave_max(float v) {
     float x = v, y = v;
     asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y));
     return __builtin_fmaxf(x, y);
+}
+// half_wave_max of four values at once, in place: each DPP step reads its
+// source in the instruction itself, and the four values' turns between two
+// steps of one value cover the wait a DPP source needs after its write.
+__device__ __forceinline__ void half_wave_max4(float (&v)[4]) {
+    float a = v[0], b = v[1], c = v[2], d = v[3];
+#define CH_MAX4(CTRL)                                                                     \
+    "v_max_f32_dpp %0, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                    \
+    "v_max_f32_dpp %1, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                    \
+    "v_max_f32_dpp %2, %2, %2 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                    \
+    "v_max_f32_dpp %3, %3, %3 " CTRL " row_mask:0xf bank_mask:0xf\n\t"
+    asm volatile("s_nop 1\n\t" CH_MAX4("quad_perm:[1,0,3,2]") CH_MAX4("quad_perm:[2,3,0,1]")
+                     CH_MAX4("row_half_mirror") CH_MAX4("row_mirror")
+                 : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+#undef CH_MAX4
+    float w[4] = {a, b, c, d};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float x = w[i], y = w[i];
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y));
+        v[i] = __builtin_fmaxf(x, y);
+    }
 }
 __device__ __forceinline__ float wave_max(float v) {
     v = __builtin_fmaxf(v, dpp_move_keep<0xB1>(v));    // quad_perm [1,0,3,2]

@@ -504,6 +504,9 @@ def test_attention_f16_mask_noncausal(dev, orc):
     (128, 1500, 128, 16, 8, 128),  # prefill chunk deep into the context
     (50, 300, 50, 8, 1, 128),      # 8 query heads per kv head, prefill
     (33, 64, 33, 4, 4, 64),        # one query head per kv head, prefill
+    (4, 61, 4, 8, 1, 64),          # one 32-vector tile, a block ending inside the first new rows
+    (70, 5, 70, 2, 2, 128),        # several tiles, most keys fp16
+    (600, 40, 600, 4, 2, 64),      # several sub-tiles per workgroup
 ])
 def test_attention_hybrid(dev, orc, S, cache, new, Hq, Hkv, d):
     _attention_hybrid(dev, orc, S, cache, new, Hq, Hkv, d, 1.0)
