@@ -674,7 +674,7 @@ size_t CactusGraph::compute_shared_matmuls(size_t i) {
     const BufferDesc& a = node(n0.inputs[0]).out;
     const BufferDesc& b0 = node(n0.inputs[1]).out;
     const size_t K = a.shape.back(), M = a.total_size / K;
-    if (M < 32) return 0;   // decode sizes: the fused GEMV per node
+    if (M < kBatchedRows) return 0;   // decode sizes: the fused GEMV per node
     size_t count = 1;
     while (count < 3 && i + count < nodes_.size()) {
         const GraphNode& nj = *nodes_[i + count];

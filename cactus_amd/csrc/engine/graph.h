@@ -18,6 +18,11 @@
 
 namespace cactus {
 
+// Rows from which the grouped matmuls of FP16 activations run on the matrix
+// cores whatever their format: the nodes in front of them then quantize the
+// rows once for all their consumers, and consumers of one input share a launch.
+constexpr size_t kBatchedRows = 5;
+
 // graph.h:99-104 (same order: INT8, FP16, FP32, INT4)
 enum class Precision { INT8, FP16, FP32, INT4 };
 

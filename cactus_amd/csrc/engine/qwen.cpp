@@ -310,14 +310,14 @@ size_t QwenModel::shared_matmul_input(size_t x) {
     CactusGraph& g = *cur_;
     const BufferDesc& b = g.get_output_buffer(x);
     if (b.precision == Precision::INT8) return x;   // already codes with row scales
-    return b.shape[0] >= 32 ? g.quantize_activations(x) : x;
+    return b.shape[0] >= kBatchedRows ? g.quantize_activations(x) : x;
 }
 
 // The RMSNorm in front of q/k/v and of gate/up feeds only those matmuls: at
 // prefill sizes it is one node with their row quantization.
 size_t QwenModel::norm_for_matmuls(size_t h, size_t weight) {
     CactusGraph& g = *cur_;
-    if (g.get_output_buffer(h).shape[0] >= 32) return g.rms_norm_quantize(h, weight, cfg_.eps);
+    if (g.get_output_buffer(h).shape[0] >= kBatchedRows) return g.rms_norm_quantize(h, weight, cfg_.eps);
     return g.rms_norm(h, weight, cfg_.eps);
 }
 
@@ -371,7 +371,7 @@ size_t QwenModel::build_mlp(size_t x, uint32_t l, size_t residual) {
     size_t up = g.matmul(xq, L.n_up, true);
     // at prefill sizes the SwiGLU product is one node with the down
     // projection's row quantization
-    if (g.get_output_buffer(gate).shape[0] >= 32) {
+    if (g.get_output_buffer(gate).shape[0] >= kBatchedRows) {
         const size_t q = g.silu_mul_quantize(gate, up);
         if (residual != NO_RESIDUAL) return g.matmul_add(q, L.n_down, residual);
         return g.matmul(q, L.n_down, true);
@@ -388,7 +388,7 @@ size_t QwenModel::build_block(size_t h, uint32_t l, size_t pos) {
     const QwenLayer& L = layers_[l];
     size_t x = norm_for_matmuls(h, L.n_input_norm);
     // at prefill sizes the residual adds ride on the o-proj and down matmuls
-    const bool fuse = g.get_output_buffer(h).shape[0] >= 32;
+    const bool fuse = g.get_output_buffer(h).shape[0] >= kBatchedRows;
     size_t h1 = build_attention(x, l, pos, fuse ? h : NO_RESIDUAL);
     if (!fuse) h1 = g.add(h, h1);
     size_t x2 = norm_for_matmuls(h1, L.n_post_norm);

@@ -594,8 +594,15 @@ static int gemm_scratch(hipStream_t st, size_t bytes, void** out) {
     return stream_scratch(SCR_GEMM_ACT, st, bytes, false, out);
 }
 
-// Rows from which the MFMA path pays off over the streaming GEMV.
-constexpr size_t GEMM_MIN_M = 32;
+// Rows from which the MFMA path pays off over the streaming GEMV, which takes
+// four rows per pass over the weights.  Measured (us, GEMV / MFMA with the row
+// quantization): INT8 K=1024 N=2048 M=2 6.2 / 6.7, M=4 8.4 / 6.7, M=5 13.6 /
+// 6.7, M=19 40 / 6.9, M=31 66 / 7.0; INT4 K=3072 N=1024 M=4 10.5 / 11.7, M=5
+// 16.5 / 11.7.  Pre-quantized rows skip the 2-4 us quantization launch.
+constexpr size_t GEMM_MIN_M_INT8 = 3, GEMM_MIN_M_INT4 = 5, GEMM_MIN_M_CODES = 3;
+// Below this many rows the FP16 forms never needed device memory of their
+// own: inside a graph capture that would have to allocate they keep the GEMV.
+constexpr size_t GEMM_NOALLOC_M = 32;
 
 // Returns *handled = false when the shape is left to the GEMV path.
 // Activation codes ([M][K] int8, padded to 256 bytes) and row scales
@@ -606,10 +613,14 @@ int gemm_grouped_mfma(const uint16_t* A16, const int8_t* A8, const float* As, co
                       const uint16_t* Bs, uint16_t* C, size_t M, size_t K, size_t N, size_t gs,
                       bool int4, hipStream_t st, bool* handled, const uint16_t* R, void* ext_scratch) {
     *handled = false;
-    if (M < GEMM_MIN_M || gs % 32 != 0 || N < 32) return CACTUS_HIP_OK;
+    if (M < (A16 ? (int4 ? GEMM_MIN_M_INT4 : GEMM_MIN_M_INT8) : GEMM_MIN_M_CODES)) return CACTUS_HIP_OK;
+    if (gs % 32 != 0 || N < 32) return CACTUS_HIP_OK;
     if (((uintptr_t)B & 15) != 0) return CACTUS_HIP_OK;
     if (!A16 && (((uintptr_t)A8 & 15) != 0)) return CACTUS_HIP_OK;
     if (M >= (1u << 30) || N >= (1u << 30) || K >= (1u << 20)) return CACTUS_HIP_OK;
+    if (A16 && !ext_scratch && M < GEMM_NOALLOC_M &&
+        !stream_scratch_ready(SCR_GEMM_ACT, st, gemm_act_scratch_bytes(M, K)))
+        return CACTUS_HIP_OK;
     const int8_t* Aq = A8;
     const float* Asc = As;
     if (A16) {
@@ -657,7 +668,7 @@ int gemm_grouped_mfma_multi(const int8_t* A8, const float* As, int np, const uin
                             const uint16_t* const* Bs, uint16_t* const* C, const size_t* N, size_t M, size_t K,
                             size_t gs, bool int4, hipStream_t st, bool* handled) {
     *handled = false;
-    if (np < 1 || np > 3 || M < GEMM_MIN_M || gs % 32 != 0) return CACTUS_HIP_OK;
+    if (np < 1 || np > 3 || M < GEMM_MIN_M_CODES || gs % 32 != 0) return CACTUS_HIP_OK;
     if (((uintptr_t)A8 & 15) != 0 || M >= (1u << 30) || K >= (1u << 20)) return CACTUS_HIP_OK;
     for (int p = 0; p < np; p++)
         if (N[p] < 32 || N[p] >= (1u << 30) || ((uintptr_t)B[p] & 15) != 0 || ((uintptr_t)Bs[p] & 3) != 0)

@@ -243,6 +243,8 @@ __global__ void __launch_bounds__(GEMV_THREADS) gemv_grouped_kernel(GemvArgs a, 
     }
 }
 
+constexpr size_t GEMV_MAX_LDS = 60 * 1024;
+
 static size_t gemv_smem(int MR, int K, int rows, int G) {
     size_t s = (size_t)((MR * K + 15) & ~15);
     s += (size_t)2 * MR * rows * G * 4;
@@ -526,12 +528,14 @@ template <bool F16ACT, bool INT4>
 static int launch_gemv(GemvArgs a, size_t batch, hipStream_t st) {
     const int G = a.K / a.gs;
     const int cpr = INT4 ? a.K / 32 : a.K / 16;
-    const int MR = a.M >= 4 ? 4 : (a.M >= 2 ? 2 : 1);
+    // rows per pass: three rows take one pass of four unless its codes no
+    // longer fit the LDS
+    const int MR = a.M >= 4 || (a.M == 3 && gemv_smem(4, a.K, 1, G) <= GEMV_MAX_LDS) ? 4 : (a.M >= 2 ? 2 : 1);
     int wch = 0, wrows = 0;
     // INT4 with 32-wide groups: one group per chunk, fp32 epilogue operands
     const bool fe = INT4 && a.gs == 32;
     if (pick_wave_tile(cpr, a.N, batch, &wch, &wrows) &&
-        gemv_wave_smem(MR, a.K, wrows, G, fe) <= 60 * 1024) {
+        gemv_wave_smem(MR, a.K, wrows, G, fe) <= GEMV_MAX_LDS) {
         // wave tiles per workgroup: 4 (one per wave) up to 4 * cap.  Every
         // workgroup quantizes the activation row once, so INT4 rows (the
         // K = 3072 MLP down shape) take more tiles per workgroup: swept on
@@ -563,8 +567,8 @@ static int launch_gemv(GemvArgs a, size_t batch, hipStream_t st) {
     if (rows < 1) rows = 1;
     if (rows > a.N) rows = a.N;
     while (rows > 1 && (size_t)ceil_div(a.N, rows) * batch < 1024) rows = (rows + 1) / 2;
-    while (rows > 1 && gemv_smem(MR, a.K, rows, G) > 60 * 1024) rows = (rows + 1) / 2;
-    if (gemv_smem(MR, a.K, rows, G) > 60 * 1024 || rows * cpr > 8 * GEMV_THREADS)
+    while (rows > 1 && gemv_smem(MR, a.K, rows, G) > GEMV_MAX_LDS) rows = (rows + 1) / 2;
+    if (gemv_smem(MR, a.K, rows, G) > GEMV_MAX_LDS || rows * cpr > 8 * GEMV_THREADS)
         return fail(CACTUS_HIP_EUNSUPPORTED, "grouped matmul: K too large for the GEMV path");
     const int chunks = (rows * cpr + GEMV_THREADS - 1) / GEMV_THREADS;
     const int ch = chunks <= 1 ? 1 : chunks <= 2 ? 2 : chunks <= 4 ? 4 : chunks <= 6 ? 6 : 8;
@@ -584,6 +588,12 @@ static int launch_gemv(GemvArgs a, size_t batch, hipStream_t st) {
         if (rc) return rc;
     }
     return CACTUS_HIP_OK;
+}
+
+// whether launch_gemv takes the shape (its smallest tile, one weight row)
+static bool gemv_takes(size_t M, size_t K, size_t gs, bool int4) {
+    const int MR = M >= 4 ? 4 : (M >= 2 ? 2 : 1);
+    return gemv_smem(MR, (int)K, 1, (int)(K / gs)) <= GEMV_MAX_LDS && K / (int4 ? 32 : 16) <= 8 * GEMV_THREADS;
 }
 
 static bool is_pow2(size_t v) { return v && !(v & (v - 1)); }
@@ -630,7 +640,10 @@ int grouped_dispatch(const uint16_t* A16, const int8_t* A8, const float* As,
     CH_REQUIRE(B && Bs && C && (A16 || (A8 && As)), "grouped matmul: null pointer");
     CH_REQUIRE(((uintptr_t)B & 15) == 0, "grouped matmul: weights must be 16-byte aligned");
     bool handled = false;
-    rc = gemm_grouped_mfma(A16, A8, As, B, Bs, C, M, K, N, gs, int4, st, &handled, R, ext_scratch);
+    // few rows with a K beyond the GEMV stay refused below, whichever kernel
+    // serves their sizes
+    if (M >= 32 || gemv_takes(M, K, gs, int4))
+        rc = gemm_grouped_mfma(A16, A8, As, B, Bs, C, M, K, N, gs, int4, st, &handled, R, ext_scratch);
     if (rc || handled) return rc;
     GemvArgs a{};
     a.A16 = A16; a.A8 = A8; a.As = As; a.B = B; a.Bs = Bs; a.C = C;
@@ -729,7 +742,9 @@ int cactus_hip_matmul_grouped_multi(const int8_t* A, const float* A_scales, size
     }
     const hipStream_t st = as_stream(stream);
     bool handled = false;
-    int rc = gemm_grouped_mfma_multi(A, A_scales, (int)count, bp, B_scales, C, N, M, K, group_size, int4 != 0, st,
+    int rc = CACTUS_HIP_OK;
+    if (M >= 32 || gemv_takes(M, K, group_size, int4 != 0))
+        rc = gemm_grouped_mfma_multi(A, A_scales, (int)count, bp, B_scales, C, N, M, K, group_size, int4 != 0, st,
                                      &handled);
     if (rc || handled) return rc;
     // one launch per problem: the same per-output arithmetic

@@ -65,6 +65,9 @@ enum ScratchKind {
     SCR_KINDS
 };
 int stream_scratch(int kind, void* stream, size_t bytes, bool zero, void** out);
+// whether stream_scratch can serve the request without allocating inside a
+// graph capture (which the capture mode may refuse)
+bool stream_scratch_ready(int kind, void* stream, size_t bytes);
 // frees every scratch buffer of `stream` (all devices) after synchronizing it
 int stream_scratch_release(void* stream);
 

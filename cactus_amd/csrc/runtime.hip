@@ -117,6 +117,17 @@ int stream_scratch(int kind, void* stream, size_t bytes, bool zero, void** out) 
     return CACTUS_HIP_OK;
 }
 
+bool stream_scratch_ready(int kind, void* stream, size_t bytes) {
+    const hipStream_t st = as_stream(stream);
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (!st || hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusActive) return true;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lk(g_scr_mu);
+    const auto it = g_scr.find(std::make_pair(dev, stream));
+    return it != g_scr.end() && it->second.cur[kind].ptr && it->second.cur[kind].bytes >= bytes;
+}
+
 int stream_scratch_release(void* stream) {
     std::lock_guard<std::mutex> lk(g_scr_mu);
     bool synced = false;

@@ -191,6 +191,59 @@ def test_int32_accumulator_exact_mfma(dev, orc, M, N):
     assert (got == acc).all()
 
 
+@pytest.mark.parametrize("int4", [False, True])
+@pytest.mark.parametrize("M,K,N,gs", [(2, 256, 33, 32), (3, 1024, 2048, 32), (4, 128, 32, 64), (5, 640, 100, 32),
+                                      (16, 256, 31, 32), (17, 384, 129, 128), (19, 1024, 2048, 32), (31, 96, 1000, 32),
+                                      (3, 12288, 64, 32)])
+def test_matmul_few_rows(dev, orc, M, K, N, gs, int4):
+    """Row counts around the GEMV / matrix-core boundary, narrow and ragged N,
+    K off the stage size, a K whose codes fit the LDS two rows at a time."""
+    say("matmul few rows", M, K, N, gs, int4)
+    rng = np.random.default_rng(M + K + N)
+    x = activations(rng, M, K)
+    rq, rs = orc.quantize_activations(x)
+    if int4:
+        codes, B, Bs = grouped_int4_weights(rng, N, K, gs)
+        ref = orc.matmul_int4(rq, rs, B, Bs, gs)
+    else:
+        B, Bs = grouped_int8_weights(rng, N, K, gs)
+        ref = orc.matmul_int8(rq, rs, B, Bs, gs)
+    name = "cactus_hip_matmul_int4" if int4 else "cactus_hip_matmul_int8"
+    Bp, Bsp = dev.put(B), dev.put(Bs)
+    C, C2 = dev.empty(M * N * 2), dev.empty(M * N * 2)
+    dev.cm.call(name, dev.put(rq), dev.put(rs), Bp, Bsp, C.ptr, M, K, N, gs, None)
+    dev.cm.call(name + "_f16act", dev.put(x), Bp, Bsp, C2.ptr, M, K, N, gs, None)
+    assert_bits(dev.get(C, np.uint16, (M, N)), ref, "pre-quantized")
+    assert_bits(dev.get(C2, np.uint16, (M, N)), ref, "f16act")
+
+
+def test_matmul_few_rows_captured_cold(dev, orc):
+    """Eight rows captured into a graph as the stream's first call: no device
+    memory is taken inside the capture; every replay equals the oracle."""
+    say("matmul few rows captured")
+    M, K, N, gs = 8, 1024, 512, 32
+    rng = np.random.default_rng(8)
+    x = activations(rng, M, K)
+    B, Bs = grouped_int8_weights(rng, N, K, gs)
+    ref = orc.matmul_int8(*orc.quantize_activations(x), B, Bs, gs)
+    xp, Bp, Bsp, C = dev.put(x), dev.put(B), dev.put(Bs), dev.empty(M * N * 2)
+    st = dev.cm.Stream()
+    dev.cm.call("cactus_hip_graph_capture_begin", st.handle)
+    dev.cm.call("cactus_hip_matmul_int8_f16act", xp, Bp, Bsp, C.ptr, M, K, N, gs, st.handle)
+    g = ctypes.c_void_p()
+    dev.cm.call("cactus_hip_graph_capture_end", st.handle, ctypes.byref(g))
+    for rep in range(3):
+        dev.cm.call("cactus_hip_memset", C.ptr, 0, M * N * 2, st.handle)
+        dev.cm.call("cactus_hip_graph_launch", g.value, st.handle)
+        st.sync()
+        assert_bits(dev.get(C, np.uint16, (M, N)), ref, "replay %d" % rep)
+        # an eager call in between takes the stream's scratch
+        dev.cm.call("cactus_hip_matmul_int8_f16act", xp, Bp, Bsp, C.ptr, M, K, N, gs, st.handle)
+        st.sync()
+        assert_bits(dev.get(C, np.uint16, (M, N)), ref, "eager %d" % rep)
+    dev.cm.call("cactus_hip_graph_destroy", g.value)
+
+
 def test_matmul_int8_batched(dev, orc):
     say("matmul_int8_f16act_batched")
     rng = np.random.default_rng(4)
