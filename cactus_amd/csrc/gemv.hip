@@ -26,6 +26,7 @@ struct GemvArgs {
     const uint8_t* B;       // weights, int8 [N][K] or packed int4 [N][K/2]
     const uint16_t* Bs;     // fp16 group scales [N][G]
     uint16_t* C;            // fp16 out [M][N]
+    const uint16_t* R;      // fp16 residual added to the output (the add node), laid out as C, or null
     int M, K, N, gs, rows, tiles;
     size_t sA, sB, sBs, sC; // batch strides: elements of A/Bs/C, bytes of B
 };
@@ -233,10 +234,13 @@ __global__ void __launch_bounds__(GEMV_THREADS) gemv_grouped_kernel(GemvArgs a, 
         // reference epilogue, one thread per output of this tile
         for (int o = tid; o < mr * nr; o += GEMV_THREADS) {
             const int m = o / nr, r = o % nr;
+            const size_t co = bi * a.sC + (size_t)(m0 + m) * a.N + n0 + r;
+            const uint16_t res = a.R ? a.R[co] : (uint16_t)0;   // in flight behind the chain
             const int32_t* ag = accb + (m * rows + r) * G;
             const uint16_t* sg = sclb + r * G;
             const float rs = group_epilogue(ag, sg, G);
-            a.C[bi * a.sC + (size_t)(m0 + m) * a.N + n0 + r] = f2h(rs * rsc[m]);
+            const uint16_t c = f2h(rs * rsc[m]);
+            a.C[co] = a.R ? hadd(c, res) : c;
         }
 #pragma unroll
         for (int i = 0; i < CH; i++) wcur[i] = wnext[i];
@@ -416,6 +420,8 @@ __global__ void __launch_bounds__(GEMV_THREADS) gemv_wave_kernel(GemvArgs a, int
         // reference epilogue, one lane per output of this tile
         for (int o = lane; o < mr * nr; o += 64) {
             const int m = o / nr, r = o - (o / nr) * nr;
+            const size_t co = bi * a.sC + (size_t)(m0 + m) * a.N + n0 + r;
+            const uint16_t res = a.R ? a.R[co] : (uint16_t)0;   // in flight behind the chain
             float rs;
             if constexpr (FE) {
                 rs = group_epilogue_f(accf + (m * rows + r) * Gs, sclf + r * Gs, G);
@@ -429,7 +435,8 @@ __global__ void __launch_bounds__(GEMV_THREADS) gemv_wave_kernel(GemvArgs a, int
 #pragma unroll
             for (int mm = 1; mm < MR; mm++)
                 if (m == mm) s = rsm[mm];
-            a.C[bi * a.sC + (size_t)(m0 + m) * a.N + n0 + r] = f2h(rs * s);
+            const uint16_t c = f2h(rs * s);
+            a.C[co] = a.R ? hadd(c, res) : c;
         }
         wave_lds_order();
     }
@@ -621,12 +628,6 @@ int gemm_grouped_mfma_multi(const int8_t* A8, const float* As, int np, const uin
                             const uint16_t* const* Bs, uint16_t* const* C, const size_t* N, size_t M, size_t K,
                             size_t gs, bool int4, hipStream_t st, bool* handled);
 
-// C[i] = fp16(C[i] + R[i]): the residual add node after a small-M matmul
-__global__ void add_residual_kernel(uint16_t* C, const uint16_t* R, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        C[i] = hadd(C[i], R[i]);
-}
-
 // ext_scratch: caller-provided device memory for the MFMA path's activation
 // codes and row scales (at least gemm_act_scratch_bytes(M, K)), or null for
 // the library's own per-stream buffer.
@@ -646,19 +647,11 @@ int grouped_dispatch(const uint16_t* A16, const int8_t* A8, const float* As,
         rc = gemm_grouped_mfma(A16, A8, As, B, Bs, C, M, K, N, gs, int4, st, &handled, R, ext_scratch);
     if (rc || handled) return rc;
     GemvArgs a{};
-    a.A16 = A16; a.A8 = A8; a.As = As; a.B = B; a.Bs = Bs; a.C = C;
+    a.A16 = A16; a.A8 = A8; a.As = As; a.B = B; a.Bs = Bs; a.C = C; a.R = R;
     a.M = (int)M; a.K = (int)K; a.N = (int)N; a.gs = (int)gs;
     a.sA = M * K; a.sB = 0; a.sBs = 0; a.sC = 0;
-    if (A16) rc = int4 ? launch_gemv<true, true>(a, 1, st) : launch_gemv<true, false>(a, 1, st);
-    else rc = int4 ? launch_gemv<false, true>(a, 1, st) : launch_gemv<false, false>(a, 1, st);
-    // small M: the residual add runs as its own kernel, in place on C
-    if (rc == 0 && R) {
-        const size_t n = M * N;
-        const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 65535);
-        hipLaunchKernelGGL(add_residual_kernel, dim3(blocks), dim3(256), 0, st, C, R, n);
-        rc = check_launch("matmul_add (residual)");
-    }
-    return rc;
+    if (A16) return int4 ? launch_gemv<true, true>(a, 1, st) : launch_gemv<true, false>(a, 1, st);
+    return int4 ? launch_gemv<false, true>(a, 1, st) : launch_gemv<false, false>(a, 1, st);
 }
 }  // namespace cactus_hip
 
