@@ -224,6 +224,54 @@ __global__ void __launch_bounds__(256) attn_scores_kernel(AttnArgs a_in) {
     }
 }
 
+// ------------------------------------------------ value product tiles
+// The decode value chains stream fp32 products (float)code * scale from tiles
+// (chain_stream.hip).  A call that brings no tiles builds them in scratch:
+// one wave per 64-key x 64-dim tile, 4 keys x 4 dims per lane and step, every
+// load in flight before the first product, whole kilobytes written per step.
+// 4096 keys of 8 heads of 128 dims (4 MB read, 17 MB written) run beside the
+// scores on CUs those leave idle; chains that convert the cache themselves
+// took 42 us there, the streamed ones 20.
+__device__ __forceinline__ void value_tile(const AttnArgs& a, int kvh, int sl, size_t t) {
+    const int lane = threadIdx.x & 63, d = a.d, nsl = (d + 63) / 64;
+    const int dq = lane & 15, dim0 = sl * 64 + dq * 4;
+    const bool live = dim0 < d;                        // d % 8 == 0: whole quads
+    const int dim = live ? dim0 : 0, grp = (dim / 8) * 8 / a.qgs;
+    uint32_t c[16];
+    float s[16];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const size_t key = min(t * SH_TILE_KEYS + 16 * j + 4 * (lane >> 4) + e, a.cache_len - 1);
+            c[4 * j + e] = *reinterpret_cast<const uint32_t*>(a.vc + (key * a.Hkv + kvh) * d + dim);
+            s[4 * j + e] = a.vs[(key * a.Hkv + kvh) * a.nqg + grp];
+        }
+    float* out = const_cast<float*>(a.vsh) + sh_index(kvh, nsl, sl, a.sh_ntile, t * SH_TILE_KEYS, 0);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            f32x4 p;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                p[e] = live ? (float)(int8_t)((c[4 * j + e] >> (8 * x)) & 0xFF) * s[4 * j + e] : 0.0f;
+            *reinterpret_cast<f32x4*>(out + (4 * j + (lane >> 4)) * 256 + (dq * 4 + x) * 4) = p;
+        }
+}
+
+// workgroup i -> tile: kv head h's tiles on XCD h % 8, where its chains run
+__device__ __forceinline__ void value_tile_wg(const AttnArgs& a, unsigned i) {
+    const int nsl = (a.d + 63) / 64;
+    const unsigned per = (unsigned)(nsl * a.sh_ntile), j = i >> 3;
+    const int kvh = (int)((i & 7) + 8 * (j / per));
+    if (kvh < a.Hkv) value_tile(a, kvh, (int)(j % per % nsl), j % per / nsl);
+}
+static unsigned value_tile_wgs(const AttnArgs& a) {
+    return 8u * (unsigned)((a.Hkv + 7) / 8) * (unsigned)((size_t)((a.d + 63) / 64) * a.sh_ntile);
+}
+__global__ void __launch_bounds__(64) value_tiles_kernel(AttnArgs a) { value_tile_wg(a, blockIdx.x); }
+
 // ------------------------------------------------ kernel A, decode row
 // One query row of up to two heads per kv head: a one-wave workgroup per 64
 // keys and query head.  A lane owns one key, whose whole INT8 row is loaded
@@ -250,10 +298,17 @@ __device__ __forceinline__ void sq_group16(float (&acc)[NQ][8], const float (&qv
 }
 
 // the gq heads of a kv head in gq workgroups per chunk (hsplit)
-template <bool HYBRID, int D>
+// (TILES: workgroups from tile_first on build value product tiles)
+template <bool HYBRID, int D, bool TILES = false>
 __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
     constexpr int NQ = 1;                              // query vectors per wave
     const AttnArgs a = resolve(a_in);
+    if constexpr (TILES) {
+        if (blockIdx.x >= a.tile_first) {
+            value_tile_wg(a, blockIdx.x - a.tile_first);
+            return;
+        }
+    }
     __shared__ float qsh[NQ][D];
     __shared__ __align__(16) float wsh[NQ][64];
     __shared__ float msh[NQ][2];
@@ -1927,6 +1982,9 @@ static int attn_scratch(void* stream, size_t bytes, void** out) {
     return stream_scratch(SCR_ATTN, stream, bytes, false, out);
 }
 
+// scratch a call may take for its product tiles (32768 keys of 16 heads of 128 dims)
+constexpr size_t TILES_MAX_BYTES = (size_t)256 << 20;
+
 template <bool HYBRID>
 static int launch_attention(AttnArgs a, void* stream) {
     // largest key range over the launch (query 0 .. S-1)
@@ -1963,6 +2021,26 @@ static int launch_attention(AttnArgs a, void* stream) {
     a.bmax = reinterpret_cast<float*>(static_cast<char*>(scratch) + wbytes);
     a.bsum = a.bmax + rows * a.nbstride;
     const size_t chunks = (maxr + 63) / 64;
+    // a decode call over an INT8 cache without product tiles: built in
+    // scratch, which the streamed chains more than pay for at every length
+    // (us per call, 16 / 8 heads of 128 dims: 64 keys 14.6 -> 10.9, 520 17.6
+    // -> 13.2, 4096 50.2 -> 33.3)
+    bool tiles = false;
+    if constexpr (HYBRID) {
+        const size_t nt = (a.cache_len + a.new_len + SH_TILE_KEYS - 1) / SH_TILE_KEYS;
+        const size_t bytes = (size_t)a.Hkv * ((a.d + 63) / 64) * nt * SH_TILE_FLOATS * sizeof(float);
+        if (!a.vsh && !a.dyn && a.B == 1 && a.S <= 2 && a.new_len <= 2 && a.d % 8 == 0 &&
+            (a.qgs % 64 == 0 || a.qgs >= a.d) && (uintptr_t)a.vc % 4 == 0 && (uintptr_t)a.vs % 4 == 0 &&
+            a.cache_len > 0 && bytes <= TILES_MAX_BYTES &&
+            stream_scratch_ready(SCR_ATTN_TILES, stream, bytes)) {
+            void* p = nullptr;
+            rc = stream_scratch(SCR_ATTN_TILES, stream, bytes, false, &p);
+            if (rc) return rc;
+            a.vsh = static_cast<const float*>(p);
+            a.sh_ntile = nt;
+            tiles = true;
+        }
+    }
     const bool windowed = !HYBRID && a.window > 0 && a.window < a.Skv;
     // scores of prefill rows and of a decode row: 16-byte key rows, one scale
     // per 16 dims, whole groups of query heads
@@ -1986,23 +2064,31 @@ static int launch_attention(AttnArgs a, void* stream) {
             hipLaunchKernelGGL((attn_scores_mfma_kernel<HYBRID, 128>), ga, dim3(256), 0, as_stream(stream), a, nsub);
         rc = check_launch("attention scores (rows)");
         if (rc) return rc;
-    } else if (rows_ok && (a.gq == 1 || a.gq == 2)) {
+    } else if (rows_ok) {
         // decode: one query row, its gq heads per wave, one wave per 64 keys
         // (with the fused head preparation, one more workgroup per kv head
         // appends the step's key and value)
         // workgroups of kv head h on XCD h % 8, where the chain kernel's are;
-        // two query heads per kv head split over two workgroups per chunk
-        // (consecutive, so on one XCD: the second reads the key rows from
-        // its L2), which halves each wave's dot and weight work
+        // a kv head's query heads each take a workgroup per chunk
+        // (consecutive, so on one XCD: all but the first read the key rows
+        // from its L2), so a wave's dot and weight work is one head's (with
+        // 8 heads per kv head in one wave the whole call took 35 us at 64 keys)
         a.hsplit = a.gq;
         a.xcd_chunks = (int)(chunks + (a.prep.q_raw ? 1 : 0)) * a.hsplit;
         a.xcd_rest = a.B * a.S;                          // row groups of one row, one head
         const size_t nwg = 8 * (size_t)((a.Hkv + 7) / 8) * a.xcd_chunks * a.xcd_rest;
         CH_REQUIRE(nwg < (1u << 31), "attention: decode key range too long");
-        dim3 ga((unsigned)nwg);
-        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, ga, dim3(64), 0, as_stream(stream), a); };
-        if (a.d == 64) go(attn_scores_row_kernel<HYBRID, 64>);
-        else go(attn_scores_row_kernel<HYBRID, 128>);
+        auto go = [&](auto kern, size_t n) { hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64), 0, as_stream(stream), a); };
+        if (tiles) {
+            a.tile_first = (unsigned)nwg;
+            if (a.d == 64) go(attn_scores_row_kernel<HYBRID, 64, HYBRID>, nwg + value_tile_wgs(a));
+            else go(attn_scores_row_kernel<HYBRID, 128, HYBRID>, nwg + value_tile_wgs(a));
+            tiles = false;   // built by this launch
+        } else if (a.d == 64) {
+            go(attn_scores_row_kernel<HYBRID, 64>, nwg);
+        } else {
+            go(attn_scores_row_kernel<HYBRID, 128>, nwg);
+        }
         rc = check_launch("attention scores (decode)");
         if (rc) return rc;
     } else if (chunks > 0) {
@@ -2023,6 +2109,11 @@ static int launch_attention(AttnArgs a, void* stream) {
     if (qpg < 1) qpg = 1;
     const int nbmax = a.nbstride;
     const size_t nsl = (size_t)(a.d + 63) / 64;
+    if (tiles) {
+        hipLaunchKernelGGL(value_tiles_kernel, dim3(value_tile_wgs(a)), dim3(64), 0, as_stream(stream), a);
+        rc = check_launch("attention value tiles");
+        if (rc) return rc;
+    }
     if (HYBRID && a.vsh) return launch_chain_stream(a, nbmax, stream);   // decode with value product tiles
     {
         // prefill: many query rows per workgroup, several chains per lane

@@ -39,6 +39,9 @@ struct AttnArgs {
     // fp32 value-product tiles of the INT8 cache (kv_shadow.hip), or null
     const float* vsh;
     size_t sh_ntile;
+    // decode scores that also build those tiles from the cache (vsh is then
+    // scratch of the launch): the first of the workgroups that do, 0 = none
+    unsigned tile_first;
     // decode score grid mapped onto the XCDs (0: plain 2-D grid): workgroup
     // i runs on XCD i % 8, kv head h's workgroups on XCD h % 8; xcd_chunks
     // workgroups per (row group, kv head), xcd_rest row groups

@@ -301,7 +301,7 @@ __global__ void __launch_bounds__(CS_THREADS) attn_chain_stream_kernel(AttnArgs 
             const uint32_t nlive = kend > bs0 ? kend - bs0 : 0u;      // keys of the block in the row
 #pragma unroll
             for (int k = 0; k < ATT_BLOCK; k++) {
-                const float pv = (uint32_t)k < ncache ? pr[r % CS_R][k / 4][k % 4] : pnew[(k - (int)ncache) & 1];
+                const float pv = (uint32_t)k < ncache ? pr[r % CS_R][k / 4][k % 4] : pnew[(bs0 + k - clen) & 1];
                 const float w = (uint32_t)k < nlive ? wr[r % CS_R][k / 4][k % 4] : 0.0f;
                 const float f = __builtin_fmaf(pv, w, as);
                 as = w != 0.0f ? f : as;

@@ -59,6 +59,7 @@ __host__ __device__ inline size_t sh_index(int kvh, int nsl, int sl, size_t ntil
 enum ScratchKind {
     SCR_GEMM_ACT = 0,    // matmul activation codes + row scales
     SCR_ATTN,            // exact attention weights, block maxima and sums
+    SCR_ATTN_TILES,      // value product tiles of a decode call without its own
     SCR_LM,              // LM head partial maxima + completion counter
     SCR_FAST_PART,       // split-K attention partials
     SCR_FAST_CNT,        // split-K attention completion counters

@@ -557,6 +557,11 @@ def test_attention_f16_mask_noncausal(dev, orc):
     (128, 1500, 128, 16, 8, 128),  # prefill chunk deep into the context
     (50, 300, 50, 8, 1, 128),      # 8 query heads per kv head, prefill
     (33, 64, 33, 4, 4, 64),        # one query head per kv head, prefill
+    (1, 1, 1, 2, 1, 64),           # product tiles built per call: one cached key
+    (1, 64, 1, 8, 2, 128),         # one whole tile, 4 query heads per kv head
+    (2, 63, 2, 16, 2, 64),         # two rows, a tile short of one key, 8 query heads per kv head
+    (1, 1000, 1, 9, 9, 128),       # more kv heads than XCDs
+    (1, 65, 1, 2, 1, 72),          # a slice of 8 dims
     (4, 61, 4, 8, 1, 64),          # one 32-vector tile, a block ending inside the first new rows
     (70, 5, 70, 2, 2, 128),        # several tiles, most keys fp16
     (600, 40, 600, 4, 2, 64),      # several sub-tiles per workgroup
