@@ -695,7 +695,7 @@ __device__ __forceinline__ void sm_step16(f32x4 (&acc)[8], float a, const float*
 }
 
 template <bool HYBRID, int D>
-__global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in, int nsub) {
+__global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in, int nsub, int qv, int rows_follow) {
     const AttnArgs a = resolve(a_in);
     // lane 4 t + i of a register: dim t of vector i (rows 4 banks apart: the
     // staging writes of a wave fall on 64 banks)
@@ -704,7 +704,7 @@ __global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in,
     __shared__ float msh[4][SM_Q][2];
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const float NEG_INF = -__builtin_inff();
-    const int gq = a.gq, qr = SM_Q / gq;                 // query rows of a sub-tile
+    const int gq = a.gq, qr = qv / gq;                   // query rows of a sub-tile (qv <= SM_Q vectors)
     const int ngrp = (a.S + qr * nsub - 1) / (qr * nsub);
     size_t gy = blockIdx.y;
     const int kvh = (int)(gy % a.Hkv);
@@ -819,7 +819,7 @@ __global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in,
         store_q();
         __syncthreads();
         if (qp0 + qr < qp_end) load_q(qp0 + qr);             // in flight while this one is used
-        for (int g = 0; g < SM_Q / 4; g++) {
+        for (int g = 0; g < qv / 4; g++) {
             if (qp0 + (4 * g >> lgq) >= a.S) break;
             int lim_g;
             if (wbase >= row_end(min(qp0 + ((4 * g + 3) >> lgq), a.S - 1), lim_g)) continue;
@@ -886,13 +886,16 @@ __global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in,
         const int q = lane >> 1, half = lane & 1;
         const int qp = qp0 + q / gq;
         const int bs = wbase + 32 * half;
-        if (qp < a.S) {
+        if (q < qv && qp < a.S) {
             int blk_limit;
             const int kv_end = row_end(qp, blk_limit);
             if (bs < kv_end) {
                 const int bsz = min(ATT_BLOCK, blk_limit - bs);
                 const bool is_decode = (!HYBRID) && (qp == a.S - 1) && a.S > 1;
                 const bool block_skipped = !HYBRID && !is_decode && a.causal && bs > (int)a.pos_off + qp;
+                // the rows kernel never takes the keys past a row's causal end,
+                // so their zero weights need no flag there
+                const int zsz = rows_follow ? min(bsz, kv_end - bs) : bsz;
                 // slots past bsz hold other keys' weights or stale values; they
                 // are selected out
                 const f32x4* x4 = reinterpret_cast<const f32x4*>(&wsh[wid][q][32 * half]);
@@ -909,7 +912,7 @@ __global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in,
                         for (int u = 0; u < 4; u++) sum = 4 * t + u < bsz ? sum + x[u] : sum;
                     }
 #pragma unroll
-                    for (int u = 0; u < 4; u++) has_zero |= 4 * t + u < bsz && !(x[u] != 0.0f);
+                    for (int u = 0; u < 4; u++) has_zero |= 4 * t + u < zsz && !(x[u] != 0.0f);
                 }
                 const size_t row = (b * a.S + qp) * a.Hq + h0 + q % gq;
                 const int blk = bs / ATT_BLOCK;
@@ -1186,9 +1189,7 @@ struct CdCfg {
 // (the running max is the last finite block max), else NEG_INF (the block
 // leaves the accumulators unscaled); bsum[blk] is the block's flagged sum.
 // One whole wave.
-// ST: floats between a row's blocks in LDS; none: what an unscaled block holds.
-template <int ST = 1>
-__device__ __forceinline__ void chain_corr_scan(int nb, float* corr, float none = -__builtin_inff());
+__device__ __forceinline__ void chain_corr_scan(int nb, float* corr);
 __device__ __forceinline__ void chain_corr(const AttnArgs& a, size_t row, int nb, float* corr, float* bsum) {
     const int lane = threadIdx.x & 63;
     const float* bm = a.bmax + row * a.nbstride;
@@ -1201,14 +1202,13 @@ __device__ __forceinline__ void chain_corr(const AttnArgs& a, size_t row, int nb
     chain_corr_scan(nb, corr);
 }
 // block maxima in corr[0, nb) -> the corrections, in place (one wave)
-template <int ST>
-__device__ __forceinline__ void chain_corr_scan(int nb, float* corr, float none) {
+__device__ __forceinline__ void chain_corr_scan(int nb, float* corr) {
     const int lane = threadIdx.x & 63;
     const float NEG_INF = -__builtin_inff();
     float carry = NEG_INF;
     for (int c0 = 0; c0 < nb; c0 += 64) {
         const int i = c0 + lane;
-        const float m = i < nb ? corr[i * ST] : NEG_INF;
+        const float m = i < nb ? corr[i] : NEG_INF;
         const bool fin = m > NEG_INF;
         int idx = fin ? lane : -1;
 #pragma unroll
@@ -1220,7 +1220,7 @@ __device__ __forceinline__ void chain_corr_scan(int nb, float* corr, float none)
         if (lane == 0) ex = -1;
         const float pm = __shfl(m, ex < 0 ? 0 : ex, 64);
         const float prev = ex >= 0 ? pm : carry;
-        if (i < nb) corr[i * ST] = fin ? cactus_expf(prev - m) : none;
+        if (i < nb) corr[i] = fin ? cactus_expf(prev - m) : NEG_INF;
         const int last = __shfl(idx, 63, 64);
         if (last >= 0) carry = __shfl(m, last, 64);
     }
@@ -1831,8 +1831,37 @@ __global__ void __launch_bounds__(RW_THREADS) attn_rows_kernel(AttnArgs a_in, in
         for (int i = 0; i < CPW; i++) corr_s[blk * RW_CS + wv * CPW + i] = blk < cnb[i] ? m[i] : 1.0f;
     }
     wave_lds_order();
+    // chain_corr_scan of the four chains side by side: the running max before
+    // a block is its last finite block max, found by a max-scan of the lanes
+    // that hold one; blocks without one, and past the chain's end, hold 1
+    float carry[CPW];
 #pragma unroll
-    for (int i = 0; i < CPW; i++) chain_corr_scan<RW_CS>(cnb[i], corr_s + wv * CPW + i, 1.0f);
+    for (int i = 0; i < CPW; i++) carry[i] = -__builtin_inff();
+    for (int b0 = 0; b0 < nbt; b0 += 64) {
+        const int blk = b0 + lane;
+        float m[CPW], x[CPW];
+        int idx[CPW];
+#pragma unroll
+        for (int i = 0; i < CPW; i++) {
+            m[i] = blk < cnb[i] ? corr_s[min(blk, nbt - 1) * RW_CS + wv * CPW + i] : -__builtin_inff();
+            idx[i] = m[i] > -__builtin_inff() ? lane : -1;
+        }
+#pragma unroll
+        for (int i = 0; i < CPW; i++) idx[i] = wave_scan_max(idx[i]);
+#pragma unroll
+        for (int i = 0; i < CPW; i++) {
+            const int ex = __builtin_amdgcn_update_dpp(-1, idx[i], 0x138, 0xF, 0xF, false);   // wave_shr:1
+            const float pm = __shfl(m[i], ex < 0 ? 0 : ex, 64);
+            x[i] = (ex >= 0 ? pm : carry[i]) - m[i];
+            const int last = __builtin_amdgcn_readlane(idx[i], 63);
+            if (last >= 0) carry[i] = lane_f(m[i], last);
+        }
+        float e[CPW];
+        cactus_expf_n<CPW>(x, e);
+#pragma unroll
+        for (int i = 0; i < CPW; i++)
+            if (blk < nbt) corr_s[blk * RW_CS + wv * CPW + i] = m[i] > -__builtin_inff() ? e[i] : 1.0f;
+    }
     if (!is_chain) {
         // tiles 0 and 1 before the first barrier; after barrier t the tile
         // t + 2 goes to the buffer that tile t - 1 left
@@ -1865,10 +1894,9 @@ __global__ void __launch_bounds__(RW_THREADS) attn_rows_kernel(AttnArgs a_in, in
         if (qp < a.S) {
             size_t rks, rke, rbl;
             kv_range<HYBRID>(a, (size_t)qp, rks, rke, rbl);
-            if (rke > rks) {
-                const size_t full = (rke - rks + ATT_BLOCK - 1) / ATT_BLOCK * ATT_BLOCK;
-                klen[c] = (int)(rks + full < rbl ? full : rbl - rks);
-            }
+            // (an FP16 block reaches past the row's causal end, with zero
+            // weights: skipped keys)
+            if (rke > rks) klen[c] = (int)(rke - rks);
             kmin = min(kmin, klen[c]);
             kmax = max(kmax, klen[c]);
         }
@@ -2042,6 +2070,21 @@ static int launch_attention(AttnArgs a, void* stream) {
         }
     }
     const bool windowed = !HYBRID && a.window > 0 && a.window < a.Skv;
+    // the values of prefill rows run in the many-rows kernel
+    bool rows_follow = !windowed && (size_t)a.B * a.S > 2 && a.gq <= ATT_MAX_GQ && RW_CH % a.gq == 0 && a.d % 4 == 0 &&
+                       (HYBRID ? (uintptr_t)a.vc % 4 == 0 && (uintptr_t)a.vs % 4 == 0 : true) &&
+                       (uintptr_t)a.v % 8 == 0 && rows_smem(a.nbstride) <= 160 * 1024;
+    if (rows_follow) {
+        static hipError_t attr[2] = {
+            hipFuncSetAttribute((const void*)attn_rows_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                160 * 1024),
+            hipFuncSetAttribute((const void*)attn_rows_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                160 * 1024)};
+        if (attr[HYBRID] != hipSuccess) {
+            (void)hipGetLastError();  // clear the sticky attribute error before the other forms
+            rows_follow = false;
+        }
+    }
     // scores of prefill rows and of a decode row: 16-byte key rows, one scale
     // per 16 dims, whole groups of query heads
     const bool k16 = HYBRID ? ((uintptr_t)a.kc % 16 == 0 && (uintptr_t)a.ks % 4 == 0 && a.qgs % 16 == 0) : true;
@@ -2053,15 +2096,21 @@ static int launch_attention(AttnArgs a, void* stream) {
     if (rows_ok && (size_t)a.B * a.S > 2) {
         // sub-tiles of query vectors per workgroup: the keys are converted
         // once for all of them, as long as two workgroups per CU remain
-        const int qr = SM_Q / a.gq;
-        auto grid_y = [&](int n) { return (size_t)a.B * (((size_t)a.S + (size_t)qr * n - 1) / ((size_t)qr * n)) * a.Hkv; };
+        // (short grids take fewer vectors per workgroup instead: a wave's
+        // vectors follow one another, about 1 us per four; 64 rows over
+        // themselves 26 -> 17 us with it and the side-by-side rescale scans)
+        auto grid_y = [&](int n) { return (size_t)a.B * (((size_t)a.S * a.gq + n - 1) / n) * a.Hkv; };
+        int qv = SM_Q;
+        while (qv > ATT_MAX_GQ && (chunks + 3) / 4 * grid_y(qv) < 512) qv /= 2;
         int nsub = 1;
-        while (nsub < 8 && (size_t)qr * nsub < (size_t)a.S && (chunks + 3) / 4 * grid_y(2 * nsub) >= 512) nsub *= 2;
-        dim3 ga((unsigned)((chunks + 3) / 4), (unsigned)grid_y(nsub));
+        while (nsub < 8 && (size_t)qv * nsub < (size_t)a.S * a.gq && (chunks + 3) / 4 * grid_y(2 * nsub * qv) >= 512) nsub *= 2;
+        dim3 ga((unsigned)((chunks + 3) / 4), (unsigned)grid_y(nsub * qv));
         if (a.d == 64)
-            hipLaunchKernelGGL((attn_scores_mfma_kernel<HYBRID, 64>), ga, dim3(256), 0, as_stream(stream), a, nsub);
+            hipLaunchKernelGGL((attn_scores_mfma_kernel<HYBRID, 64>), ga, dim3(256), 0, as_stream(stream), a, nsub, qv,
+                               (int)rows_follow);
         else
-            hipLaunchKernelGGL((attn_scores_mfma_kernel<HYBRID, 128>), ga, dim3(256), 0, as_stream(stream), a, nsub);
+            hipLaunchKernelGGL((attn_scores_mfma_kernel<HYBRID, 128>), ga, dim3(256), 0, as_stream(stream), a, nsub, qv,
+                               (int)rows_follow);
         rc = check_launch("attention scores (rows)");
         if (rc) return rc;
     } else if (rows_ok) {
@@ -2115,26 +2164,13 @@ static int launch_attention(AttnArgs a, void* stream) {
         if (rc) return rc;
     }
     if (HYBRID && a.vsh) return launch_chain_stream(a, nbmax, stream);   // decode with value product tiles
-    {
+    if (rows_follow) {
         // prefill: many query rows per workgroup, several chains per lane
-        const bool aligned = (HYBRID ? (uintptr_t)a.vc % 4 == 0 && (uintptr_t)a.vs % 4 == 0 : true) &&
-                             (uintptr_t)a.v % 8 == 0;
-        if (!windowed && (size_t)a.B * a.S > 2 && a.gq <= ATT_MAX_GQ && RW_CH % a.gq == 0 && a.d % 4 == 0 &&
-            aligned && rows_smem(nbmax) <= 160 * 1024) {
-            static hipError_t attr[2] = {
-                hipFuncSetAttribute((const void*)attn_rows_kernel<false>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
-                hipFuncSetAttribute((const void*)attn_rows_kernel<true>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)};
-            if (attr[HYBRID] == hipSuccess) {
-                const int qr = RW_CH / a.gq;
-                const size_t groups = (size_t)a.B * (((size_t)a.S + qr - 1) / qr) * a.Hkv * nsl;
-                hipLaunchKernelGGL(attn_rows_kernel<HYBRID>, dim3((unsigned)groups), dim3(RW_THREADS),
-                                   rows_smem(nbmax), as_stream(stream), a, nbmax);
-                return check_launch("attention values (rows)");
-            }
-            (void)hipGetLastError();  // clear the sticky attribute error before the forms below
-        }
+        const int qr = RW_CH / a.gq;
+        const size_t groups = (size_t)a.B * (((size_t)a.S + qr - 1) / qr) * a.Hkv * nsl;
+        hipLaunchKernelGGL(attn_rows_kernel<HYBRID>, dim3((unsigned)groups), dim3(RW_THREADS), rows_smem(nbmax),
+                           as_stream(stream), a, nbmax);
+        return check_launch("attention values (rows)");
     }
     // LDS-DMA form: value rows in 16- or 4-byte chunks, one scale group per
     // 64-dim slice; otherwise the register-staged form

@@ -58,18 +58,6 @@ __device__ __forceinline__ void wait_vm_tie2(V* p, V* w) {
                  : "n"(N));
 }
 
-// inclusive max-scan over the wave's lanes (identity -1): row_shr 1, 2, 4,
-// 8 within each 16-lane row, then row_bcast:15 and row_bcast:31 across rows
-__device__ __forceinline__ int wave_scan_max(int v) {
-    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x111, 0xF, 0xF, false));
-    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x112, 0xF, 0xF, false));
-    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x114, 0xF, 0xF, false));
-    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x118, 0xF, 0xF, false));
-    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x142, 0xA, 0xF, false));
-    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x143, 0xC, 0xF, false));
-    return v;
-}
-
 struct CsMap {
     int row, kvh, hj, sl;
     bool valid;

@@ -344,6 +344,17 @@ __device__ __forceinline__ float wave_max(float v) {
     auto lane_v = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l)); };
     return __builtin_fmaxf(__builtin_fmaxf(lane_v(0), lane_v(16)), __builtin_fmaxf(lane_v(32), lane_v(48)));
 }
+// inclusive max-scan over the wave's lanes (identity -1): row_shr 1, 2, 4,
+// 8 within each 16-lane row, then row_bcast:15 and row_bcast:31 across rows
+__device__ __forceinline__ int wave_scan_max(int v) {
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x111, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x112, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x114, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x118, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x142, 0xA, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x143, 0xC, 0xF, false));
+    return v;
+}
 __device__ __forceinline__ int wave_sum_i32(int v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
