@@ -769,14 +769,32 @@ __device__ __forceinline__ float xrow_sum(float v) {
     return x + y;
 }
 
+// v_max3_f32 (a NaN operand yields the others): fmaxf would canonicalise each operand first
+__device__ __forceinline__ float max3f(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// Bound by vector instructions (softmax, INT8-to-FP16 staging: ~250 per wave
+// and tile against 32 MFMAs) and by the partials, written and read once.
+// What brought 333 rows at 3000 keys, 16 / 8 heads, 49.9 -> 36.0 us: two waves
+// per SIMD (it held 304 registers: one), tile t + 2 fetched before tile t's
+// work instead of after it, one uniform mask branch per block of vectors
+// instead of one per score, value fragments read ahead of the softmax, eight
+// waves per staged tile.  The maximum of each tile is taken exactly: moving
+// it only when a score passes it by 2^8 spared rescales, but the weight of
+// the largest score was then rounded (error 3.32e-4 -> 3.49e-4).
 template <int D, int GQ, int W, int NB, int VB>
-__global__ void __launch_bounds__(64 * W) attn_prefill_mfma_kernel(PrefillArgs a) {
+__global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArgs a) {
     static_assert(D == 64 || D == 128, "head_dim 64 or 128");
-    static_assert(64 * W >= 2 * D, "staging threads: 32 keys x D/16 pieces");
+    static_assert(W == 4 || W == 8, "staging: every thread a piece of a key, 8 or 16 dims");
+    constexpr float LOG2E = 1.4426950408889634f;
     constexpr int NV = 16 * W * VB;            // query vectors per workgroup (16 VB per wave)
     constexpr int KS = D + 8;                  // LDS row of a key tile, halves
     constexpr int VS = PF_T + 8;               // LDS row of a transposed value tile, halves
-    constexpr int CPR = D / 16;                // 16-dim pieces per key row
+    constexpr int NP = D == 128 && W == 4 ? 2 : 1;   // 8-dim pieces a thread stages per tile
+    constexpr int CPR = D / (8 * NP);          // staging threads per key row
     constexpr int NC = D / 32;                 // 32-dim MFMA steps of a score
     constexpr int ND = D / 16;                 // 16-dim output blocks
     __shared__ __align__(16) _Float16 ksh[2][PF_T][KS];
@@ -802,147 +820,125 @@ __global__ void __launch_bounds__(64 * W) attn_prefill_mfma_kernel(PrefillArgs a
     // ---- this lane's query vectors: lr of each of the wave's VB blocks of
     // 16 (B operands of S^T = K Q^T; every key and value fragment read from
     // LDS feeds VB MFMAs, and the blocks' softmax chains interleave)
-    int vm[VB], vrow[VB];
-    bool vok[VB];
-    size_t vpos[VB];
-#pragma unroll
-    for (int vb = 0; vb < VB; vb++) {
-        vm[vb] = gm0 + (wid * VB + vb) * 16 + lr;
-        vrow[vb] = vm[vb] / GQ;
-        vok[vb] = vrow[vb] < a.S;
-        vpos[vb] = a.pos_off + (size_t)vrow[vb];
-    }
-    // the wave's first row (its smallest position) and whether all its rows exist
-    const int wrow0 = (gm0 + wid * 16 * VB) / GQ, wrow1 = (gm0 + wid * 16 * VB + 16 * VB - 1) / GQ;
-    const bool wave_all_rows = wrow1 < a.S;
-    const size_t wave_min_pos = a.pos_off + (size_t)wrow0;
+    const int vm0 = gm0 + wid * VB * 16 + lr;   // block vb's vector is vm0 + 16 vb
+    int vlim[VB];   // keys each vector sees: positions below vlim (0 for a vector past the last row)
     h16x8 qv[VB][NC];
 #pragma unroll
     for (int vb = 0; vb < VB; vb++) {
+        const int row = (vm0 + 16 * vb) / GQ;
+        const bool vok = row < a.S;
+        vlim[vb] = vok ? (int)min(a.pos_off + (size_t)row + 1, kv_end) : 0;
         const uint16_t* qp =
-            a.q + (((size_t)b * a.S + (vok[vb] ? vrow[vb] : 0)) * a.Hq + (size_t)g * GQ + vm[vb] % GQ) * D;
+            a.q + (((size_t)b * a.S + (vok ? row : 0)) * a.Hq + (size_t)g * GQ + (vm0 + 16 * vb) % GQ) * D;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            const uint4 u = vok[vb] ? *reinterpret_cast<const uint4*>(qp + 32 * c + 8 * lg) : make_uint4(0, 0, 0, 0);
+            const uint4 u = vok ? *reinterpret_cast<const uint4*>(qp + 32 * c + 8 * lg) : make_uint4(0, 0, 0, 0);
             qv[vb][c] = __builtin_bit_cast(h16x8, u);
         }
     }
+    // keys that all of the wave's vectors see (its first row is its smallest
+    // position; 0 if a row is missing)
+    const int wrow0 = (gm0 + wid * 16 * VB) / GQ, wrow1 = (gm0 + wid * 16 * VB + 16 * VB - 1) / GQ;
+    const int wave_lim = wrow1 < a.S ? (int)min(a.pos_off + (size_t)wrow0 + 1, kv_end) : 0;
 
-    // ---- tile staging: thread -> (key sj, 16-dim piece sp), lanes of a
-    // wave on 32 different keys so the transposed value writes spread over
-    // the LDS banks.  Every tile issues the same loads -- the key's INT8
-    // cache piece and its FP16 new-row piece, each from a clamped in-bounds
-    // row -- and picks one when staging, so the loads take no branch and
-    // the compiler keeps NB tiles in flight (slot t % NB).
+    // ---- tile staging: thread -> (key sj, NP 8-dim pieces from sp NP), lanes
+    // of a wave on 32 different keys so the transposed value writes spread
+    // over the LDS banks.  A lane's key is either cached (codes) or new (FP16
+    // values): the address is chosen per lane, a piece is one 16-byte load in
+    // both forms (of a cached key the aligned 16 codes that hold it), from a
+    // clamped in-bounds row, so the loads take no branch and the compiler
+    // keeps NB tiles in flight (slot t % NB).  Loading both forms and picking
+    // one when staging held 26 registers a slot: one wave per SIMD.
     const int sj = tid % PF_T, sp = tid / PF_T;
     const bool stager = sp < CPR;
-    const size_t rstride = (size_t)a.Hkv * D;   // elements between consecutive keys
-    const int8_t* kcb = nullptr;
-    const int8_t* vcb = nullptr;
-    const float* ksb = nullptr;
-    const float* vsb = nullptr;
-    const uint16_t* knb = nullptr;
-    const uint16_t* vnb = nullptr;
-    {
-        // a valid stand-in for a missing part (its values are never used)
-        const uint16_t* any16 = a.q;
-        if (a.cache_len > 0) {
-            kcb = a.kc + ((size_t)b * a.cache_len * a.Hkv + g) * D + 16 * sp;
-            vcb = a.vc + ((size_t)b * a.cache_len * a.Hkv + g) * D + 16 * sp;
-            ksb = a.ks + (size_t)g * a.nqg;
-            vsb = a.vs + (size_t)g * a.nqg;
-        } else {
-            kcb = vcb = reinterpret_cast<const int8_t*>(any16);
-            ksb = vsb = reinterpret_cast<const float*>(any16);
-        }
-        if (a.new_len > 0) {
-            knb = a.kn + ((size_t)b * a.new_len * a.Hkv + g) * D + 16 * sp;
-            vnb = a.vn + ((size_t)b * a.new_len * a.Hkv + g) * D + 16 * sp;
-        } else {
-            knb = vnb = any16;
-        }
-    }
+    const int p0 = stager ? sp * NP : 0;        // first piece
     const int clen = (int)a.cache_len, nlen = (int)a.new_len;
-    const size_t cstride = a.cache_len > 0 ? rstride : 0;   // stand-ins do not move
-    const size_t nstride = a.new_len > 0 ? rstride : 0;
-    const size_t sstride = a.cache_len > 0 ? (size_t)a.Hkv * a.nqg : 0;
+    const size_t rstride = (size_t)a.Hkv * D;   // elements between consecutive keys
+    const int sstride = clen > 0 ? a.Hkv * a.nqg : 0;
+    const int8_t* kcb = a.kc + ((size_t)b * a.cache_len * a.Hkv + g) * D + 16 * (p0 / 2);
+    const int8_t* vcb = a.vc + ((size_t)b * a.cache_len * a.Hkv + g) * D + 16 * (p0 / 2);
+    const uint16_t* knb = a.kn + ((size_t)b * a.new_len * a.Hkv + g) * D + 8 * p0;
+    const uint16_t* vnb = a.vn + ((size_t)b * a.new_len * a.Hkv + g) * D + 8 * p0;
+    // without a cache the scale loads read query words (never used)
+    const float* ksb = clen > 0 ? a.ks + (size_t)g * a.nqg : reinterpret_cast<const float*>(a.q);
+    const float* vsb = clen > 0 ? a.vs + (size_t)g * a.nqg : reinterpret_cast<const float*>(a.q);
+    const float sl2 = a.scale * LOG2E;   // scores in units of ln 2: weights are 2^(s - max)
     struct Raw {
-        uint4 kc, vc;            // 16 INT8 codes
-        uint4 kn[2], vn[2];      // 16 FP16 values
+        uint4 k[NP], v[NP];      // per piece 16 INT8 codes (its 8 among them) or 8 FP16 values
         float ks, vs;
     };
     Raw raw[NB];
     auto fetch = [&](int t, Raw& r) {
-        const int kp = t * PF_T + sj;
-        const int ci = min(kp, max(clen - 1, 0)), ni = min(max(kp - clen, 0), max(nlen - 1, 0));
-        r.kc = *reinterpret_cast<const uint4*>(kcb + (size_t)ci * cstride);
-        r.vc = *reinterpret_cast<const uint4*>(vcb + (size_t)ci * cstride);
-        const uint4* k4 = reinterpret_cast<const uint4*>(knb + (size_t)ni * nstride);
-        const uint4* v4 = reinterpret_cast<const uint4*>(vnb + (size_t)ni * nstride);
-        r.kn[0] = k4[0];
-        r.kn[1] = k4[1];
-        r.vn[0] = v4[0];
-        r.vn[1] = v4[1];
-        r.ks = ksb[(size_t)ci * sstride];
-        r.vs = vsb[(size_t)ci * sstride];
+        // keys past the last row reload it: cache_len + new_len > 0 here
+        const int kp = min(t * PF_T + sj, clen + nlen - 1);
+        const bool cached = kp < clen;
+        const size_t ro = (size_t)(cached ? kp : kp - clen) * rstride;
+        const char* kp0 = cached ? reinterpret_cast<const char*>(kcb + ro) : reinterpret_cast<const char*>(knb + ro);
+        const char* vp0 = cached ? reinterpret_cast<const char*>(vcb + ro) : reinterpret_cast<const char*>(vnb + ro);
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int o = cached ? 0 : 16 * i;
+            r.k[i] = *reinterpret_cast<const uint4*>(kp0 + o);
+            r.v[i] = *reinterpret_cast<const uint4*>(vp0 + o);
+        }
+        const size_t so = (size_t)(cached ? kp : max(clen - 1, 0)) * sstride;
+        r.ks = ksb[so];
+        r.vs = vsb[so];
     };
     auto stage = [&](int t, int buf, const Raw& r) {
         if (!stager) return;
         const int kp = t * PF_T + sj;
         const bool live = kp < (int)kv_end, cached = kp < clen;
-        h16x8 k0, k1;
-        _Float16 vh[16];
-        if (cached) {
-            // key codes to exact fp16: the biased byte b ^ 0x80 = b + 128
-            // under the exponent byte 0x64 reads as 1024 + b + 128, and 1152
-            // comes off in packed fp16 (integers below 2048 are exact)
-            const uint32_t kx[4] = {r.kc.x ^ 0x80808080u, r.kc.y ^ 0x80808080u, r.kc.z ^ 0x80808080u,
-                                    r.kc.w ^ 0x80808080u};
-            typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
-            const h16x2 bias = {(_Float16)1152.0f, (_Float16)1152.0f};
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const h16x2 lo = __builtin_bit_cast(h16x2, __builtin_amdgcn_perm(0x64646464u, kx[j], 0x04010400u)) - bias;
-                const h16x2 hi = __builtin_bit_cast(h16x2, __builtin_amdgcn_perm(0x64646464u, kx[j], 0x04030402u)) - bias;
-                h16x8& kd = j < 2 ? k0 : k1;
-                const int e0 = 4 * (j & 1);
-                kd[e0] = lo[0];
-                kd[e0 + 1] = lo[1];
-                kd[e0 + 2] = hi[0];
-                kd[e0 + 3] = hi[1];
+        for (int i = 0; i < NP; i++) {
+            const int pc = p0 + i;
+            h16x8 kh;
+            _Float16 vh[8];
+            if (cached) {
+                // key codes to exact fp16: the biased byte b ^ 0x80 = b + 128
+                // under the exponent byte 0x64 reads as 1024 + b + 128, and 1152
+                // comes off in packed fp16 (integers below 2048 are exact)
+                const uint32_t odd = 0u - (uint32_t)(pc & 1);   // an odd piece takes the upper 8 codes
+                const uint32_t kx[2] = {((r.k[i].z & odd) | (r.k[i].x & ~odd)) ^ 0x80808080u,
+                                        ((r.k[i].w & odd) | (r.k[i].y & ~odd)) ^ 0x80808080u};
+                typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
+                const h16x2 bias = {(_Float16)1152.0f, (_Float16)1152.0f};
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const h16x2 lo = __builtin_bit_cast(h16x2, __builtin_amdgcn_perm(0x64646464u, kx[j], 0x04010400u)) - bias;
+                    const h16x2 hi = __builtin_bit_cast(h16x2, __builtin_amdgcn_perm(0x64646464u, kx[j], 0x04030402u)) - bias;
+                    kh[4 * j] = lo[0];
+                    kh[4 * j + 1] = lo[1];
+                    kh[4 * j + 2] = hi[0];
+                    kh[4 * j + 3] = hi[1];
+                }
+                // values fp16(fp32(code * scale)): with u = code + 128 (an unsigned
+                // byte), fma(u, scale, -128 scale) is that fp32 product exactly
+                // (one rounding of u scale - 128 scale = code scale; -128 scale is exact)
+                const float ms = -128.0f * r.vs;
+                const uint32_t vx[2] = {((r.v[i].z & odd) | (r.v[i].x & ~odd)) ^ 0x80808080u,
+                                        ((r.v[i].w & odd) | (r.v[i].y & ~odd)) ^ 0x80808080u};
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    vh[e] = (_Float16)fp32_barrier(__builtin_fmaf((float)((vx[e >> 2] >> (8 * (e & 3))) & 0xFFu), r.vs, ms));
+            } else {
+                kh = __builtin_bit_cast(h16x8, r.k[i]);
+                const h16x8 v0 = __builtin_bit_cast(h16x8, r.v[i]);
+#pragma unroll
+                for (int e = 0; e < 8; e++) vh[e] = v0[e];
             }
-            // values fp16(fp32(code * scale)): with u = code + 128 (an unsigned
-            // byte), fma(u, scale, -128 scale) is that fp32 product exactly
-            // (one rounding of u scale - 128 scale = code scale; -128 scale is exact)
-            const float ms = -128.0f * r.vs;
-            const uint32_t vx[4] = {r.vc.x ^ 0x80808080u, r.vc.y ^ 0x80808080u, r.vc.z ^ 0x80808080u,
-                                    r.vc.w ^ 0x80808080u};
+            if (!live) {
+                // keys past the block's causal end: zero values (their weights are 0)
 #pragma unroll
-            for (int e = 0; e < 16; e++)
-                vh[e] = (_Float16)fp32_barrier(__builtin_fmaf((float)((vx[e >> 2] >> (8 * (e & 3))) & 0xFFu), r.vs, ms));
-        } else {
-            k0 = __builtin_bit_cast(h16x8, r.kn[0]);
-            k1 = __builtin_bit_cast(h16x8, r.kn[1]);
-            const h16x8 v0 = __builtin_bit_cast(h16x8, r.vn[0]), v1 = __builtin_bit_cast(h16x8, r.vn[1]);
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                vh[e] = v0[e];
-                vh[8 + e] = v1[e];
+                for (int e = 0; e < 8; e++) vh[e] = (_Float16)0.0f;
             }
-        }
-        if (!live) {
-            // keys past the block's causal end: zero values (their weights are 0)
+            *reinterpret_cast<h16x8*>(&ksh[buf][sj][8 * pc]) = kh;
 #pragma unroll
-            for (int e = 0; e < 16; e++) vh[e] = (_Float16)0.0f;
+            for (int e = 0; e < 8; e++) vt[buf][8 * pc + e][sj] = vh[e];
         }
-        *reinterpret_cast<h16x8*>(&ksh[buf][sj][16 * sp]) = k0;
-        *reinterpret_cast<h16x8*>(&ksh[buf][sj][16 * sp + 8]) = k1;
-#pragma unroll
-        for (int e = 0; e < 16; e++) vt[buf][16 * sp + e][sj] = vh[e];
-        if (sp == 0) ksc[buf][sj] = (cached ? r.ks : 1.0f) * a.scale;
+        if (sp == 0) ksc[buf][sj] = (cached ? r.ks : 1.0f) * sl2;
     };
 
-    constexpr float LOG2E = 1.4426950408889634f;
     const float NEG_INF = -__builtin_inff();
     float m_run[VB], l_run[VB];
     f32x4 acc[VB][ND];   // O^T: lane l holds dims 16 db + 4 lg + i of vector lr of each block
@@ -965,6 +961,9 @@ __global__ void __launch_bounds__(64 * W) attn_prefill_mfma_kernel(PrefillArgs a
         if (tl >= nt) break;
         const int t = t_begin + tl;
         const int buf = tl & 1;
+        // tile t is staged, so its slot takes tile t + NB: its loads have NB
+        // tiles' work to arrive in (clamped rows: in bounds past the split too)
+        fetch(t + NB, raw[u]);
         // scores S^T for keys 16h + 4lg + i of the tile, vector lr of each block
         f32x4 st[VB][2];
 #pragma unroll
@@ -981,65 +980,81 @@ __global__ void __launch_bounds__(64 * W) attn_prefill_mfma_kernel(PrefillArgs a
         }
         // a tile below every row's causal end and the key range needs no
         // mask (wave-uniform test); the others mask key by key
-        const size_t tile_last = (size_t)t * PF_T + PF_T - 1;
-        const bool interior = wave_all_rows && tile_last < kv_end && tile_last <= wave_min_pos;
+        const bool interior = t * PF_T + PF_T <= wave_lim;
         const f32x4 ksv0 = *reinterpret_cast<const f32x4*>(&ksc[buf][4 * lg]);
         const f32x4 ksv1 = *reinterpret_cast<const f32x4*>(&ksc[buf][16 + 4 * lg]);
-        float corr[VB];
-        h16x8 pa[VB];   // P^T operands: keys {4 lg + j, 16 + 4 lg + j} of vector lr
-#pragma unroll
-        for (int vb = 0; vb < VB; vb++) {
-            float s[8];
-            float mx = NEG_INF;
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const f32x4 ksv = h ? ksv1 : ksv0;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    if (interior) {
-                        s[4 * h + i] = st[vb][h][i] * ksv[i];
-                    } else {
-                        const size_t kp = (size_t)t * PF_T + 16 * h + 4 * lg + i;
-                        const bool ok = vok[vb] && kp < kv_end && kp <= vpos[vb];
-                        s[4 * h + i] = ok ? st[vb][h][i] * ksv[i] : NEG_INF;
-                    }
-                    mx = __builtin_fmaxf(mx, s[4 * h + i]);
-                }
-            }
-            mx = xrow_max(mx);
-            const float m_new = __builtin_fmaxf(m_run[vb], mx);
-            const bool live = m_new > NEG_INF;
-            corr[vb] = live ? fast_exp2((m_run[vb] - m_new) * LOG2E) : 1.0f;
-            float psum = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float pv = (live && s[j] > NEG_INF) ? fast_exp2((s[j] - m_new) * LOG2E) : 0.0f;
-                psum += pv;
-                pa[vb][j] = (_Float16)pv;
-            }
-            l_run[vb] = l_run[vb] * corr[vb] + xrow_sum(psum);
-            m_run[vb] = m_new;
-        }
-        // O^T += V^T P^T: A = V^T (dims 16 db + lr, the same 8 keys)
+        // A = V^T (dims 16 db + lr, the same 8 keys): all reads in flight
+        // during the softmax (left to the compiler each waits at its MFMAs)
+        h16x8 va[ND];
 #pragma unroll
         for (int db = 0; db < ND; db++) {
             const h16x4 v0 = *reinterpret_cast<const h16x4*>(&vt[buf][16 * db + lr][4 * lg]);
             const h16x4 v1 = *reinterpret_cast<const h16x4*>(&vt[buf][16 * db + lr][16 + 4 * lg]);
-            const h16x8 va = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+            va[db] = (h16x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        h16x8 pa[VB];   // P^T operands: keys {4 lg + j, 16 + 4 lg + j} of vector lr
+#pragma unroll
+        for (int vb = 0; vb < VB; vb++) {
+            float s[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) s[j] = st[vb][j >> 2][j & 3] * (j < 4 ? ksv0[j & 3] : ksv1[j & 3]);
+            if (!interior) {
+                const int rem = vlim[vb] - t * PF_T - 4 * lg;   // visible keys from the lane's first
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (16 * (j >> 2) + (j & 3) >= rem) s[j] = NEG_INF;
+            }
+            float mx = max3f(max3f(max3f(s[0], s[1], s[2]), s[3], s[4]), max3f(s[5], s[6], s[7]), NEG_INF);
+            // a tile that moves no running max of the wave's 16 vectors needs
+            // no rescale (wave-uniform branch)
+            mx = xrow_max(mx);
+            const float m_old = m_run[vb];
+            if (__any(mx > m_old)) {
+                const float m_new = __builtin_fmaxf(m_old, mx);
+                const float corr = m_new > NEG_INF ? fast_exp2(m_old - m_new) : 1.0f;
+                l_run[vb] *= corr;
+                m_run[vb] = m_new;
+#pragma unroll
+                for (int db = 0; db < ND; db++) acc[vb][db] *= corr;
+            }
+            // masked scores weigh 2^-inf = 0 (also while no key is live: 2^(-inf - 0))
+            const float m = m_run[vb] > NEG_INF ? m_run[vb] : 0.0f;
+            float pv[8], psum = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                pv[j] = fast_exp2(s[j] - m);
+                psum += pv[j];
+            }
+            if (__any(psum != psum)) {   // a NaN score is left out, as a masked one
+                psum = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    if (!(s[j] > NEG_INF)) pv[j] = 0.0f;
+                    psum += pv[j];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) pa[vb][j] = (_Float16)pv[j];
+            l_run[vb] += psum;   // this lane's keys; the four lanes add up at the end
+        }
+        // O^T += V^T P^T
+#pragma unroll
+        for (int db = 0; db < ND; db++) {
 #pragma unroll
             for (int vb = 0; vb < VB; vb++)
-                acc[vb][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pa[vb], acc[vb][db] * corr[vb], 0, 0, 0);
+                acc[vb][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[db], pa[vb], acc[vb][db], 0, 0, 0);
         }
         // the next tile into the other LDS buffer (its last readers finished
-        // before the previous barrier), then tile t + NB into this slot
+        // before the previous barrier)
         if (tl + 1 < nt) stage(t + 1, buf ^ 1, raw[(u + 1) % NB]);
-        if (tl + NB < nt) fetch(t + NB, raw[u]);
         __syncthreads();
     }
 
     // ---- output: vector lr of each block, dims 16 db + 4 lg + i
 #pragma unroll
     for (int vb = 0; vb < VB; vb++) {
+        l_run[vb] = xrow_sum(l_run[vb]);
         if (a.nsplit > 1) {
             // this split's partial (acc, running max, sum) of the vector
             const int nqb = (int)gridDim.x / a.nsplit;
@@ -1053,8 +1068,9 @@ __global__ void __launch_bounds__(64 * W) attn_prefill_mfma_kernel(PrefillArgs a
             }
             continue;
         }
-        if (!vok[vb]) continue;
-        uint16_t* op = a.o + (((size_t)b * a.S + vrow[vb]) * a.Hq + (size_t)g * GQ + vm[vb] % GQ) * D;
+        const int vm = vm0 + 16 * vb;
+        if (vm / GQ >= a.S) continue;
+        uint16_t* op = a.o + (((size_t)b * a.S + vm / GQ) * a.Hq + (size_t)g * GQ + vm % GQ) * D;
         const float inv = l_run[vb] > 0.0f ? 1.0f / l_run[vb] : 0.0f;
 #pragma unroll
         for (int db = 0; db < ND; db++) {
@@ -1068,14 +1084,13 @@ __global__ void __launch_bounds__(64 * W) attn_prefill_mfma_kernel(PrefillArgs a
 // Combine of the key splits: grid (query blocks x NV / 16, B * Hkv), 256
 // threads; a workgroup takes 16 query vectors, 16 threads per vector with
 // D/16 dims each.  M = max_s M_s, L = sum_s e^(M_s - M) l_s,
-// o = sum_s e^(M_s - M) acc_s / L.  Loads are branch-free (clamped splits,
+// o = sum_s e^(M_s - M) acc_s / L (maxima in units of ln 2).  Loads are branch-free (clamped splits,
 // weight 0 past the block's split count) and issued per batch of splits.
 constexpr int PF_MAX_SPLITS = 16;
 
 template <int D, int GQ, int NV>
 __global__ void __launch_bounds__(256) attn_prefill_combine_kernel(PrefillArgs a) {
     constexpr int VPW = 16, DS = D / 16, SB = 4;
-    constexpr float LOG2E = 1.4426950408889634f;
     const int tid = threadIdx.x, vl = tid / 16, dq = (tid % 16) * DS;
     const int qb = blockIdx.x / (NV / VPW), v = (blockIdx.x % (NV / VPW)) * VPW + vl;
     const int bg = blockIdx.y, b = bg / a.Hkv, g = bg % a.Hkv;
@@ -1106,7 +1121,7 @@ __global__ void __launch_bounds__(256) attn_prefill_combine_kernel(PrefillArgs a
     float L = 0.0f;
 #pragma unroll
     for (int s = 0; s < PF_MAX_SPLITS; s++) {
-        ms[s] = (s < ns && ms[s] > -__builtin_inff()) ? fast_exp2((ms[s] - M) * LOG2E) : 0.0f;   // weights
+        ms[s] = (s < ns && ms[s] > -__builtin_inff()) ? fast_exp2(ms[s] - M) : 0.0f;   // weights
         L = __builtin_fmaf(ms[s], ls[s], L);
     }
     float out[DS];
@@ -1233,22 +1248,45 @@ int attention_prefill_fast(const uint16_t* q, const int8_t* kc, const int8_t* vc
                            const uint16_t* k_new, const uint16_t* v_new, uint16_t* o, size_t B, size_t S,
                            size_t cache_len, size_t new_len, size_t Hq, size_t Hkv, size_t d, float scale,
                            size_t pos_off, size_t qgs, void* stream) {
-    constexpr int W = 4, NB = 2, VB = 2, NV = 16 * W * VB;
+    constexpr int NB = 2, VB = 2;
     PrefillArgs a{};
     a.q = q; a.kc = kc; a.vc = vc; a.ks = ks; a.vs = vs; a.kn = k_new; a.vn = v_new; a.o = o;
     a.B = (int)B; a.S = (int)S; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.nqg = (int)((d + qgs - 1) / qgs);
     a.cache_len = cache_len; a.new_len = new_len; a.pos_off = pos_off; a.scale = scale;
     const int gq = (int)(Hq / Hkv);
-    const size_t nqb = (S * gq + NV - 1) / NV;
-    // key splits: enough workgroups to cover the CUs, at least 4 tiles each
     size_t kv_last = pos_off + S;
     if (kv_last > cache_len + new_len) kv_last = cache_len + new_len;
     const size_t tiles = (kv_last + PF_T - 1) / PF_T;
-    size_t nsplit = (512 + nqb * B * Hkv - 1) / (nqb * B * Hkv);
-    const size_t max_split = (tiles + 3) / 4;
-    if (nsplit > max_split) nsplit = max_split;
-    if (nsplit > PF_MAX_SPLITS) nsplit = PF_MAX_SPLITS;
-    if (nsplit < 1) nsplit = 1;
+    // Waves per workgroup (16 VB vectors each, one staged tile for all) and
+    // key splits, by the least time of a workgroup's tiles plus about three
+    // tiles' worth of start and partials, per round of the 256 CUs: a tile
+    // takes 1.6 us on a CU that holds four waves, 2.8 us with two such
+    // workgroups, 2.5 us with one of eight waves (half the staging per wave).
+    // 512 rows at 4096 keys, 16 / 8 heads: 54.8 us with four, 50.2 with
+    // eight; over themselves 20.2 and 22.5.  A few workgroups past a full
+    // round cost a round (333 rows at 3000 keys: 528 of four waves 51 us, 480
+    // 42).  At least 4 tiles per split; partials stay below 70 MB.
+    size_t max_split = (tiles + 3) / 4;
+    if (max_split > PF_MAX_SPLITS) max_split = PF_MAX_SPLITS;
+    int W = 4;
+    size_t nsplit = 1;
+    float best = __builtin_inff();
+    for (int w = 4; w <= 8; w += 4) {
+        const size_t wgs = (S * gq + 16 * w * VB - 1) / (16 * w * VB) * B * Hkv;
+        if (w == 8 && S * gq <= 128) break;
+        for (size_t ns = 1; ns == 1 || (ns <= max_split && wgs * ns <= (size_t)(4096 / w)); ns++) {
+            const size_t per = 2048 / w, n = wgs * ns;
+            const float tile = w == 8 ? 2.5f : n <= 256 ? 1.6f : 2.8f;
+            const float cost = (float)((n + per - 1) / per) * (float)((tiles + ns - 1) / ns + 3) * tile;
+            if (cost < best) {
+                best = cost;
+                W = w;
+                nsplit = ns;
+            }
+        }
+    }
+    const int NV = 16 * W * VB;
+    const size_t nqb = (S * gq + NV - 1) / NV;
     a.tps = (int)((tiles + nsplit - 1) / nsplit);
     a.nsplit = (int)((tiles + a.tps - 1) / a.tps);
     if (a.nsplit < 1) a.nsplit = 1;
@@ -1267,9 +1305,10 @@ int attention_prefill_fast(const uint16_t* q, const int8_t* kc, const int8_t* vc
         hipLaunchKernelGGL(comb, cgrid, dim3(256), 0, as_stream(stream), a);
         return check_launch("attention (prefill, split combine)");
     };
-#define PF_CASE(D_, G_) \
-    if (d == D_ && gq == G_) \
-        return go(attn_prefill_mfma_kernel<D_, G_, W, NB, VB>, attn_prefill_combine_kernel<D_, G_, NV>);
+#define PF_CASE(D_, G_)                                                                                           \
+    if (d == D_ && gq == G_)                                                                                      \
+        return W == 8 ? go(attn_prefill_mfma_kernel<D_, G_, 8, NB, VB>, attn_prefill_combine_kernel<D_, G_, 256>) \
+                      : go(attn_prefill_mfma_kernel<D_, G_, 4, NB, VB>, attn_prefill_combine_kernel<D_, G_, 128>);
     PF_CASE(128, 2) PF_CASE(128, 1) PF_CASE(128, 4) PF_CASE(64, 2) PF_CASE(64, 1) PF_CASE(64, 4)
 #undef PF_CASE
     return fail(CACTUS_HIP_EUNSUPPORTED, "attention (prefill, MFMA): head_dim 64/128 with 1, 2 or 4 query heads per KV head");

@@ -224,6 +224,9 @@ def test_decode_prep_attention_fast(dev, orc, cache, Hq, Hkv, d):
     (1, 3, 5, 4, 2, 128, 1.0, None),         # tiny
     (1, 500, 64, 16, 8, 128, 1.0, 530),      # position past the cache length (a windowed cache)
     (1, 0, 40, 4, 2, 128, 1.0, 17),          # no cache, rows from position 17
+    (1, 2077, 240, 16, 8, 128, 1.0, None),   # eight waves per workgroup, ragged rows, the cache ends inside a tile
+    (1, 2030, 470, 8, 8, 64, 1.0, None),     # the same at head_dim 64, where half the threads stage
+    (1, 1000, 65, 4, 2, 128, 1.0, None),     # one row past a four-wave workgroup
 ])
 def test_attention_hybrid_prefill_fast(dev, orc, B, cache, new, Hq, Hkv, d, qmul, pos):
     """Prefill rows (S = new rows at positions pos..pos+new-1, pos the
