@@ -727,45 +727,63 @@ struct PrefillArgs {
     float* part;              // split partials [B*Hkv][nqb][nsplit][16 W][D + 4]: acc[D], max, sum
     int B, S, Hq, Hkv, nqg;
     int nsplit, tps;          // key splits per query block (1: no partials), tiles per split
+    int nqb;                  // workgroups of query vectors per KV head
     size_t cache_len, new_len, pos_off;
     float scale;
 };
 
-// tiles (32 keys) a query block reads: keys up to its last row's position
-__device__ __forceinline__ int pf_block_tiles(const PrefillArgs& a, int gm0, int nv, int gq) {
-    const int last_row = min(a.S - 1, (gm0 + nv - 1) / gq);
-    size_t kv_end = a.pos_off + (size_t)last_row + 1;
-    const size_t Skv = a.cache_len + a.new_len;
-    if (kv_end > Skv) kv_end = Skv;
-    return (int)((kv_end + PF_T - 1) / PF_T);
+// Query vectors of a block: the block decides the key splits and which tiles a
+// vector takes, so a vector's result is the same bits however many blocks a
+// workgroup holds.
+constexpr int PF_BV = 128;
+
+// keys of the query block that holds vector gm: up to its last row's position
+__device__ __forceinline__ int pf_block_keys(const PrefillArgs& a, int gm, int gq) {
+    const int last_row = min(a.S - 1, (gm / PF_BV * PF_BV + PF_BV - 1) / gq);
+    const size_t kv_end = a.pos_off + (size_t)last_row + 1, Skv = a.cache_len + a.new_len;
+    return (int)(kv_end > Skv ? Skv : kv_end);
 }
 
-// max / sum over the four lanes l % 16 == c of a wave (lanes c, c + 16,
-// c + 32, c + 48), same bits in all four: v_permlane16_swap_b32 /
-// v_permlane32_swap_b32 on a value and its copy leave the lane's own value
-// in one register and its partner's (lane l ^ 16, l ^ 32) in the other.
+// first workgroup of nv query vectors whose keys reach split sp
+__host__ __device__ __forceinline__ int pf_first_block(const PrefillArgs& a, int sp, int nv, int gq) {
+    const size_t k0 = (size_t)sp * a.tps * PF_T;   // below cache_len + new_len
+    return k0 <= a.pos_off ? 0 : (int)((k0 - a.pos_off) * gq / nv);
+}
+
+// Max / sum over the four lanes l % 16 == c of a wave (lanes c, c + 16,
+// c + 32, c + 48), of two values at once.  v_permlane16_swap_b32 of a and b
+// exchanges a's odd 16-lane rows with b's even ones: a's first partial results
+// fall into the even rows and b's into the odd ones, so that the second step,
+// v_permlane32_swap_b32 of a value and its copy (the lane's own value in one
+// register, its partner's, lane l ^ 32, in the other), serves both.
 // Issued as inline assembly: the builtins' second result is lowered as a
 // copy of the first by this compiler.
-__device__ __forceinline__ void swap_pair16(float v, float& x, float& y) {
-    x = v;
-    y = v;
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y));
+__device__ __forceinline__ void swap_rows(float& a, float& b) {
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
 }
 __device__ __forceinline__ void swap_pair32(float v, float& x, float& y) {
     x = v;
     y = v;
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y));
 }
-__device__ __forceinline__ float xrow_max(float v) {
-    float x, y;
-    swap_pair16(v, x, y);
-    swap_pair32(__builtin_fmaxf(x, y), x, y);
-    return __builtin_fmaxf(x, y);
+__device__ __forceinline__ float max2f(float a, float b) {   // (a NaN operand yields the other)
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
 }
-__device__ __forceinline__ float xrow_sum(float v) {
+// a's and b's maxima, in place
+__device__ __forceinline__ void xrow_max2(float& a, float& b) {
     float x, y;
-    swap_pair16(v, x, y);
-    swap_pair32(x + y, x, y);
+    swap_rows(a, b);
+    swap_pair32(max2f(a, b), x, y);
+    a = b = max2f(x, y);
+    swap_rows(a, b);
+}
+// a's sum in the even rows, b's in the odd ones
+__device__ __forceinline__ float xrow_sum2(float a, float b) {
+    float x, y;
+    swap_rows(a, b);
+    swap_pair32(a + b, x, y);
     return x + y;
 }
 
@@ -778,13 +796,16 @@ __device__ __forceinline__ float max3f(float a, float b, float c) {
 
 // Bound by vector instructions (softmax, INT8-to-FP16 staging: ~250 per wave
 // and tile against 32 MFMAs) and by the partials, written and read once.
-// What brought 333 rows at 3000 keys, 16 / 8 heads, 49.9 -> 36.0 us: two waves
-// per SIMD (it held 304 registers: one), tile t + 2 fetched before tile t's
-// work instead of after it, one uniform mask branch per block of vectors
-// instead of one per score, value fragments read ahead of the softmax, eight
-// waves per staged tile.  The maximum of each tile is taken exactly: moving
-// it only when a score passes it by 2^8 spared rescales, but the weight of
-// the largest score was then rounded (error 3.32e-4 -> 3.49e-4).
+// What brought 333 rows at 3000 keys, 16 / 8 heads, 49.4 -> 34.9 us, every
+// rounding as before: two waves per SIMD (it held 304 registers: one), tile
+// t + 2 fetched before tile t's work instead of after it, one uniform mask
+// branch per block of vectors instead of one per score, value fragments read
+// ahead of the softmax, the row reductions of a wave's two blocks in one,
+// the splits without keys left out and the short ones last (528 workgroups
+// took three rounds of the CUs, or two; 256 of eight waves take one).  Fewer
+// splits of more keys, or scores in units of ln 2, are no slower to compute
+// but round the weights otherwise: error 3.316e-4 -> 3.329e-4 here, 3.25e-4 ->
+// 3.29e-4 for 257 rows at 1025 keys.
 template <int D, int GQ, int W, int NB, int VB>
 __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArgs a) {
     static_assert(D == 64 || D == 128, "head_dim 64 or 128");
@@ -804,14 +825,24 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lg = lane >> 4, lr = lane & 15;
-    const int bg = blockIdx.y, b = bg / a.Hkv, g = bg % a.Hkv;
-    const int qb = blockIdx.x / a.nsplit, sp_ = blockIdx.x % a.nsplit;
+    // workgroup -> (split, KV head, query blocks): split by split, so that the
+    // last split's shorter ones come last, and only those that hold keys.  KV
+    // heads are spread over the XCDs: with each on one of them (its rows lie
+    // one in Hkv, on few of the L2's channels) 256 rows at 2048 keys took 31.2
+    // us instead of 28.9
+    int id = blockIdx.x, sp_ = 0, nq = a.nqb;
+    for (; sp_ < a.nsplit; sp_++) {
+        nq = a.nqb - pf_first_block(a, sp_, NV, GQ);
+        if (id < nq * a.B * a.Hkv) break;
+        id -= nq * a.B * a.Hkv;
+    }
+    const int bg = id / nq, b = bg / a.Hkv, g = bg % a.Hkv;
+    const int qb = a.nqb - nq + id % nq;
     const int gm0 = qb * NV;
-    const size_t Skv = a.cache_len + a.new_len;
-    const int last_row = min(a.S - 1, (gm0 + NV - 1) / GQ);
-    size_t kv_end = a.pos_off + (size_t)last_row + 1;
-    if (kv_end > Skv) kv_end = Skv;
-    const int ntile_all = (int)((kv_end + PF_T - 1) / PF_T);
+    const int kv_end = pf_block_keys(a, gm0 + NV - 1, GQ);
+    const int ntile_all = (kv_end + PF_T - 1) / PF_T;
+    // this wave's block and its tiles
+    const int blk_end = pf_block_keys(a, gm0 + wid * 16 * VB, GQ), blk_tiles = (blk_end + PF_T - 1) / PF_T;
     // this workgroup's split of the tiles
     const int t_begin = sp_ * a.tps;
     const int nt = min(ntile_all - t_begin, a.tps);
@@ -827,7 +858,7 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
     for (int vb = 0; vb < VB; vb++) {
         const int row = (vm0 + 16 * vb) / GQ;
         const bool vok = row < a.S;
-        vlim[vb] = vok ? (int)min(a.pos_off + (size_t)row + 1, kv_end) : 0;
+        vlim[vb] = vok ? (int)min(a.pos_off + (size_t)row + 1, (size_t)blk_end) : 0;
         const uint16_t* qp =
             a.q + (((size_t)b * a.S + (vok ? row : 0)) * a.Hq + (size_t)g * GQ + (vm0 + 16 * vb) % GQ) * D;
 #pragma unroll
@@ -839,7 +870,7 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
     // keys that all of the wave's vectors see (its first row is its smallest
     // position; 0 if a row is missing)
     const int wrow0 = (gm0 + wid * 16 * VB) / GQ, wrow1 = (gm0 + wid * 16 * VB + 16 * VB - 1) / GQ;
-    const int wave_lim = wrow1 < a.S ? (int)min(a.pos_off + (size_t)wrow0 + 1, kv_end) : 0;
+    const int wave_lim = wrow1 < a.S ? (int)min(a.pos_off + (size_t)wrow0 + 1, (size_t)blk_end) : 0;
 
     // ---- tile staging: thread -> (key sj, NP 8-dim pieces from sp NP), lanes
     // of a wave on 32 different keys so the transposed value writes spread
@@ -862,7 +893,6 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
     // without a cache the scale loads read query words (never used)
     const float* ksb = clen > 0 ? a.ks + (size_t)g * a.nqg : reinterpret_cast<const float*>(a.q);
     const float* vsb = clen > 0 ? a.vs + (size_t)g * a.nqg : reinterpret_cast<const float*>(a.q);
-    const float sl2 = a.scale * LOG2E;   // scores in units of ln 2: weights are 2^(s - max)
     struct Raw {
         uint4 k[NP], v[NP];      // per piece 16 INT8 codes (its 8 among them) or 8 FP16 values
         float ks, vs;
@@ -888,7 +918,7 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
     auto stage = [&](int t, int buf, const Raw& r) {
         if (!stager) return;
         const int kp = t * PF_T + sj;
-        const bool live = kp < (int)kv_end, cached = kp < clen;
+        const bool live = kp < kv_end, cached = kp < clen;
 #pragma unroll
         for (int i = 0; i < NP; i++) {
             const int pc = p0 + i;
@@ -936,16 +966,16 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
 #pragma unroll
             for (int e = 0; e < 8; e++) vt[buf][8 * pc + e][sj] = vh[e];
         }
-        if (sp == 0) ksc[buf][sj] = (cached ? r.ks : 1.0f) * sl2;
+        if (sp == 0) ksc[buf][sj] = (cached ? r.ks : 1.0f) * a.scale;
     };
 
     const float NEG_INF = -__builtin_inff();
-    float m_run[VB], l_run[VB];
+    static_assert(VB == 2, "the row reductions take the wave's blocks in pairs");
+    float m_run[VB], l_run = 0.0f;   // l_run: block 0's sums in the even 16-lane rows, block 1's in the odd
     f32x4 acc[VB][ND];   // O^T: lane l holds dims 16 db + 4 lg + i of vector lr of each block
 #pragma unroll
     for (int vb = 0; vb < VB; vb++) {
         m_run[vb] = NEG_INF;
-        l_run[vb] = 0.0f;
 #pragma unroll
         for (int db = 0; db < ND; db++) acc[vb][db] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
     }
@@ -964,86 +994,98 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
         // tile t is staged, so its slot takes tile t + NB: its loads have NB
         // tiles' work to arrive in (clamped rows: in bounds past the split too)
         fetch(t + NB, raw[u]);
-        // scores S^T for keys 16h + 4lg + i of the tile, vector lr of each block
-        f32x4 st[VB][2];
+        if (W * 16 * VB == PF_BV || t < blk_tiles) {   // (the same for the whole wave)
+            // scores S^T for keys 16h + 4lg + i of the tile, vector lr of each block
+            f32x4 st[VB][2];
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+            for (int h = 0; h < 2; h++) {
 #pragma unroll
-            for (int vb = 0; vb < VB; vb++) st[vb][h] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+                for (int vb = 0; vb < VB; vb++) st[vb][h] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int c = 0; c < NC; c++) {
-                const h16x8 kv = *reinterpret_cast<const h16x8*>(&ksh[buf][16 * h + lr][32 * c + 8 * lg]);
+                for (int c = 0; c < NC; c++) {
+                    const h16x8 kv = *reinterpret_cast<const h16x8*>(&ksh[buf][16 * h + lr][32 * c + 8 * lg]);
 #pragma unroll
-                for (int vb = 0; vb < VB; vb++)
-                    st[vb][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv, qv[vb][c], st[vb][h], 0, 0, 0);
-            }
-        }
-        // a tile below every row's causal end and the key range needs no
-        // mask (wave-uniform test); the others mask key by key
-        const bool interior = t * PF_T + PF_T <= wave_lim;
-        const f32x4 ksv0 = *reinterpret_cast<const f32x4*>(&ksc[buf][4 * lg]);
-        const f32x4 ksv1 = *reinterpret_cast<const f32x4*>(&ksc[buf][16 + 4 * lg]);
-        // A = V^T (dims 16 db + lr, the same 8 keys): all reads in flight
-        // during the softmax (left to the compiler each waits at its MFMAs)
-        h16x8 va[ND];
-#pragma unroll
-        for (int db = 0; db < ND; db++) {
-            const h16x4 v0 = *reinterpret_cast<const h16x4*>(&vt[buf][16 * db + lr][4 * lg]);
-            const h16x4 v1 = *reinterpret_cast<const h16x4*>(&vt[buf][16 * db + lr][16 + 4 * lg]);
-            va[db] = (h16x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        h16x8 pa[VB];   // P^T operands: keys {4 lg + j, 16 + 4 lg + j} of vector lr
-#pragma unroll
-        for (int vb = 0; vb < VB; vb++) {
-            float s[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) s[j] = st[vb][j >> 2][j & 3] * (j < 4 ? ksv0[j & 3] : ksv1[j & 3]);
-            if (!interior) {
-                const int rem = vlim[vb] - t * PF_T - 4 * lg;   // visible keys from the lane's first
-#pragma unroll
-                for (int j = 0; j < 8; j++)
-                    if (16 * (j >> 2) + (j & 3) >= rem) s[j] = NEG_INF;
-            }
-            float mx = max3f(max3f(max3f(s[0], s[1], s[2]), s[3], s[4]), max3f(s[5], s[6], s[7]), NEG_INF);
-            // a tile that moves no running max of the wave's 16 vectors needs
-            // no rescale (wave-uniform branch)
-            mx = xrow_max(mx);
-            const float m_old = m_run[vb];
-            if (__any(mx > m_old)) {
-                const float m_new = __builtin_fmaxf(m_old, mx);
-                const float corr = m_new > NEG_INF ? fast_exp2(m_old - m_new) : 1.0f;
-                l_run[vb] *= corr;
-                m_run[vb] = m_new;
-#pragma unroll
-                for (int db = 0; db < ND; db++) acc[vb][db] *= corr;
-            }
-            // masked scores weigh 2^-inf = 0 (also while no key is live: 2^(-inf - 0))
-            const float m = m_run[vb] > NEG_INF ? m_run[vb] : 0.0f;
-            float pv[8], psum = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                pv[j] = fast_exp2(s[j] - m);
-                psum += pv[j];
-            }
-            if (__any(psum != psum)) {   // a NaN score is left out, as a masked one
-                psum = 0.0f;
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    if (!(s[j] > NEG_INF)) pv[j] = 0.0f;
-                    psum += pv[j];
+                    for (int vb = 0; vb < VB; vb++)
+                        st[vb][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv, qv[vb][c], st[vb][h], 0, 0, 0);
                 }
             }
+            // a tile below every row's causal end and the key range needs no
+            // mask (wave-uniform test); the others mask key by key
+            const bool interior = t * PF_T + PF_T <= wave_lim;
+            const f32x4 ksv0 = *reinterpret_cast<const f32x4*>(&ksc[buf][4 * lg]);
+            const f32x4 ksv1 = *reinterpret_cast<const f32x4*>(&ksc[buf][16 + 4 * lg]);
+            // A = V^T (dims 16 db + lr, the same 8 keys): all reads in flight
+            // during the softmax (left to the compiler each waits at its MFMAs)
+            h16x8 va[ND];
 #pragma unroll
-            for (int j = 0; j < 8; j++) pa[vb][j] = (_Float16)pv[j];
-            l_run[vb] += psum;   // this lane's keys; the four lanes add up at the end
-        }
-        // O^T += V^T P^T
+            for (int db = 0; db < ND; db++) {
+                const h16x4 v0 = *reinterpret_cast<const h16x4*>(&vt[buf][16 * db + lr][4 * lg]);
+                const h16x4 v1 = *reinterpret_cast<const h16x4*>(&vt[buf][16 * db + lr][16 + 4 * lg]);
+                va[db] = (h16x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            float sc[VB][8], mx[VB];
 #pragma unroll
-        for (int db = 0; db < ND; db++) {
+            for (int vb = 0; vb < VB; vb++) {
+                float(&s)[8] = sc[vb];
 #pragma unroll
-            for (int vb = 0; vb < VB; vb++)
-                acc[vb][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[db], pa[vb], acc[vb][db], 0, 0, 0);
+                for (int j = 0; j < 8; j++) s[j] = st[vb][j >> 2][j & 3] * (j < 4 ? ksv0[j & 3] : ksv1[j & 3]);
+                if (!interior) {
+                    const int rem = vlim[vb] - t * PF_T - 4 * lg;   // visible keys from the lane's first
+#pragma unroll
+                    for (int j = 0; j < 8; j++)
+                        if (16 * (j >> 2) + (j & 3) >= rem) s[j] = NEG_INF;
+                }
+                mx[vb] = max3f(max3f(max3f(s[0], s[1], s[2]), s[3], s[4]), max3f(s[5], s[6], s[7]), NEG_INF);
+            }
+            xrow_max2(mx[0], mx[1]);
+            // a tile that moves no running max of the wave's vectors needs no
+            // rescale (wave-uniform branch)
+            if (__any(mx[0] > m_run[0] || mx[1] > m_run[1])) {
+                float corr[VB];
+#pragma unroll
+                for (int vb = 0; vb < VB; vb++) {
+                    const float m_new = max2f(m_run[vb], mx[vb]);
+                    corr[vb] = m_new > NEG_INF ? fast_exp2((m_run[vb] - m_new) * LOG2E) : 1.0f;
+                    m_run[vb] = m_new;
+#pragma unroll
+                    for (int db = 0; db < ND; db++) acc[vb][db] *= corr[vb];
+                }
+                l_run *= lg & 1 ? corr[1] : corr[0];
+            }
+            h16x8 pa[VB];   // P^T operands: keys {4 lg + j, 16 + 4 lg + j} of vector lr
+            float psum[VB];
+#pragma unroll
+            for (int vb = 0; vb < VB; vb++) {
+                const float(&s)[8] = sc[vb];
+                // masked scores weigh 2^-inf = 0 (also while no key is live: 2^(-inf - 0))
+                const float m = m_run[vb] > NEG_INF ? m_run[vb] : 0.0f;
+                float pv[8];
+                psum[vb] = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    pv[j] = fast_exp2((s[j] - m) * LOG2E);
+                    psum[vb] += pv[j];
+                }
+                if (__any(psum[vb] != psum[vb])) {   // a NaN score is left out, as a masked one
+                    psum[vb] = 0.0f;
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        if (!(s[j] > NEG_INF)) pv[j] = 0.0f;
+                        psum[vb] += pv[j];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j++) pa[vb][j] = (_Float16)pv[j];
+            }
+            l_run += xrow_sum2(psum[0], psum[1]);
+            // O^T += V^T P^T
+#pragma unroll
+            for (int db = 0; db < ND; db++) {
+#pragma unroll
+                for (int vb = 0; vb < VB; vb++)
+                    acc[vb][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[db], pa[vb], acc[vb][db], 0, 0, 0);
+            }
         }
         // the next tile into the other LDS buffer (its last readers finished
         // before the previous barrier)
@@ -1052,26 +1094,26 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
     }
 
     // ---- output: vector lr of each block, dims 16 db + 4 lg + i
+    float l_sum[VB] = {l_run, l_run};
+    swap_rows(l_sum[0], l_sum[1]);
 #pragma unroll
     for (int vb = 0; vb < VB; vb++) {
-        l_run[vb] = xrow_sum(l_run[vb]);
         if (a.nsplit > 1) {
             // this split's partial (acc, running max, sum) of the vector
-            const int nqb = (int)gridDim.x / a.nsplit;
             float* pp = a.part +
-                        ((((size_t)bg * nqb + qb) * a.nsplit + sp_) * NV + (wid * VB + vb) * 16 + lr) * (D + 4);
+                        ((((size_t)bg * a.nqb + qb) * a.nsplit + sp_) * NV + (wid * VB + vb) * 16 + lr) * (D + 4);
 #pragma unroll
             for (int db = 0; db < ND; db++) *reinterpret_cast<f32x4*>(pp + 16 * db + 4 * lg) = acc[vb][db];
             if (lg == 0) {
                 pp[D] = m_run[vb];
-                pp[D + 1] = l_run[vb];
+                pp[D + 1] = l_sum[vb];
             }
             continue;
         }
         const int vm = vm0 + 16 * vb;
         if (vm / GQ >= a.S) continue;
         uint16_t* op = a.o + (((size_t)b * a.S + vm / GQ) * a.Hq + (size_t)g * GQ + vm % GQ) * D;
-        const float inv = l_run[vb] > 0.0f ? 1.0f / l_run[vb] : 0.0f;
+        const float inv = l_sum[vb] > 0.0f ? 1.0f / l_sum[vb] : 0.0f;
 #pragma unroll
         for (int db = 0; db < ND; db++) {
             const uint32_t lo = (uint32_t)f2h(acc[vb][db][0] * inv) | ((uint32_t)f2h(acc[vb][db][1] * inv) << 16);
@@ -1084,28 +1126,28 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
 // Combine of the key splits: grid (query blocks x NV / 16, B * Hkv), 256
 // threads; a workgroup takes 16 query vectors, 16 threads per vector with
 // D/16 dims each.  M = max_s M_s, L = sum_s e^(M_s - M) l_s,
-// o = sum_s e^(M_s - M) acc_s / L (maxima in units of ln 2).  Loads are branch-free (clamped splits,
+// o = sum_s e^(M_s - M) acc_s / L.  Loads are branch-free (clamped splits,
 // weight 0 past the block's split count) and issued per batch of splits.
 constexpr int PF_MAX_SPLITS = 16;
 
 template <int D, int GQ, int NV>
 __global__ void __launch_bounds__(256) attn_prefill_combine_kernel(PrefillArgs a) {
     constexpr int VPW = 16, DS = D / 16, SB = 4;
+    constexpr float LOG2E = 1.4426950408889634f;
     const int tid = threadIdx.x, vl = tid / 16, dq = (tid % 16) * DS;
     const int qb = blockIdx.x / (NV / VPW), v = (blockIdx.x % (NV / VPW)) * VPW + vl;
     const int bg = blockIdx.y, b = bg / a.Hkv, g = bg % a.Hkv;
-    const int nqb = (int)gridDim.x / (NV / VPW);
     const int gm0 = qb * NV;
-    const int ns = min(a.nsplit, (pf_block_tiles(a, gm0, NV, GQ) + a.tps - 1) / a.tps);
     const int vm = gm0 + v, row = vm / GQ;
     if (row >= a.S) return;
+    const int ns = min(a.nsplit, ((pf_block_keys(a, vm, GQ) + PF_T - 1) / PF_T + a.tps - 1) / a.tps);
     uint16_t* op = a.o + (((size_t)b * a.S + row) * a.Hq + (size_t)g * GQ + vm % GQ) * D + dq;
     if (ns <= 0) {   // no key tile reaches this block: zero rows, as with L = 0
 #pragma unroll
         for (int e = 0; e < DS; e += 2) *reinterpret_cast<uint32_t*>(op + e) = 0u;
         return;
     }
-    const float* pb = a.part + (((size_t)bg * nqb + qb) * a.nsplit * NV + v) * (D + 4);
+    const float* pb = a.part + (((size_t)bg * a.nqb + qb) * a.nsplit * NV + v) * (D + 4);
     const size_t sstep = (size_t)NV * (D + 4);
     float ms[PF_MAX_SPLITS], ls[PF_MAX_SPLITS];
 #pragma unroll
@@ -1121,7 +1163,7 @@ __global__ void __launch_bounds__(256) attn_prefill_combine_kernel(PrefillArgs a
     float L = 0.0f;
 #pragma unroll
     for (int s = 0; s < PF_MAX_SPLITS; s++) {
-        ms[s] = (s < ns && ms[s] > -__builtin_inff()) ? fast_exp2(ms[s] - M) : 0.0f;   // weights
+        ms[s] = (s < ns && ms[s] > -__builtin_inff()) ? fast_exp2((ms[s] - M) * LOG2E) : 0.0f;   // weights
         L = __builtin_fmaf(ms[s], ls[s], L);
     }
     float out[DS];
@@ -1257,46 +1299,46 @@ int attention_prefill_fast(const uint16_t* q, const int8_t* kc, const int8_t* vc
     size_t kv_last = pos_off + S;
     if (kv_last > cache_len + new_len) kv_last = cache_len + new_len;
     const size_t tiles = (kv_last + PF_T - 1) / PF_T;
-    // Waves per workgroup (16 VB vectors each, one staged tile for all) and
-    // key splits, by the least time of a workgroup's tiles plus about three
-    // tiles' worth of start and partials, per round of the 256 CUs: a tile
-    // takes 1.6 us on a CU that holds four waves, 2.8 us with two such
-    // workgroups, 2.5 us with one of eight waves (half the staging per wave).
-    // 512 rows at 4096 keys, 16 / 8 heads: 54.8 us with four, 50.2 with
-    // eight; over themselves 20.2 and 22.5.  A few workgroups past a full
-    // round cost a round (333 rows at 3000 keys: 528 of four waves 51 us, 480
-    // 42).  At least 4 tiles per split; partials stay below 70 MB.
-    size_t max_split = (tiles + 3) / 4;
-    if (max_split > PF_MAX_SPLITS) max_split = PF_MAX_SPLITS;
-    int W = 4;
-    size_t nsplit = 1;
-    float best = __builtin_inff();
-    for (int w = 4; w <= 8; w += 4) {
-        const size_t wgs = (S * gq + 16 * w * VB - 1) / (16 * w * VB) * B * Hkv;
-        if (w == 8 && S * gq <= 128) break;
-        for (size_t ns = 1; ns == 1 || (ns <= max_split && wgs * ns <= (size_t)(4096 / w)); ns++) {
-            const size_t per = 2048 / w, n = wgs * ns;
-            const float tile = w == 8 ? 2.5f : n <= 256 ? 1.6f : 2.8f;
-            const float cost = (float)((n + per - 1) / per) * (float)((tiles + ns - 1) / ns + 3) * tile;
-            if (cost < best) {
-                best = cost;
-                W = w;
-                nsplit = ns;
-            }
-        }
-    }
-    const int NV = 16 * W * VB;
-    const size_t nqb = (S * gq + NV - 1) / NV;
+    // Key splits: two workgroups of one block per CU, at least 4 tiles each.
+    // The blocks and their splits, and with them the result's bits, do not
+    // depend on how many blocks a workgroup holds.
+    static_assert(16 * 4 * VB == PF_BV, "four waves hold one block");
+    const size_t nblk = (S * gq + PF_BV - 1) / PF_BV * B * Hkv;
+    size_t nsplit = (512 + nblk - 1) / nblk;
+    if (nsplit > (tiles + 3) / 4) nsplit = (tiles + 3) / 4;
+    if (nsplit > PF_MAX_SPLITS) nsplit = PF_MAX_SPLITS;
+    if (nsplit < 1) nsplit = 1;
     a.tps = (int)((tiles + nsplit - 1) / nsplit);
     a.nsplit = (int)((tiles + a.tps - 1) / a.tps);
     if (a.nsplit < 1) a.nsplit = 1;
+    auto set_blocks = [&](int nv) {
+        a.nqb = (int)((S * gq + nv - 1) / nv);
+        size_t n = 0;
+        for (int sp = 0; sp < a.nsplit; sp++) n += (size_t)(a.nqb - pf_first_block(a, sp, nv, gq)) * B * Hkv;
+        return n;
+    };
+    // Eight waves per staged tile (half the staging per wave, but one
+    // workgroup per CU) where a tile's staging is large (128 dims), the start
+    // of a workgroup is spread over several tiles and its rounds of the 256
+    // CUs are nearly full (us, four / eight waves, 16 / 8 heads of 128 dims:
+    // 333 rows at 3000 keys 35.4 / 34.9, 512 at 4096 49.4 / 47.5; four tiles a
+    // split, 256 at 2048, 29.1 / 29.5; half a round, 512 over themselves,
+    // 18.7 / 22.3; 512 at 4096 with 64 dims, 8 / 8 heads, 23.5 / 26.4).
+    int W = 8;
+    size_t wgs = set_blocks(16 * 8 * VB);
+    if (d != 128 || a.tps < 6 || wgs * 8 < (wgs + 255) / 256 * 256 * 7) {
+        W = 4;
+        wgs = set_blocks(16 * 4 * VB);
+    }
+    const int NV = 16 * W * VB;
+    const size_t nqb = (size_t)a.nqb;
     if (a.nsplit > 1) {
         FastWs w;
         const int rc = fast_ws(stream, B * Hkv * nqb * (size_t)a.nsplit * NV * (d + 4), 0, &w);
         if (rc) return rc;
         a.part = w.part;
     }
-    const dim3 grid((unsigned)(nqb * a.nsplit), (unsigned)(B * Hkv));
+    const dim3 grid((unsigned)wgs);
     const dim3 cgrid((unsigned)(nqb * (NV / 16)), (unsigned)(B * Hkv));
     auto go = [&](auto kern, auto comb) {
         hipLaunchKernelGGL(kern, grid, dim3(64 * W), 0, as_stream(stream), a);
@@ -1307,8 +1349,9 @@ int attention_prefill_fast(const uint16_t* q, const int8_t* kc, const int8_t* vc
     };
 #define PF_CASE(D_, G_)                                                                                           \
     if (d == D_ && gq == G_)                                                                                      \
-        return W == 8 ? go(attn_prefill_mfma_kernel<D_, G_, 8, NB, VB>, attn_prefill_combine_kernel<D_, G_, 256>) \
-                      : go(attn_prefill_mfma_kernel<D_, G_, 4, NB, VB>, attn_prefill_combine_kernel<D_, G_, 128>);
+        return D_ == 128 && W == 8                                                                                \
+                   ? go(attn_prefill_mfma_kernel<128, G_, 8, NB, VB>, attn_prefill_combine_kernel<128, G_, 256>)  \
+                   : go(attn_prefill_mfma_kernel<D_, G_, 4, NB, VB>, attn_prefill_combine_kernel<D_, G_, 128>);
     PF_CASE(128, 2) PF_CASE(128, 1) PF_CASE(128, 4) PF_CASE(64, 2) PF_CASE(64, 1) PF_CASE(64, 4)
 #undef PF_CASE
     return fail(CACTUS_HIP_EUNSUPPORTED, "attention (prefill, MFMA): head_dim 64/128 with 1, 2 or 4 query heads per KV head");

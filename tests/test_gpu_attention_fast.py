@@ -15,6 +15,7 @@ form run the FP16-MFMA flash kernel (chunk shapes of a 4096-token prefill,
 with and without key splits and their combine).
 """
 import ctypes
+import hashlib
 import math
 import sys
 
@@ -263,3 +264,29 @@ def test_attention_hybrid_prefill_fast(dev, orc, B, cache, new, Hq, Hkv, d, qmul
                 dev.put(vn), o.ptr, B, new, cache, new, Hq, Hkv, d, ctypes.c_float(scale), pos, 1, 128, None)
     err = close(dev.get(o, np.uint16, q.shape), ref, "attention_hybrid_prefill_fast")
     print(f"[prefill fast] max abs error {err:.2e}", flush=True)
+
+
+@pytest.mark.parametrize("S,T,Hq,Hkv,d,digest", [
+    (333, 3000, 16, 8, 128, "ea278d1ad75ae9f9"), (512, 3000, 8, 2, 128, "d9ad33f4081e79c5"),   # eight waves per tile
+    (130, 500, 16, 4, 64, "bb1c32ea27e7e56f"), (37, 517, 2, 2, 128, "3a9d1f1fd9dffa24"),
+    (70, 70, 4, 4, 64, "b86b7539f6f7e537")])
+def test_attention_hybrid_prefill_fast_bits(dev, S, T, Hq, Hkv, d, digest):
+    """The roundings of the tolerance-mode prefill stay what they are: scores
+    times scale, weights 2^((s - max) log2 e) against each key split's running
+    maximum, sums per 32-key tile, the splits of 128-vector blocks.  The
+    digests are those of the first form of the kernel (four waves per
+    workgroup, one block each); forms with other splits and with scores in
+    units of ln 2 gave other bits and an error against 64 bits up to 1.4%
+    larger."""
+    say("attention_hybrid_prefill_fast bits", S, T, Hq, Hkv, d)
+    r = np.random.RandomState(S + T)
+    C = T - S
+    half = lambda *s: (r.randint(-512, 513, s) / 256).astype(np.float16)
+    q, kn, vn = half(S, Hq, d), half(S, Hkv, d), half(S, Hkv, d)
+    kc, vc = (r.randint(-127, 128, (max(C, 1), Hkv, d)).astype(np.int8) for _ in range(2))
+    ks, vs = ((r.randint(64, 256, (max(C, 1), Hkv, 1)) / 16384).astype(np.float32) for _ in range(2))
+    o = dev.put(np.full(q.shape, 9.0, np.float16))
+    dev.cm.call("cactus_hip_attention_hybrid_int8_fp16_fast", *map(dev.put, (q, kc, vc, ks, vs, kn, vn)), o, 1, S, C, S,
+                Hq, Hkv, d, ctypes.c_float(1 / math.sqrt(d)), C, 1, 128, None)
+    got = dev.get_ptr(o, np.uint16, q.shape)
+    assert hashlib.sha256(got.tobytes()).hexdigest()[:16] == digest
