@@ -600,9 +600,13 @@ static int gemm_scratch(hipStream_t st, size_t bytes, void** out) {
 // 6.7, M=19 40 / 6.9, M=31 66 / 7.0; INT4 K=3072 N=1024 M=4 10.5 / 11.7, M=5
 // 16.5 / 11.7.  Pre-quantized rows skip the 2-4 us quantization launch.
 constexpr size_t GEMM_MIN_M_INT8 = 3, GEMM_MIN_M_INT4 = 5, GEMM_MIN_M_CODES = 3;
-// Below this many rows the FP16 forms never needed device memory of their
-// own: inside a graph capture that would have to allocate they keep the GEMV.
-constexpr size_t GEMM_NOALLOC_M = 32;
+// Below this many rows the FP16 forms take the matrix cores only where the
+// stream's scratch, which they pass the codes on through, is theirs alone: a
+// captured graph outlives the call, and its stream's scratch with it may not,
+// or may be in use when the graph runs on another stream; the static buffer of
+// the no-allocation entry belongs to every stream; hipStreamPerThread is one
+// handle for many streams.  Those calls keep the GEMV, which needs no memory.
+constexpr size_t GEMM_SCRATCH_M = 32;
 
 // Returns *handled = false when the shape is left to the GEMV path.
 // Activation codes ([M][K] int8, padded to 256 bytes) and row scales
@@ -618,9 +622,9 @@ int gemm_grouped_mfma(const uint16_t* A16, const int8_t* A8, const float* As, co
     if (((uintptr_t)B & 15) != 0) return CACTUS_HIP_OK;
     if (!A16 && (((uintptr_t)A8 & 15) != 0)) return CACTUS_HIP_OK;
     if (M >= (1u << 30) || N >= (1u << 30) || K >= (1u << 20)) return CACTUS_HIP_OK;
-    if (A16 && !ext_scratch && M < GEMM_NOALLOC_M &&
-        !stream_scratch_ready(SCR_GEMM_ACT, st, gemm_act_scratch_bytes(M, K)))
+    if (A16 && M < GEMM_SCRATCH_M && (ext_scratch || st == hipStreamPerThread || stream_capturing(st)))
         return CACTUS_HIP_OK;
+    std::unique_lock<std::mutex> order;
     const int8_t* Aq = A8;
     const float* Asc = As;
     if (A16) {
@@ -628,7 +632,12 @@ int gemm_grouped_mfma(const uint16_t* A16, const int8_t* A8, const float* As, co
         const size_t qbytes = (M * K + 255) & ~(size_t)255;
         void* scr = ext_scratch;
         if (!scr) {
-            int rc = gemm_scratch(st, gemm_act_scratch_bytes(M, K), &scr);
+            order = stream_launch_lock(st);
+            const int rc = gemm_scratch(st, gemm_act_scratch_bytes(M, K), &scr);
+            if (rc && M < GEMM_SCRATCH_M) {
+                (void)hipGetLastError();
+                return CACTUS_HIP_OK;   // no memory to be had: the GEMV
+            }
             if (rc) return rc;
         }
         int rc;

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stddef.h>
+#include <mutex>
 #include <string>
 #include <cstring>
 
@@ -69,6 +70,12 @@ int stream_scratch(int kind, void* stream, size_t bytes, bool zero, void** out);
 // whether stream_scratch can serve the request without allocating inside a
 // graph capture (which the capture mode may refuse)
 bool stream_scratch_ready(int kind, void* stream, size_t bytes);
+// whether a graph is being captured on `stream` (and if that cannot be told)
+bool stream_capturing(void* stream);
+// To be held over the launches of a call that pass data on through the
+// stream's scratch: another host thread's call on the stream then comes before
+// or behind all of them.
+std::unique_lock<std::mutex> stream_launch_lock(void* stream);
 // frees every scratch buffer of `stream` (all devices) after synchronizing it
 int stream_scratch_release(void* stream);
 

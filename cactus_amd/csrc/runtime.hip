@@ -117,6 +117,18 @@ int stream_scratch(int kind, void* stream, size_t bytes, bool zero, void** out) 
     return CACTUS_HIP_OK;
 }
 
+bool stream_capturing(void* stream) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return stream && (hipStreamIsCapturing(as_stream(stream), &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
+}
+
+std::unique_lock<std::mutex> stream_launch_lock(void* stream) {
+    static std::mutex mu[64];   // streams that share one only wait for each other's launches
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    return std::unique_lock<std::mutex>(mu[(((uintptr_t)stream >> 4) + (uintptr_t)dev) * 0x9E3779B97F4A7C15ull >> 58]);
+}
+
 bool stream_scratch_ready(int kind, void* stream, size_t bytes) {
     const hipStream_t st = as_stream(stream);
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;

@@ -109,12 +109,12 @@ int cactus_hip_matmul_int8_f16act(const uint16_t* A, const int8_t* B, const uint
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc): the same kernels
  * and results, with the activation codes and row scales of the MFMA path
- * (a few rows and more) in a static 4 MiB device buffer instead of a buffer
- * the library allocates.  Rejects, with CACTUS_HIP_EINVAL and before any launch, shapes
+ * (M >= 32) in a static 4 MiB device buffer instead of a buffer the library
+ * allocates.  Rejects, with CACTUS_HIP_EINVAL and before any launch, shapes
  * whose ((M*K + 255) & ~255) + 4*M bytes exceed 4 MiB (e.g. M = 4096 at
  * K = 1024).  Calls no hipMalloc / hipFree.  Every call on one GPU shares
- * that GPU's buffer: calls that overlap on one GPU (two streams, two host
- * threads) race.  Each call rewrites every byte it reads, so nothing
+ * that GPU's buffer: calls of 32 rows and more that overlap on one GPU (two
+ * streams, two host threads) race.  Each call rewrites every byte it reads, so nothing
  * carries over from the previous call. */
 int cactus_hip_matmul_int8_f16act_noalloc(const uint16_t* A, const int8_t* B, const uint16_t* B_scales,
                                           uint16_t* C, size_t M, size_t K, size_t N, size_t group_size,

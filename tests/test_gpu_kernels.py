@@ -7,6 +7,7 @@ HIP kernels follow the reference's order of operations exactly.
 import ctypes
 import math
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -242,6 +243,83 @@ def test_matmul_few_rows_captured_cold(dev, orc):
         st.sync()
         assert_bits(dev.get(C, np.uint16, (M, N)), ref, "eager %d" % rep)
     dev.cm.call("cactus_hip_graph_destroy", g.value)
+
+
+@pytest.mark.parametrize("entry,M", [("int8_f16act", 4), ("int8_f16act", 31), ("int8_f16act_noalloc", 4),
+                                     ("int4_f16act", 12)])
+def test_matmul_few_rows_captured_warm(dev, orc, entry, M):
+    """Few rows captured on a stream whose scratch is there already: the graph
+    holds GEMV launches of four rows, none that passes data on through
+    library memory, and is right on another stream and after its own is gone."""
+    say("matmul few rows captured, warm", entry, M)
+    K, N, gs = 1024, 512, 32
+    rng = np.random.default_rng(M)
+    x, other = activations(rng, M, K), activations(rng, M, K)
+    if entry.startswith("int4"):
+        _, B, Bs = grouped_int4_weights(rng, N, K, gs)
+        ref = orc.matmul_int4(*orc.quantize_activations(x), B, Bs, gs)
+    else:
+        B, Bs = grouped_int8_weights(rng, N, K, gs)
+        ref = orc.matmul_int8(*orc.quantize_activations(x), B, Bs, gs)
+    xp, op, Bp, Bsp, C, C2 = dev.put(x), dev.put(other), dev.put(B), dev.put(Bs), dev.empty(M * N * 2), dev.empty(M * N * 2)
+    name = "cactus_hip_matmul_" + entry
+    st, st2 = dev.cm.Stream(), dev.cm.Stream()
+    dev.cm.call(name, xp, Bp, Bsp, C.ptr, M, K, N, gs, st.handle)
+    hip = dev.cm.hip()   # (symbols of the HIP runtime it is linked to)
+    hip.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    hip.hipGraphGetNodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    hip.hipGraphDestroy.argtypes = [ctypes.c_void_p]
+    graph, nodes = ctypes.c_void_p(), ctypes.c_size_t()
+    dev.cm.call("cactus_hip_graph_capture_begin", st.handle)
+    dev.cm.call(name, xp, Bp, Bsp, C.ptr, M, K, N, gs, st.handle)
+    assert hip.hipStreamEndCapture(st.handle, ctypes.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    assert nodes.value == -(-M // 4)
+    g = ctypes.c_void_p()
+    dev.cm.call("cactus_hip_graph_capture_begin", st.handle)
+    dev.cm.call(name, xp, Bp, Bsp, C.ptr, M, K, N, gs, st.handle)
+    dev.cm.call("cactus_hip_graph_capture_end", st.handle, ctypes.byref(g))
+    for rep in range(4):
+        if rep == 2:
+            st.sync()
+            dev.cm.call("cactus_hip_stream_destroy", st.handle)
+            st.handle = None
+        if rep < 2:
+            dev.cm.call(name, op, Bp, Bsp, C2.ptr, M, K, N, gs, st.handle)   # beside the graph
+        dev.cm.call("cactus_hip_memset", C.ptr, 0, M * N * 2, st2.handle)
+        dev.cm.call("cactus_hip_graph_launch", g.value, st2.handle)
+        st2.sync()
+        assert_bits(dev.get(C, np.uint16, (M, N)), ref, "replay %d" % rep)
+    dev.cm.call("cactus_hip_graph_destroy", g.value)
+
+
+@pytest.mark.parametrize("M", [8, 40])
+def test_matmul_two_threads_one_stream(dev, orc, M):
+    """Two host threads with rows of their own on the default stream: every
+    call multiplies the rows it was given."""
+    say("matmul two threads", M)
+    K, N, gs, reps = 1024, 256, 32, 100
+    rng = np.random.default_rng(M)
+    B, Bs = grouped_int8_weights(rng, N, K, gs)
+    Bp, Bsp = dev.put(B), dev.put(Bs)
+    xs = [activations(rng, M, K) for _ in range(2)]
+    xp = [dev.put(x) for x in xs]
+    out = [dev.empty(reps * M * N * 2) for _ in xs]
+
+    def work(i):
+        for r in range(reps):
+            dev.cm.call("cactus_hip_matmul_int8_f16act", xp[i], Bp, Bsp, out[i].ptr + r * M * N * 2, M, K, N, gs, None)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i in range(2):
+        got = dev.get(out[i], np.uint16, (reps, M, N))
+        ref = orc.matmul_int8(*orc.quantize_activations(xs[i]), B, Bs, gs)
+        assert all((got[r] == ref).all() for r in range(reps)), i
 
 
 def test_matmul_int8_batched(dev, orc):
