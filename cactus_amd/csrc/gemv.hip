@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(GEMV_THREADS) gemv_grouped_kernel(GemvArgs a, 
     for (int m = 0; m < mr; m++) {
         if (F16ACT) {
             const uint16_t* x = a.A16 + bi * a.sA + (size_t)(m0 + m) * K;
-            const float mx = block_max_abs_f16(x, K, red);
+            const float mx = block_max_abs_f16<GEMV_THREADS>(x, K, red);
             const float s = row_scale_from_max(mx);
             const float inv = 1.0f / s;
             if constexpr (INT4) {
@@ -346,7 +346,7 @@ __global__ void __launch_bounds__(GEMV_THREADS) gemv_wave_kernel(GemvArgs a, int
     for (int m = 0; m < mr; m++) {
         if (F16ACT) {
             const uint16_t* x = a.A16 + bi * a.sA + (size_t)(m0 + m) * K;
-            const float mx = block_max_abs_f16(x, K, red);
+            const float mx = block_max_abs_f16<GEMV_THREADS>(x, K, red);
             const float s = row_scale_from_max(mx);
             const float inv = 1.0f / s;
             if constexpr (INT4) {

@@ -26,12 +26,17 @@ __device__ __forceinline__ float row_scale_from_max(float m) {
 }
 
 // Block-wide max of |x[0..K)|; every thread returns the result.  `red` must
-// hold blockDim.x/64 floats of LDS.
+// hold a float per wave in LDS.  NT: the workgroup's threads where the kernel
+// fixes them: blockDim.x is one more dependent scalar load, from a cache line
+// of its own behind a launch's arguments (GEMV, us at M=1: INT8 K=640 N=1024
+// 4.48 -> 4.14, INT4 K=1024 N=2048 4.33 -> 4.01; M=2 INT8 K=640 N=1024 5.72 ->
+// 5.25; the one that loses is M=2 INT8 K=3072 N=1024, 8.7 -> 9.0).
+template <int NT = 0>
 __device__ __forceinline__ float block_max_abs_f16(const uint16_t* __restrict__ x, int K,
                                                    float* red) {
     float m = 0.0f;
     const int tid = threadIdx.x;
-    const int nt = blockDim.x;
+    const int nt = NT ? NT : (int)blockDim.x;
     // 8 fp16 per 16-byte load when aligned
     if ((((uintptr_t)x) & 15) == 0) {
         const int K8 = K / 8;
