@@ -19,8 +19,9 @@
 namespace cactus {
 
 // Rows from which the grouped matmuls of FP16 activations run on the matrix
-// cores whatever their format: the nodes in front of them then quantize the
-// rows once for all their consumers, and consumers of one input share a launch.
+// cores, INT8 or INT4 in groups of up to 128: the nodes in front of them then
+// quantize the rows once for all their consumers, and consumers of one input
+// share a launch.
 constexpr size_t kBatchedRows = 5;
 
 // graph.h:99-104 (same order: INT8, FP16, FP32, INT4)

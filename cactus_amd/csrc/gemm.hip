@@ -599,7 +599,16 @@ static int gemm_scratch(hipStream_t st, size_t bytes, void** out) {
 // quantization): INT8 K=1024 N=2048 M=2 6.2 / 6.7, M=4 8.4 / 6.7, M=5 13.6 /
 // 6.7, M=19 40 / 6.9, M=31 66 / 7.0; INT4 K=3072 N=1024 M=4 10.5 / 11.7, M=5
 // 16.5 / 11.7.  Pre-quantized rows skip the 2-4 us quantization launch.
-constexpr size_t GEMM_MIN_M_INT8 = 3, GEMM_MIN_M_INT4 = 5, GEMM_MIN_M_CODES = 3;
+// The register-streamed kernel (groups above 128, K off the LDS kernel's
+// stage) needs more rows the longer K is, two GEMV passes' worth for INT8 and
+// three for INT4: K=4096 N=2048, groups of 256, M=4 17.0 / 27.3 and M=8 33.6 /
+// 27.8 (INT8), M=8 24.5 / 30.8 and M=16 48.9 / 31.7 (INT4); K=1024 M=4 8.6 /
+// 10.2, M=5 13.9 / 10.3 (INT8), 11.8 / 11.1 (INT4).
+static bool mfma_pays(size_t M, size_t K, size_t gs, bool int4, bool scales4, bool codes) {
+    const bool lds = scales4 && (gs == 32 || gs == 64 || gs == 128) && K % (gs == 128 ? 256 : 128) == 0;
+    if (lds) return M >= (int4 && !codes ? 5 : 3);
+    return M >= (K <= 2048 ? 5 : int4 ? 13 : 8);
+}
 // Below this many rows the FP16 forms take the matrix cores only where the
 // stream's scratch, which they pass the codes on through, is theirs alone: a
 // captured graph outlives the call, and its stream's scratch with it may not,
@@ -617,8 +626,9 @@ int gemm_grouped_mfma(const uint16_t* A16, const int8_t* A8, const float* As, co
                       const uint16_t* Bs, uint16_t* C, size_t M, size_t K, size_t N, size_t gs,
                       bool int4, hipStream_t st, bool* handled, const uint16_t* R, void* ext_scratch) {
     *handled = false;
-    if (M < (A16 ? (int4 ? GEMM_MIN_M_INT4 : GEMM_MIN_M_INT8) : GEMM_MIN_M_CODES)) return CACTUS_HIP_OK;
-    if (gs % 32 != 0 || N < 32) return CACTUS_HIP_OK;
+    // the LDS path moves group scales as dwords
+    const bool scales4 = ((uintptr_t)Bs & 3) == 0;
+    if (gs % 32 != 0 || N < 32 || !mfma_pays(M, K, gs, int4, scales4, !A16)) return CACTUS_HIP_OK;
     if (((uintptr_t)B & 15) != 0) return CACTUS_HIP_OK;
     if (!A16 && (((uintptr_t)A8 & 15) != 0)) return CACTUS_HIP_OK;
     if (M >= (1u << 30) || N >= (1u << 30) || K >= (1u << 20)) return CACTUS_HIP_OK;
@@ -649,8 +659,6 @@ int gemm_grouped_mfma(const uint16_t* A16, const int8_t* A8, const float* As, co
         Asc = s;
     }
     GemmArgs a{Aq, Asc, B, Bs, C, (int)M, (int)K, (int)N, (int)gs, R};
-    // the LDS path moves group scales as dwords
-    const bool scales4 = ((uintptr_t)Bs & 3) == 0;
     if (scales4 && (int4 ? launch_lds_any<true>(a, st) : launch_lds_any<false>(a, st))) {
         *handled = true;
         return check_launch("grouped matmul (mfma, lds)");
@@ -677,7 +685,7 @@ int gemm_grouped_mfma_multi(const int8_t* A8, const float* As, int np, const uin
                             const uint16_t* const* Bs, uint16_t* const* C, const size_t* N, size_t M, size_t K,
                             size_t gs, bool int4, hipStream_t st, bool* handled) {
     *handled = false;
-    if (np < 1 || np > 3 || M < GEMM_MIN_M_CODES || gs % 32 != 0) return CACTUS_HIP_OK;
+    if (np < 1 || np > 3 || gs % 32 != 0 || !mfma_pays(M, K, gs, int4, true, true)) return CACTUS_HIP_OK;
     if (((uintptr_t)A8 & 15) != 0 || M >= (1u << 30) || K >= (1u << 20)) return CACTUS_HIP_OK;
     for (int p = 0; p < np; p++)
         if (N[p] < 32 || N[p] >= (1u << 30) || ((uintptr_t)B[p] & 15) != 0 || ((uintptr_t)Bs[p] & 3) != 0)

@@ -218,6 +218,14 @@ def test_matmul_few_rows(dev, orc, M, K, N, gs, int4):
     assert_bits(dev.get(C2, np.uint16, (M, N)), ref, "f16act")
 
 
+@pytest.mark.parametrize("int4", [False, True])
+@pytest.mark.parametrize("M,K,N,gs", [(4, 640, 64, 128), (5, 2048, 33, 256), (7, 3072, 64, 256), (8, 3072, 64, 256),
+                                      (12, 4096, 64, 1024), (13, 4096, 64, 1024)])
+def test_matmul_few_rows_wide_groups(dev, orc, M, K, N, gs, int4):
+    """The boundary where the LDS matrix kernel does not take the group size."""
+    test_matmul_few_rows(dev, orc, M, K, N, gs, int4)
+
+
 def test_matmul_few_rows_captured_cold(dev, orc):
     """Eight rows captured into a graph as the stream's first call: no device
     memory is taken inside the capture; every replay equals the oracle."""
