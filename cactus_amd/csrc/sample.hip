@@ -999,7 +999,10 @@ __global__ void __launch_bounds__(1024) entropy_kernel(const uint16_t* __restric
     if (tid == 0) *out = (float)(rd[0] / log((double)V));
 }
 
-// per-device scratch (grown) and token history (zeroed once)
+// per-device scratch (grown) and token history (zeroed once); a call holds
+// g_sample_mu until its last launch, so that the launches of another host
+// thread's call come before or behind all of its own, and a call that grows the
+// buffers finds every launch that reads them queued
 struct SampleState {
     uint16_t* f = nullptr;
     float* f32 = nullptr;
@@ -1014,10 +1017,10 @@ struct SampleState {
 static std::mutex g_sample_mu;
 static std::map<int, SampleState> g_sample;
 
-static int sample_state(size_t V, SampleState** out) {
+static int sample_state(size_t V, SampleState** out, std::unique_lock<std::mutex>& lk) {
     int dev = 0;
     CH_HIP(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lk(g_sample_mu);
+    lk = std::unique_lock<std::mutex>(g_sample_mu);
     SampleState& s = g_sample[dev];
     if (!s.hist) {
         CH_HIP(hipMalloc(&s.hist, (1 + SP_HIST) * sizeof(uint32_t)));
@@ -1069,7 +1072,8 @@ int cactus_hip_sample_f16(const uint16_t* logits, uint32_t* out, size_t vocab, f
     CH_REQUIRE(vocab < (1ull << 31), "sample: vocabulary too large");
     CH_REQUIRE(temperature >= 0.0f && temperature == temperature, "sample: temperature must be >= 0");
     SampleState* s = nullptr;
-    int rc = sample_state(vocab, &s);
+    std::unique_lock<std::mutex> lk;
+    int rc = sample_state(vocab, &s, lk);
     if (rc) return rc;
     // the reference's draw (kernel_nn.cpp:609-612): mt19937 seeded with the
     // 32-bit seed (a random one for seed 0), first output through libc++'s
@@ -1129,7 +1133,8 @@ int cactus_hip_sample_f32(const float* logits, uint32_t* out, size_t vocab, floa
     if (biased && bias_count > (size_t)SP_BIAS)
         return fail(CACTUS_HIP_EUNSUPPORTED, "sample_f32: at most 128 logit-bias entries");
     SampleState* s = nullptr;
-    int rc = sample_state(vocab, &s);
+    std::unique_lock<std::mutex> lk;
+    int rc = sample_state(vocab, &s, lk);
     if (rc) return rc;
     const uint32_t seed = random_seed ? (uint32_t)random_seed : std::random_device{}();
     std::mt19937 gen(seed);
@@ -1169,8 +1174,10 @@ int cactus_hip_logits_entropy_f16(const uint16_t* logits, size_t vocab, float* o
 int cactus_hip_sample_history(uint32_t* tokens, size_t* count, void* stream) {
     CH_REQUIRE(tokens && count, "sample_history: null argument");
     SampleState* s = nullptr;
-    int rc = sample_state(0, &s);
+    std::unique_lock<std::mutex> lk;
+    int rc = sample_state(0, &s, lk);
     if (rc) return rc;
+    lk.unlock();   // (the history stays where it is)
     uint32_t h[1 + SP_HIST];
     CH_HIP(hipMemcpyAsync(h, s->hist, sizeof(h), hipMemcpyDeviceToHost, as_stream(stream)));
     CH_HIP(hipStreamSynchronize(as_stream(stream)));
@@ -1181,7 +1188,8 @@ int cactus_hip_sample_history(uint32_t* tokens, size_t* count, void* stream) {
 
 int cactus_hip_sample_history_reset(void* stream) {
     SampleState* s = nullptr;
-    int rc = sample_state(0, &s);
+    std::unique_lock<std::mutex> lk;
+    int rc = sample_state(0, &s, lk);
     if (rc) return rc;
     return cactus_hip_memset(s->hist, 0, (1 + SP_HIST) * sizeof(uint32_t), stream);
 }

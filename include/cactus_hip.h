@@ -326,7 +326,9 @@ int cactus_hip_embedding_f16(const uint16_t* table, const float* ids, uint16_t* 
  * Top-p works with any top_k (0: the whole vocabulary); the reference's
  * unspecified order of tied values is taken as ascending token where a tie
  * straddles the top-p cut.  Always writes a token id < vocab (0 when every
- * logit is -inf) as one uint32 to *out (device memory), stream-ordered. */
+ * logit is -inf) as one uint32 to *out (device memory), stream-ordered.  The
+ * history and the working buffers belong to the device: calls of several host
+ * threads on one stream take turns, calls on streams that overlap race. */
 int cactus_hip_sample_f16(const uint16_t* logits, uint32_t* out, size_t vocab,
                           float temperature, float top_p, size_t top_k, size_t random_seed,
                           void* stream);

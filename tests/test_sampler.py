@@ -14,6 +14,7 @@ temperature / top-k / top-p mixes on 151936-entry and tied logits.
 """
 import ctypes
 import math
+import threading
 
 import numpy as np
 import pytest
@@ -219,6 +220,38 @@ def test_sampler_filtered_top_k(hip_ready, orc, vocab, cfg):
         assert rc == 0
         assert got == s.sample(x, *cfg, seed), step
     assert (history() == s.history()).all() and len(history()) == 128
+
+
+@pytest.mark.gpu
+def test_sampler_two_threads_one_stream(hip_ready):
+    """Two host threads sampling on the default stream from vocabularies of
+    their own: every token comes from the logits its call was given."""
+    cm = hip_ready
+    say("sampler two threads")
+    reps, live = 100, ((4096, 100), (151936, 140000))
+    rng = np.random.default_rng(5)
+    logits, out = [], []
+    for V, first in live:
+        x = rng.normal(0, 1, V)
+        x[first:first + 20] += 40.0
+        logits.append(cm.DeviceBuffer.from_numpy(f16(x)))
+        out.append(cm.DeviceBuffer(4 * reps))
+
+    def work(i):
+        for r in range(reps):
+            cm.call("cactus_hip_sample_f16", logits[i].ptr, out[i].ptr + 4 * r, live[i][0], ctypes.c_float(1.0),
+                    ctypes.c_float(0.9), 20, r + 1, None)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    cm.call("cactus_hip_stream_sync", None)
+    for i, (V, first) in enumerate(live):
+        tok = out[i].to_numpy(np.uint32, (reps,))
+        assert ((tok >= first) & (tok < first + 20)).all(), i
+    cm.call("cactus_hip_sample_history_reset", None)
 
 
 @pytest.mark.gpu
