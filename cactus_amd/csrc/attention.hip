@@ -1758,12 +1758,8 @@ __global__ void __launch_bounds__(RW_THREADS) attn_rows_kernel(AttnArgs a_in, in
         const int kd = kind(t);
         float pr[4][4];
         auto as_i8 = [&](int e) {
-            // (float)code * scale as fma(code + 128, scale, -128 scale): the
-            // exact product rounded once
-            const uint32_t u = r.lo[e] ^ 0x80808080u;
-            const float ns = -128.0f * r.sc[e];
 #pragma unroll
-            for (int c = 0; c < 4; c++) pr[e][c] = __builtin_fmaf((float)((u >> (8 * c)) & 0xFFu), r.sc[e], ns);
+            for (int c = 0; c < 4; c++) pr[e][c] = (float)(int8_t)((r.lo[e] >> (8 * c)) & 0xFFu) * r.sc[e];
         };
         auto as_f16 = [&](int e) {
             pr[e][0] = h2f((uint16_t)(r.lo[e] & 0xFFFF));

@@ -685,6 +685,34 @@ def _attention_hybrid(dev, orc, S, cache, new, Hq, Hkv, d, qmul):
     assert_bits(dev.get(o, np.uint16, q.shape), ref, "attention_hybrid")
 
 
+@pytest.mark.parametrize("S", [1, 40])
+def test_attention_hybrid_value_scales(dev, orc, S):
+    """Value scales beyond what a quantizer writes: infinite, overflowing
+    with larger codes, and negative (a zero code is then -0)."""
+    say("attention_hybrid value scales", S)
+    rng = np.random.default_rng(S)
+    cache, Hq, Hkv, d = 200, 8, 4, 64
+    kc = rng.integers(-127, 128, (1, cache, Hkv, d), dtype=np.int8)
+    vc = rng.integers(1, 128, (1, cache, Hkv, d), dtype=np.int8) * rng.choice(np.array([-1, 1], np.int8), (1, cache, Hkv, d))
+    ks = np.abs(rng.normal(0, 0.005, (cache, Hkv, 1))).astype(np.float32)
+    vs = np.abs(rng.normal(0, 0.02, (cache, Hkv, 1))).astype(np.float32)
+    vs[70, 0] = np.inf
+    vs[100, 1] = 2.0 ** 121
+    vs[130:140, 2] *= -1
+    vs[:, 3] = -1e-3
+    vc[:, :, 3] = 0
+    kn, vn = (f16(rng.normal(0, 1, (1, S, Hkv, d))) for _ in range(2))
+    vn[:, :, 3] = 0x8000
+    q = f16(rng.normal(0, 1, (1, S, Hq, d)))
+    scale = 1.0 / math.sqrt(d)
+    ref = orc.attention_hybrid(q, kc, vc, ks[None], vs[None], kn, vn, scale, pos_off=cache)
+    o = dev.empty(q.nbytes)
+    dev.cm.call("cactus_hip_attention_hybrid_int8_fp16", dev.put(q), dev.put(kc), dev.put(vc), dev.put(ks), dev.put(vs),
+                dev.put(kn), dev.put(vn), o.ptr, 1, S, cache, S, Hq, Hkv, d, ctypes.c_float(scale), cache, 1, 128, None)
+    assert np.isinf(ref[0, :, :2].view(np.float16)).all()
+    assert_bits(dev.get(o, np.uint16, q.shape), ref, "attention_hybrid value scales")
+
+
 def test_attention_hybrid_batch2(dev, orc):
     """Two batch rows: the codes are per batch row, the scale tables are the
     first row's for both (kernel_attention.cpp:353,424 index them without
