@@ -713,7 +713,8 @@ __global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in,
     const size_t b = gy / ngrp;
     const int h0 = kvh * gq;
     // kv_range of a row on this path (no window, at most 32768 keys, so ints)
-    const int pos = (int)(a.pos_off < (1u << 30) ? a.pos_off : (1u << 30)), Skv = (int)a.Skv;
+    // (positions from 2^30 on see every key, as 2^30 does)
+    const int pos = (int)(a.pos_off < (1u << 30) ? a.pos_off : (1u << 30)), Skv = (int)(a.Skv < (1u << 30) ? a.Skv : (1u << 30));
     auto row_end = [&](int qp, int& limit) {
         const int e = a.causal ? min(pos + qp + 1, Skv) : Skv;
         limit = HYBRID ? e : Skv;
@@ -849,7 +850,7 @@ __global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in,
                     const bool block_live = bs0 < kv_end;
                     const int bsz = block_live ? min(ATT_BLOCK, blk_limit - bs0) : 0;
                     wlane[r] = jl < bsz;
-                    const int aq = (int)a.pos_off + qp;
+                    const int aq = pos + qp;
                     const bool is_decode = qp == a.S - 1 && a.S > 1;
                     bool ok = wlane[r] && !(a.causal && (kp > aq || (!is_decode && bs0 > aq)));
                     if (a.mask && ok) ok = h2f(a.mask[(b * a.S + qp) * a.Skv + kp]) != 0.0f;
@@ -892,7 +893,7 @@ __global__ void __launch_bounds__(256, 2) attn_scores_mfma_kernel(AttnArgs a_in,
             if (bs < kv_end) {
                 const int bsz = min(ATT_BLOCK, blk_limit - bs);
                 const bool is_decode = (!HYBRID) && (qp == a.S - 1) && a.S > 1;
-                const bool block_skipped = !HYBRID && !is_decode && a.causal && bs > (int)a.pos_off + qp;
+                const bool block_skipped = !HYBRID && !is_decode && a.causal && bs > pos + qp;
                 // the rows kernel never takes the keys past a row's causal end,
                 // so their zero weights need no flag there
                 const int zsz = rows_follow ? min(bsz, kv_end - bs) : bsz;

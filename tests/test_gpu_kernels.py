@@ -618,6 +618,21 @@ def test_attention_f16_unaligned_values(dev, orc):
     assert_bits(dev.get(o, np.uint16, q.shape), ref, "attention_f16 unaligned")
 
 
+@pytest.mark.parametrize("pos", [2**31 - 3, 2**31, 2**32 + 5])
+def test_attention_f16_far_position(dev, orc, pos):
+    """Rows at positions around and past 2^31: every key is visible."""
+    say("attention_f16 far position", pos)
+    rng = np.random.default_rng(31)
+    B, S, Skv, Hq, Hkv, d = 1, 12, 150, 4, 2, 64
+    q, k, v = _attn_inputs(rng, B, S, Skv, Hq, Hkv, d)
+    scale = 1.0 / math.sqrt(d)
+    ref = orc.attention_f16(q, k, v, scale, pos_off=Skv)
+    o = dev.empty(q.nbytes)
+    dev.cm.call("cactus_hip_attention_f16", dev.put(q), dev.put(k), dev.put(v), o.ptr, B, S, Skv, Hq, Hkv, d,
+                ctypes.c_float(scale), None, pos, 0, 1, None)
+    assert_bits(dev.get(o, np.uint16, q.shape), ref, "attention_f16 far position")
+
+
 def test_attention_f16_mask_noncausal(dev, orc):
     say("attention_f16 mask, non-causal")
     rng = np.random.default_rng(7)
