@@ -2059,11 +2059,13 @@ static int launch_attention(AttnArgs a, void* stream) {
             a.cache_len > 0 && bytes <= TILES_MAX_BYTES &&
             stream_scratch_ready(SCR_ATTN_TILES, stream, bytes)) {
             void* p = nullptr;
-            rc = stream_scratch(SCR_ATTN_TILES, stream, bytes, false, &p);
-            if (rc) return rc;
-            a.vsh = static_cast<const float*>(p);
-            a.sh_ntile = nt;
-            tiles = true;
+            if (stream_scratch(SCR_ATTN_TILES, stream, bytes, false, &p) == CACTUS_HIP_OK) {
+                a.vsh = static_cast<const float*>(p);
+                a.sh_ntile = nt;
+                tiles = true;
+            } else {
+                (void)hipGetLastError();   // no memory to be had: the chains convert the cache themselves
+            }
         }
     }
     const bool windowed = !HYBRID && a.window > 0 && a.window < a.Skv;

@@ -728,6 +728,46 @@ def test_attention_hybrid_value_scales(dev, orc, S):
     assert_bits(dev.get(o, np.uint16, q.shape), ref, "attention_hybrid value scales")
 
 
+def test_attention_hybrid_decode_without_tile_memory(dev, orc):
+    """A decode call that cannot get the memory of its value product tiles
+    runs without them.  Memory is refused by a capture on another stream,
+    whose mode forbids allocations everywhere; the call's stream has the
+    weights' scratch from a prefill call, and none for tiles."""
+    say("attention_hybrid decode, no tile memory")
+    rng = np.random.default_rng(77)
+    cache, Hq, Hkv, d = 300, 4, 2, 128
+    kf, vf = (f16(rng.normal(0, 1, (cache, Hkv, d))) for _ in range(2))
+    (kc, ks), (vc, vs) = orc.quantize_kv(kf), orc.quantize_kv(vf)
+    kn, vn, q = (f16(rng.normal(0, 1, (1, 8, h, d))) for h in (Hkv, Hkv, Hq))
+    scale = 1.0 / math.sqrt(d)
+    st, cap = dev.cm.Stream(), dev.cm.Stream()
+    c = [dev.put(a) for a in (kc, vc, ks, vs)]
+    o = dev.empty(q.nbytes)
+
+    def run(S):
+        dev.cm.call("cactus_hip_attention_hybrid_int8_fp16", qp, *c, knp, vnp, o.ptr, 1, S, cache, S, Hq, Hkv, d,
+                    ctypes.c_float(scale), cache, 1, 128, st.handle)
+
+    qp, knp, vnp = (dev.put(a) for a in (q, kn, vn))
+    run(8)
+    st.sync()
+    hip = dev.cm.hip()   # (symbols of the HIP runtime it is linked to)
+    hip.hipStreamBeginCapture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    hip.hipGraphDestroy.argtypes = [ctypes.c_void_p]
+    graph = ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(cap.handle, 0) == 0   # hipStreamCaptureModeGlobal
+    try:
+        run(1)
+    finally:
+        if hip.hipStreamEndCapture(cap.handle, ctypes.byref(graph)) == 0:
+            hip.hipGraphDestroy(graph)
+        hip.hipGetLastError()
+    st.sync()
+    ref = orc.attention_hybrid(q[:, :1], kc[None], vc[None], ks[None], vs[None], kn[:, :1], vn[:, :1], scale, pos_off=cache)
+    assert_bits(dev.get_ptr(o.ptr, np.uint16, ref.shape), ref, "attention_hybrid decode")
+
+
 def test_attention_hybrid_batch2(dev, orc):
     """Two batch rows: the codes are per batch row, the scale tables are the
     first row's for both (kernel_attention.cpp:353,424 index them without
