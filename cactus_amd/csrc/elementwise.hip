@@ -408,20 +408,20 @@ int cactus_hip_softmax_f16(const uint16_t* x, uint16_t* y, size_t batch, size_t 
 int cactus_hip_silu_f16(const uint16_t* x, uint16_t* y, size_t n, void* stream) {
     if (n == 0) return CACTUS_HIP_OK;
     CH_REQUIRE(x && y, "silu: null pointer");
-    return launch_pointwise<false>("silu", x, nullptr, y, n, stream, SiluOp{});
+    return launch_pointwise<SiluOp, false>("silu", x, nullptr, y, n, stream);
 }
 
 int cactus_hip_add_f16(const uint16_t* a, const uint16_t* b, uint16_t* y, size_t n, void* stream) {
     if (n == 0) return CACTUS_HIP_OK;
     CH_REQUIRE(a && b && y, "add: null pointer");
-    return launch_pointwise<true>("add", a, b, y, n, stream, AddOp{});
+    return launch_pointwise<AddOp, true>("add", a, b, y, n, stream);
 }
 
 int cactus_hip_multiply_f16(const uint16_t* a, const uint16_t* b, uint16_t* y, size_t n,
                             void* stream) {
     if (n == 0) return CACTUS_HIP_OK;
     CH_REQUIRE(a && b && y, "multiply: null pointer");
-    return launch_pointwise<true>("multiply", a, b, y, n, stream, MulOp{});
+    return launch_pointwise<MulOp, true>("multiply", a, b, y, n, stream);
 }
 
 int cactus_hip_transpose_2d_f16(const uint16_t* src, uint16_t* dst, size_t rows, size_t cols,

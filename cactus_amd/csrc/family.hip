@@ -299,13 +299,13 @@ extern "C" {
 int cactus_hip_gelu_f16(const uint16_t* in, uint16_t* out, size_t n, void* stream) {
     if (n == 0) return CACTUS_HIP_OK;
     CH_REQUIRE(in && out, "gelu: null pointer");
-    return launch_pointwise<false>("gelu", in, nullptr, out, n, stream, GeluOp{});
+    return launch_pointwise<GeluOp, false>("gelu", in, nullptr, out, n, stream);
 }
 
 int cactus_hip_gelu_erf_f16(const uint16_t* in, uint16_t* out, size_t n, void* stream) {
     if (n == 0) return CACTUS_HIP_OK;
     CH_REQUIRE(in && out, "gelu_erf: null pointer");
-    return launch_pointwise<false>("gelu_erf", in, nullptr, out, n, stream, GeluErfOp{});
+    return launch_pointwise<GeluErfOp, false>("gelu_erf", in, nullptr, out, n, stream);
 }
 
 int cactus_hip_layer_norm_f16(const uint16_t* x, const uint16_t* weight, const uint16_t* bias, uint16_t* y,

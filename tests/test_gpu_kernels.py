@@ -412,6 +412,24 @@ def test_pointwise_edges(dev, orc, n, off):
         assert got[off + n] == 0
 
 
+@pytest.mark.parametrize("n,off", [((1 << 19) - 3, 0), ((1 << 19) + 5, 0), ((1 << 19) + 5, 2), ((1 << 19) + 5, 1), (4099, 2)])
+def test_pointwise_widths(dev, orc, n, off):
+    """The five pointwise ops on both sides of the size from which a thread
+    takes eight values, at 16-, 4- and 2-byte aligned addresses."""
+    say("pointwise widths", n, off)
+    rng = np.random.default_rng(n + off)
+    a, b = (f16(rng.normal(0, 2, n)) for _ in range(2))
+    pad = np.zeros(off, np.uint16)
+    pa, pb = dev.put(np.concatenate([pad, a])) + 2 * off, dev.put(np.concatenate([pad, b])) + 2 * off
+    out = dev.put(np.zeros(n + off + 1, np.uint16))
+    for name, args, want in (("add", (pa, pb), orc.add(a, b)), ("multiply", (pa, pb), orc.multiply(a, b)),
+                             ("silu", (pa,), orc.silu(a)), ("gelu", (pa,), orc.gelu(a)), ("gelu_erf", (pa,), orc.gelu_erf(a))):
+        dev.cm.call("cactus_hip_%s_f16" % name, *args, out + 2 * off, n, None)
+        got = dev.get_ptr(out, np.uint16, n + off + 1)
+        assert_bits(got[off:off + n], want, name)
+        assert got[off + n] == 0
+
+
 @pytest.mark.parametrize("rows,dims,off", [(1, 8, 0), (5, 24, 0), (3, 2056, 0), (2, 8192, 0), (4, 129, 0), (3, 1024, 1)])
 def test_rms_norm_edges(dev, orc, rows, dims, off):
     say("rms_norm edges", rows, dims, off)
