@@ -2046,28 +2046,6 @@ static int launch_attention(AttnArgs a, void* stream) {
     a.bmax = reinterpret_cast<float*>(static_cast<char*>(scratch) + wbytes);
     a.bsum = a.bmax + rows * a.nbstride;
     const size_t chunks = (maxr + 63) / 64;
-    // a decode call over an INT8 cache without product tiles: built in
-    // scratch, which the streamed chains more than pay for at every length
-    // (us per call, 16 / 8 heads of 128 dims: 64 keys 14.6 -> 10.9, 520 17.6
-    // -> 13.2, 4096 50.2 -> 33.3)
-    bool tiles = false;
-    if constexpr (HYBRID) {
-        const size_t nt = (a.cache_len + a.new_len + SH_TILE_KEYS - 1) / SH_TILE_KEYS;
-        const size_t bytes = (size_t)a.Hkv * ((a.d + 63) / 64) * nt * SH_TILE_FLOATS * sizeof(float);
-        if (!a.vsh && !a.dyn && a.B == 1 && a.S <= 2 && a.new_len <= 2 && a.d % 8 == 0 &&
-            (a.qgs % 64 == 0 || a.qgs >= a.d) && (uintptr_t)a.vc % 4 == 0 && (uintptr_t)a.vs % 4 == 0 &&
-            a.cache_len > 0 && bytes <= TILES_MAX_BYTES &&
-            stream_scratch_ready(SCR_ATTN_TILES, stream, bytes)) {
-            void* p = nullptr;
-            if (stream_scratch(SCR_ATTN_TILES, stream, bytes, false, &p) == CACTUS_HIP_OK) {
-                a.vsh = static_cast<const float*>(p);
-                a.sh_ntile = nt;
-                tiles = true;
-            } else {
-                (void)hipGetLastError();   // no memory to be had: the chains convert the cache themselves
-            }
-        }
-    }
     const bool windowed = !HYBRID && a.window > 0 && a.window < a.Skv;
     // the values of prefill rows run in the many-rows kernel
     bool rows_follow = !windowed && (size_t)a.B * a.S > 2 && a.gq <= ATT_MAX_GQ && RW_CH % a.gq == 0 && a.d % 4 == 0 &&
@@ -2089,6 +2067,34 @@ static int launch_attention(AttnArgs a, void* stream) {
     const bool k16 = HYBRID ? ((uintptr_t)a.kc % 16 == 0 && (uintptr_t)a.ks % 4 == 0 && a.qgs % 16 == 0) : true;
     const bool rows_ok = chunks > 0 && !windowed && (a.d == 64 || a.d == 128) && a.gq <= ATT_MAX_GQ &&
                          ATT_MAX_GQ % a.gq == 0 && k16 && (uintptr_t)a.k % 16 == 0;
+    // a decode call over an INT8 cache without product tiles: built in
+    // scratch.  Beside the scores of the row kernel the streamed chains more
+    // than pay for them at every length (us per call, 16 / 8 heads of 128
+    // dims: 64 keys 14.6 -> 10.9, 520 17.6 -> 13.2, 4096 50.2 -> 33.3).  In
+    // other head dims they take a launch of their own, which two rows or eight
+    // heads per KV head always pay for, fewer from some length on (one row, 8 /
+    // 8 heads: 72 dims 65 keys 11.1 -> 12.7, 1000 22.2 -> 21.8, 4096 50.6 ->
+    // 42.0; 256 dims 1000 28.4 -> 30.3, 4096 55.3 -> 55.9; 16 / 4 heads of 72
+    // dims 65 keys 16.8 -> 17.3, 300 22.6 -> 21.5)
+    bool tiles = false;
+    if constexpr (HYBRID) {
+        const size_t nt = (a.cache_len + a.new_len + SH_TILE_KEYS - 1) / SH_TILE_KEYS;
+        const size_t bytes = (size_t)a.Hkv * ((a.d + 63) / 64) * nt * SH_TILE_FLOATS * sizeof(float);
+        const bool pays = rows_ok || a.S == 2 || a.gq == 8 || a.cache_len >= (a.gq >= 4 ? 256u : a.d <= 128 ? 512u : 2048u);
+        if (pays && !a.vsh && !a.dyn && a.B == 1 && a.S <= 2 && a.new_len <= 2 && a.d % 8 == 0 &&
+            (a.qgs % 64 == 0 || a.qgs >= a.d) && (uintptr_t)a.vc % 4 == 0 && (uintptr_t)a.vs % 4 == 0 &&
+            a.cache_len > 0 && bytes <= TILES_MAX_BYTES &&
+            stream_scratch_ready(SCR_ATTN_TILES, stream, bytes)) {
+            void* p = nullptr;
+            if (stream_scratch(SCR_ATTN_TILES, stream, bytes, false, &p) == CACTUS_HIP_OK) {
+                a.vsh = static_cast<const float*>(p);
+                a.sh_ntile = nt;
+                tiles = true;
+            } else {
+                (void)hipGetLastError();   // no memory to be had: the chains convert the cache themselves
+            }
+        }
+    }
     CH_REQUIRE(!a.prep.q_raw || (rows_ok && (size_t)a.B * a.S <= 2 && (a.gq == 1 || a.gq == 2)),
                "decode attention with fused head preparation: needs head_dim 64 or 128, 1 or 2 query heads "
                "per KV head and 16-byte aligned rows");

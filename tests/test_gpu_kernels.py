@@ -786,6 +786,13 @@ def test_attention_hybrid_decode_without_tile_memory(dev, orc):
     assert_bits(dev.get_ptr(o.ptr, np.uint16, ref.shape), ref, "attention_hybrid decode")
 
 
+@pytest.mark.parametrize("S,cache,Hq,Hkv,d", [(1, 600, 2, 1, 72), (1, 300, 8, 2, 72), (1, 2100, 2, 2, 256)])
+def test_attention_hybrid_tile_launch(dev, orc, S, cache, Hq, Hkv, d):
+    """Product tiles built by a launch of their own: head dims that the row
+    kernel does not take, from the lengths that pay for it."""
+    _attention_hybrid(dev, orc, S, cache, S, Hq, Hkv, d, 1.0)
+
+
 def test_attention_hybrid_batch2(dev, orc):
     """Two batch rows: the codes are per batch row, the scale tables are the
     first row's for both (kernel_attention.cpp:353,424 index them without
