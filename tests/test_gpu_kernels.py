@@ -302,6 +302,32 @@ def test_matmul_few_rows_captured_warm(dev, orc, entry, M):
     dev.cm.call("cactus_hip_graph_destroy", g.value)
 
 
+def test_matmul_few_rows_without_memory(dev, orc):
+    """Few rows on a stream that has no scratch and can get none (a capture on
+    another stream whose mode forbids allocations everywhere): the GEMV."""
+    say("matmul few rows, no memory")
+    M, K, N, gs = 8, 1024, 512, 32
+    rng = np.random.default_rng(9)
+    x = activations(rng, M, K)
+    B, Bs = grouped_int8_weights(rng, N, K, gs)
+    xp, Bp, Bsp, C = dev.put(x), dev.put(B), dev.put(Bs), dev.empty(M * N * 2)
+    st, cap = dev.cm.Stream(), dev.cm.Stream()
+    hip = dev.cm.hip()   # (symbols of the HIP runtime it is linked to)
+    hip.hipStreamBeginCapture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    hip.hipGraphDestroy.argtypes = [ctypes.c_void_p]
+    graph = ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(cap.handle, 0) == 0   # hipStreamCaptureModeGlobal
+    try:
+        dev.cm.call("cactus_hip_matmul_int8_f16act", xp, Bp, Bsp, C.ptr, M, K, N, gs, st.handle)
+    finally:
+        if hip.hipStreamEndCapture(cap.handle, ctypes.byref(graph)) == 0:
+            hip.hipGraphDestroy(graph)
+        hip.hipGetLastError()
+    st.sync()
+    assert_bits(dev.get_ptr(C.ptr, np.uint16, (M, N)), orc.matmul_int8(*orc.quantize_activations(x), B, Bs, gs), "GEMV")
+
+
 @pytest.mark.parametrize("M", [8, 40])
 def test_matmul_two_threads_one_stream(dev, orc, M):
     """Two host threads with rows of their own on the default stream: every
@@ -791,6 +817,62 @@ def test_attention_hybrid_tile_launch(dev, orc, S, cache, Hq, Hkv, d):
     """Product tiles built by a launch of their own: head dims that the row
     kernel does not take, from the lengths that pay for it."""
     _attention_hybrid(dev, orc, S, cache, S, Hq, Hkv, d, 1.0)
+
+
+@pytest.mark.parametrize("S", [1, 40])
+@pytest.mark.parametrize("what", ["weights", "keys"])
+def test_attention_hybrid_denormals(dev, orc, S, what):
+    """Denormal operands of the score and value chains (the matrix
+    instruction of the prefill rows takes and rounds them as fmaf does).
+    Weights e^-86 .. e^-106, some of them zero, on values near 2^124; or
+    keys near 2^-130 under a scale that brings the scores back to about 1."""
+    say("attention_hybrid denormals", S, what)
+    rng = np.random.default_rng(S)
+    cache, Hq, Hkv, d = 330, 4, 2, 64
+    vc = rng.integers(-127, 128, (1, cache, Hkv, d), dtype=np.int8)
+    if what == "weights":
+        scale = 1.0
+        q = np.zeros((1, S, Hq, d), np.float32)
+        q[..., 0] = 1.0
+        kc = np.zeros((1, cache, Hkv, d), np.int8)
+        kc[..., 0] = -100
+        ks = (rng.uniform(86, 106, (cache, Hkv, 1)) / 100).astype(np.float32)
+        kc[:, ::32] = 0                                     # the block's largest score is 0 ...
+        vc[:, ::32] = 0                                     # ... and its value too
+        vs = np.full((cache, Hkv, 1), 2.0 ** 118, np.float32)
+        kn = vn = np.zeros((1, S, Hkv, d), np.float32)
+    else:
+        scale = 2.0 ** 126
+        q = rng.normal(0, 1, (1, S, Hq, d))
+        kc = rng.integers(-127, 128, (1, cache, Hkv, d), dtype=np.int8)
+        ks = np.full((cache, Hkv, 1), 2.0 ** -135, np.float32)
+        vs = np.full((cache, Hkv, 1), 0.01, np.float32)
+        kn, vn = np.zeros((1, S, Hkv, d)), rng.normal(0, 1, (1, S, Hkv, d))
+    q, kn, vn = f16(q), f16(kn), f16(vn)
+    ref = orc.attention_hybrid(q, kc, vc, ks[None], vs[None], kn, vn, scale, pos_off=cache)
+    x = ref.view(np.float16).astype(np.float64)
+    assert np.isfinite(x).all() and np.abs(x).max() > 1e-3 and len(np.unique(ref)) > 100
+    o = dev.empty(q.nbytes)
+    dev.cm.call("cactus_hip_attention_hybrid_int8_fp16", dev.put(q), dev.put(kc), dev.put(vc), dev.put(ks), dev.put(vs),
+                dev.put(kn), dev.put(vn), o.ptr, 1, S, cache, S, Hq, Hkv, d, ctypes.c_float(scale), cache, 1, 128, None)
+    assert_bits(dev.get(o, np.uint16, q.shape), ref, "attention_hybrid denormals")
+
+
+@pytest.mark.parametrize("S,d,gs", [(40, 128, 32), (40, 64, 16), (3, 128, 64), (1, 128, 32)])
+def test_attention_hybrid_narrow_groups(dev, orc, S, d, gs):
+    """Several scales per cached key row."""
+    say("attention_hybrid narrow groups", S, d, gs)
+    rng = np.random.default_rng(gs + d)
+    cache, Hq, Hkv = 210, 8, 4
+    (kc, ks), (vc, vs) = (orc.quantize_kv(f16(rng.normal(0, 1, (cache, Hkv, d)) * rng.uniform(0.2, 3, (cache, Hkv, d))), gs)
+                          for _ in range(2))
+    kn, vn, q = (f16(rng.normal(0, 1, (1, S, h, d))) for h in (Hkv, Hkv, Hq))
+    scale = 1.0 / math.sqrt(d)
+    ref = orc.attention_hybrid(q, kc[None], vc[None], ks[None], vs[None], kn, vn, scale, pos_off=cache, qgs=gs)
+    o = dev.empty(q.nbytes)
+    dev.cm.call("cactus_hip_attention_hybrid_int8_fp16", dev.put(q), dev.put(kc), dev.put(vc), dev.put(ks), dev.put(vs),
+                dev.put(kn), dev.put(vn), o.ptr, 1, S, cache, S, Hq, Hkv, d, ctypes.c_float(scale), cache, 1, gs, None)
+    assert_bits(dev.get(o, np.uint16, q.shape), ref, "attention_hybrid narrow groups")
 
 
 def test_attention_hybrid_batch2(dev, orc):
