@@ -1318,15 +1318,17 @@ int attention_prefill_fast(const uint16_t* q, const int8_t* kc, const int8_t* vc
         return n;
     };
     // Eight waves per staged tile (half the staging per wave, but one
-    // workgroup per CU) where a tile's staging is large (128 dims), the start
-    // of a workgroup is spread over several tiles and its rounds of the 256
-    // CUs are nearly full (us, four / eight waves, 16 / 8 heads of 128 dims:
-    // 333 rows at 3000 keys 35.4 / 34.9, 512 at 4096 49.4 / 47.5; four tiles a
-    // split, 256 at 2048, 29.1 / 29.5; half a round, 512 over themselves,
-    // 18.7 / 22.3; 512 at 4096 with 64 dims, 8 / 8 heads, 23.5 / 26.4).
+    // workgroup per CU) where a tile's staging is large (128 dims), at least
+    // six blocks share a KV head, the start of a workgroup is spread over
+    // several tiles and its rounds of the 256 CUs are nearly full (us, four /
+    // eight waves, 16 / 8 heads of 128 dims: 333 rows at 3000 keys 35.2 / 34.7,
+    // 512 at 2048 33.5 / 32.9 and at 4096 49.4 / 47.5; four blocks, 256 rows at
+    // 3072 30.5 / 31.6; four tiles a split, 512 at 1024 25.6 / 26.9; half a
+    // round, 512 over themselves, 18.7 / 22.3; 64 dims, 512 at 4096, 8 / 8
+    // heads 23.5 / 26.4).
     int W = 8;
     size_t wgs = set_blocks(16 * 8 * VB);
-    if (d != 128 || a.tps < 6 || wgs * 8 < (wgs + 255) / 256 * 256 * 7) {
+    if (d != 128 || S * gq <= 5 * PF_BV || a.tps < 6 || wgs * 8 < (wgs + 255) / 256 * 256 * 7) {
         W = 4;
         wgs = set_blocks(16 * 4 * VB);
     }
