@@ -794,7 +794,7 @@ __device__ __forceinline__ float max3f(float a, float b, float c) {
     return r;
 }
 
-// Bound by vector instructions (softmax, INT8-to-FP16 staging: ~250 per wave
+// Bound by vector instructions (softmax, INT8-to-FP16 staging: ~320 per wave
 // and tile against 32 MFMAs) and by the partials, written and read once.
 // What brought 333 rows at 3000 keys, 16 / 8 heads, 49.4 -> 34.9 us, every
 // rounding as before: two waves per SIMD (it held 304 registers: one), tile
@@ -1391,8 +1391,9 @@ int cactus_hip_attention_hybrid_int8_fp16_fast(const uint16_t* q, const int8_t* 
                                                void* stream) {
     if (batch == 0 || seq_len == 0 || num_q_heads == 0 || head_dim == 0) return CACTUS_HIP_OK;
     const bool aligned16 = ((uintptr_t)k_cached & 15) == 0 && ((uintptr_t)v_cached & 15) == 0;
+    const bool keys = cache_len + new_len > 0;   // none: zero rows, by the exact kernels
     // prefill rows: flash attention on FP16 MFMA
-    const bool prefill = seq_len > 1 && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && is_causal &&
+    const bool prefill = keys && seq_len > 1 && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && is_causal &&
                          fast_prefill_supported(head_dim, num_q_heads / num_kv_heads) &&
                          quant_group_size >= head_dim && batch * num_kv_heads < 65536 && aligned16 &&
                          ((uintptr_t)q & 15) == 0 && ((uintptr_t)k_new & 15) == 0 && ((uintptr_t)v_new & 15) == 0 &&
@@ -1407,7 +1408,7 @@ int cactus_hip_attention_hybrid_int8_fp16_fast(const uint16_t* q, const int8_t* 
                                       cache_len, new_len, num_q_heads, num_kv_heads, head_dim, scale,
                                       position_offset, quant_group_size, stream);
     }
-    const bool fast = num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && is_causal &&
+    const bool fast = keys && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && is_causal &&
                       fast_attention_supported(seq_len, head_dim, num_q_heads / num_kv_heads, nullptr) &&
                       quant_group_size >= head_dim && batch * num_kv_heads < 65536 &&
                       cache_len + new_len <= FA_MAX_KEYS_HYBRID && aligned16;

@@ -266,6 +266,17 @@ def test_attention_hybrid_prefill_fast(dev, orc, B, cache, new, Hq, Hkv, d, qmul
     print(f"[prefill fast] max abs error {err:.2e}", flush=True)
 
 
+def test_attention_hybrid_fast_without_keys(dev):
+    """No cached and no new keys: zero rows, as from the exact entry point."""
+    say("attention_hybrid_fast, no keys")
+    for S in (1, 5):
+        q = f16(np.random.default_rng(S).normal(0, 1, (1, S, 4, 64)))
+        o = dev.put(np.full(q.shape, 0x7E01, np.uint16))
+        dev.cm.call("cactus_hip_attention_hybrid_int8_fp16_fast", dev.put(q), None, None, None, None, None, None, o, 1, S,
+                    0, 0, 4, 2, 64, ctypes.c_float(0.125), 0, 1, 128, None)
+        assert (dev.get_ptr(o, np.uint16, q.shape) == 0).all()
+
+
 @pytest.mark.parametrize("S,T,Hq,Hkv,d,digest", [
     (333, 3000, 16, 8, 128, "ea278d1ad75ae9f9"), (512, 3000, 8, 2, 128, "d9ad33f4081e79c5"),   # eight waves per tile
     (130, 500, 16, 4, 64, "bb1c32ea27e7e56f"), (37, 517, 2, 2, 128, "3a9d1f1fd9dffa24"),
