@@ -273,12 +273,11 @@ static unsigned value_tile_wgs(const AttnArgs& a) {
 __global__ void __launch_bounds__(64) value_tiles_kernel(AttnArgs a) { value_tile_wg(a, blockIdx.x); }
 
 // ------------------------------------------------ kernel A, decode row
-// One query row of up to two heads per kv head: a one-wave workgroup per 64
-// keys and query head.  A lane owns one key, whose whole INT8 row is loaded
-// before the query, so the two memory round trips overlap.  The query vector
-// enters the FMA through DPP row_newbcast from a register that holds 16 of
-// its dims replicated over the four 16-lane rows, so a score step is one VALU
-// op.  The reference's per-score order is kept: accumulator c takes dims
+// Decode rows: a one-wave workgroup per 64 keys, query row and query head.  A
+// lane owns one key, whose whole INT8 row is loaded before the query, so the
+// two memory round trips overlap.  The query vector enters the FMA through DPP
+// row_newbcast from a register that holds 16 of its dims replicated over the
+// four 16-lane rows, so a score step is one VALU op.  The reference's per-score order is kept: accumulator c takes dims
 // 8i+c in increasing i, then ((c0+c4)+(c1+c5)) + ((c2+c6)+(c3+c7)), times
 // scale.  The INT8 key value (float)code * scale is formed as
 // fma((float)(code + 128), scale, -128 * scale): the exact product rounded
@@ -671,8 +670,8 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
 // ------------------------------------------------ kernel A, prefill rows
 // A score is eight fp32 FMA chains in a fixed order, and
 // v_mfma_f32_4x4x1_16b_f32 is a chain step: every output takes one product,
-// fused and rounded once as fmaf (compared bit for bit on the device over
-// normal, denormal and infinite operands).  With lane = key as operand B
+// fused and rounded once as fmaf, denormal operands included (the tests hold
+// it to the oracle bit for bit).  With lane = key as operand B
 // and four query vectors as operand A -- one register holds 16 dims x 4
 // vectors, the dim picked by the instruction's A-block broadcast -- an
 // instruction advances 256 chains in 8 cycles, against 64 in ~4.5 for a
@@ -2050,7 +2049,8 @@ static int launch_attention(AttnArgs a, void* stream) {
     // the values of prefill rows run in the many-rows kernel
     bool rows_follow = !windowed && (size_t)a.B * a.S > 2 && a.gq <= ATT_MAX_GQ && RW_CH % a.gq == 0 && a.d % 4 == 0 &&
                        (HYBRID ? (uintptr_t)a.vc % 4 == 0 && (uintptr_t)a.vs % 4 == 0 : true) &&
-                       (uintptr_t)a.v % 8 == 0 && rows_smem(a.nbstride) <= 160 * 1024;
+                       (uintptr_t)a.v % 8 == 0 && rows_smem(a.nbstride) <= 160 * 1024 &&
+                       (size_t)RW_CH * a.Hkv * a.wstride < (1ull << 32);   // its 32-bit weight offsets
     if (rows_follow) {
         static hipError_t attr[2] = {
             hipFuncSetAttribute((const void*)attn_rows_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -2119,7 +2119,7 @@ static int launch_attention(AttnArgs a, void* stream) {
         rc = check_launch("attention scores (rows)");
         if (rc) return rc;
     } else if (rows_ok) {
-        // decode: one query row, its gq heads per wave, one wave per 64 keys
+        // decode: one wave per 64 keys, query row and query head
         // (with the fused head preparation, one more workgroup per kv head
         // appends the step's key and value)
         // workgroups of kv head h on XCD h % 8, where the chain kernel's are;

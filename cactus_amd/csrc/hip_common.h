@@ -164,11 +164,12 @@ __device__ __forceinline__ float exp2_bits(int32_t zi) {
     return bits_f((uint32_t)((uint32_t)zi + 127u) << 23);
 }
 
-// expf used wherever the reference calls libm expf: x = k*ln2 + r (Cody-Waite,
-// two-part ln2), e^r by its degree-12 Taylor polynomial in double (Horner,
-// fused), one rounding to float.  Relative error of the double result is a
-// few 1e-16, so the float result is the correctly rounded e^x except when
-// e^x lies within ~1e-15 (relative) of a float rounding boundary.
+// expf used wherever the reference calls libm expf: x = k*ln2 + r (Cody and
+// Waite, Software Manual for the Elementary Functions, 1980; ln 2 in the two
+// parts of Sun's fdlibm, e_exp.c), e^r by its degree-12 Taylor polynomial in
+// double (Horner, fused), one rounding to float.  Relative error of the double
+// result is a few 1e-16, so the float result is the correctly rounded e^x except
+// when e^x lies within ~1e-15 (relative) of a float rounding boundary.
 // Branch-free, so that independent calls interleave: beyond the clamps e^x
 // rounds to 0 or overflows to infinity by itself, and 2^k is applied by
 // v_ldexp_f64 (exact: the double stays normal).  The polynomial's constants
