@@ -110,9 +110,9 @@ def test_qwen3_full_shape_tolerance_mode(full):
     the tolerance mode is prefilled and run teacher-forced on the fixture's
     tokens, and its logits compared step by step with the exact mode's.  This
     random 28-layer model amplifies single-ulp attention differences.  Both
-    runs are deterministic; measured on MI355X: relative L2 of the logits
-    0.090-0.167 per step (mean 0.117; already 0.126 at step 0, from the
-    prefill) and the argmax equal on 89 of 128 steps.  The bounds sit ~20%
+    runs are deterministic; measured on MI355X: relative L2 of the logits up
+    to 0.164 per step (mean 0.117; about 0.126 at step 0 already, from the
+    prefill) and the argmax equal on 87 of 128 steps.  The bounds sit ~20%
     above the measured errors (every step <= 0.20, the mean <= 0.14) and ~10%
     below the measured agreement (at least 80 of 128 argmax equal); garbage
     attention lands near 1 and agrees on almost no step.  The free-running token prefix that matches the oracle
