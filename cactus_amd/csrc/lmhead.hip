@@ -10,6 +10,7 @@
 // FMA rate), and the LM head with the argmax (f16_argmax_kernel).
 #include "lm_device.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace cactus_hip {
@@ -395,9 +396,17 @@ static int launch_rows(const LmArgs& p, hipStream_t st) {
 
 template <int TM>
 static int launch_tile(const LmArgs& p, hipStream_t st) {
-    hipLaunchKernelGGL(f16_tile_kernel<TM>, dim3(ceil_div(p.N, 64) * ceil_div(p.M, 4 * TM)), dim3(LM_THREADS), 0, st,
-                       p.a, p.b, p.c, p.M, p.K, p.N);
-    return check_launch("matmul_f16");
+    // a launch holds fewer than 2^32 threads: 2^23 workgroups of rows at a time
+    const size_t cols = ceil_div(p.N, 64);
+    const size_t step = 4 * TM * std::max<size_t>(((size_t)1 << 23) / cols, 1);
+    for (size_t m0 = 0; m0 < (size_t)p.M; m0 += step) {
+        const int M = (int)std::min<size_t>(step, p.M - m0);
+        hipLaunchKernelGGL(f16_tile_kernel<TM>, dim3((unsigned)(cols * ceil_div(M, 4 * TM))), dim3(LM_THREADS), 0, st,
+                           p.a + m0 * p.K, p.b, p.c + m0 * p.N, M, p.K, p.N);
+        const int rc = check_launch("matmul_f16");
+        if (rc) return rc;
+    }
+    return CACTUS_HIP_OK;
 }
 
 }  // namespace cactus_hip

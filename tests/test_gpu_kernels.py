@@ -501,6 +501,26 @@ def test_matmul_f16_tiles(dev, orc, M, K, N):
     assert_bits(got, orc.matmul_f16(a, b), "matmul_f16")
 
 
+def test_matmul_f16_rows_beyond_a_launch(dev, orc):
+    """More row tiles than a launch holds: 2^28 + 5 rows of 8 values, zero
+    but for the first ones and those around the end of the first launch."""
+    M, K, N = (1 << 28) + 5, 8, 1
+    say("matmul_f16 beyond a launch", M, K, N)
+    rng = np.random.default_rng(28)
+    rows = f16(rng.normal(0, 1, (10, K)))
+    b = f16(rng.normal(0, 1, (N, K)))
+    a, c = dev.empty(M * K * 2), dev.empty(M * N * 2)
+    dev.cm.call("cactus_hip_memset", a.ptr, 0, M * K * 2, None)
+    dev.cm.call("cactus_hip_memset", c.ptr, 0x7E, M * N * 2, None)
+    for first in (0, M - 10):
+        dev.cm.call("cactus_hip_memcpy_h2d", a.ptr + first * K * 2, rows.ctypes.data, rows.nbytes, None)
+    dev.cm.call("cactus_hip_matmul_f16", a.ptr, dev.put(b), c.ptr, M, K, N, None)
+    want = orc.matmul_f16(rows, b)
+    for first in (0, M - 10):
+        assert_bits(dev.get_ptr(c.ptr + first * 2, np.uint16, (10, N)), want, "rows from %d" % first)
+    assert (dev.get_ptr(c.ptr + (M // 2) * 2, np.uint16, (64,)) == 0).all()
+
+
 def test_lm_head_argmax_qwen_vocab(dev, orc):
     say("lm_head_argmax K=1024 N=151936")
     rng = np.random.default_rng(6)
