@@ -284,23 +284,16 @@ __global__ void __launch_bounds__(64) value_tiles_kernel(AttnArgs a) { value_til
 // once, the same float as the reference's rounded multiply.  Block sums run
 // in the reference's sequential order in one lane per (query, block), from
 // the wave's weights in LDS.
-template <int NQ, int K>
-__device__ __forceinline__ void sq_step(float (&acc)[NQ][8], const float (&qv)[NQ], float k) {
-#pragma unroll
-    for (int q = 0; q < NQ; q++) fmac_row_bcast<K>(acc[q][K & 7], qv[q], k);
-}
-template <int NQ, int... K>
-__device__ __forceinline__ void sq_group16(float (&acc)[NQ][8], const float (&qv)[NQ], const float* kk,
-                                           std::integer_sequence<int, K...>) {
+template <int... K>
+__device__ __forceinline__ void sq_group16(float (&acc)[8], float qv, const float* kk, std::integer_sequence<int, K...>) {
     asm volatile("s_nop 1");   // DPP source read after a possible VALU write of qv
-    (sq_step<NQ, K>(acc, qv, kk[K]), ...);
+    (fmac_row_bcast<K>(acc[K & 7], qv, kk[K]), ...);
 }
 
-// the gq heads of a kv head in gq workgroups per chunk (hsplit)
+// the gq heads of a kv head in gq consecutive workgroups per chunk
 // (TILES: workgroups from tile_first on build value product tiles)
 template <bool HYBRID, int D, bool TILES = false>
 __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
-    constexpr int NQ = 1;                              // query vectors per wave
     const AttnArgs a = resolve(a_in);
     if constexpr (TILES) {
         if (blockIdx.x >= a.tile_first) {
@@ -308,49 +301,32 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
             return;
         }
     }
-    __shared__ float qsh[NQ][D];
-    __shared__ __align__(16) float wsh[NQ][64];
-    __shared__ float msh[NQ][2];
+    __shared__ float qsh[D];
+    __shared__ __align__(16) float wsh[64];
+    __shared__ float msh[2];
     const int lane = threadIdx.x;
-    // gq: the query heads of the kv head this workgroup takes (1 / hsplit of them)
-    const int hsp = a.hsplit > 1 ? a.hsplit : 1;
-    const int gq = a.gq / hsp, qr = NQ / gq;
-    const int ngrp = (a.S + qr - 1) / qr;
-    size_t gy = blockIdx.y;                            // (b, row group, kv head)
-    unsigned bx = blockIdx.x, nbx = gridDim.x;         // chunk, chunks (+ appender)
-    int hs = 0;                                        // head share of the split
-    if (a.xcd_chunks) {
-        const int L = blockIdx.x;
-        int j = L >> 3;
-        nbx = (unsigned)(a.xcd_chunks / hsp);
-        bx = (unsigned)(j % a.xcd_chunks);
-        hs = (int)(bx % (unsigned)hsp);
-        bx /= (unsigned)hsp;
-        j /= a.xcd_chunks;
-        const int kvx = (L & 7) + 8 * (j / a.xcd_rest);
-        if (kvx >= a.Hkv) return;                      // whole workgroup, before any barrier
-        gy = (size_t)(j % a.xcd_rest) * a.Hkv + kvx;
-    }
-    const int kvh = (int)(gy % a.Hkv);
-    gy /= a.Hkv;
-    const int qp0 = (int)(gy % ngrp) * qr;
-    const size_t b = gy / ngrp;
+    // workgroup -> (row, kv head, chunk, head), kv head h on XCD h % 8
+    int j = (int)blockIdx.x >> 3;
+    const unsigned nbx = (unsigned)(a.xcd_chunks / a.gq);         // chunks (+ appender)
+    unsigned bx = (unsigned)(j % a.xcd_chunks);
+    const int hs = (int)(bx % (unsigned)a.gq);
+    bx /= (unsigned)a.gq;
+    j /= a.xcd_chunks;
+    const int kvh = (int)(blockIdx.x & 7) + 8 * (j / a.xcd_rest);
+    if (kvh >= a.Hkv) return;                          // whole workgroup, before any barrier
+    const int qp = j % a.xcd_rest % a.S;
+    const size_t b = (size_t)(j % a.xcd_rest / a.S);
     const int d = a.d;
-    const int h0 = kvh * a.gq + hs * gq;
-    // per query vector: its row's key range (kv_start is 0 on this path)
+    const int h0 = kvh * a.gq + hs;
     const float NEG_INF = -__builtin_inff();
-    size_t kv_end_max = 0;
-    for (int r = 0; r < qr; r++) {
-        if (qp0 + r >= a.S) break;
-        size_t s0, e, bl;
-        kv_range<HYBRID>(a, (size_t)(qp0 + r), s0, e, bl);
-        if (e > kv_end_max) kv_end_max = e;
-    }
+    // the row's key range (kv_start is 0 on this path)
+    size_t kv_start, kv_end, blk_limit;
+    kv_range<HYBRID>(a, (size_t)qp, kv_start, kv_end, blk_limit);
     const size_t wbase = (size_t)bx * 64;              // first key of the wave
     const int jl = lane & 31;
     const size_t bs0 = wbase + (lane & 32);
     const size_t kp = wbase + lane;
-    const bool kload = kp < kv_end_max;
+    const bool kload = kp < kv_end;
     const bool kint8 = HYBRID && kp < a.cache_len;
     const int8_t* krow8 = nullptr;
     const uint16_t* krow16 = nullptr;
@@ -383,30 +359,28 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
     // get the reference's head RMSNorm and RoPE here (the step's attn_prep
     // arithmetic, kernel_attention.cpp:484-676); that chunk also appends the
     // new key and value to the INT8 cache (and the value's product tiles)
-    __shared__ uint16_t prow[NQ + 1][D];
-    __shared__ uint16_t pys[NQ + 1][D];
+    __shared__ uint16_t prow[2][D];
+    __shared__ uint16_t pys[2][D];
     __shared__ uint16_t krot[D];
-    __shared__ __align__(16) float nk_acc[NQ][8];
+    __shared__ __align__(16) float nk_acc[8];
     bool nk_lane = false;                               // the new key's accumulators come from nk_acc
     {
         if (a.prep.q_raw) {
             const bool appender = bx == nbx - 1;
             if (appender && hs != 0) return;               // one appender per kv head
-            if (!appender && wbase >= kv_end_max) return;   // one wave: no barrier waits for it
+            if (!appender && wbase >= kv_end) return;   // one wave: no barrier waits for it
             const int end8 = (d / 8) * 8, half = d / 2, vh = (half / 8) * 8;
             const uint32_t pos = (uint32_t)a.pos_off;
             const bool tab_ok = pos < a.prep.table_pos;
             const bool has_k = appender || (wbase <= a.cache_len && a.cache_len < wbase + 64);
-            const int nq = appender ? 0 : NQ;            // q rows of this workgroup
             // every operand of the rows' RMSNorm and RoPE is loaded up front
             constexpr int EPL = D / 64;                   // elements per lane of a row
-            uint16_t raw[NQ + 1][EPL], nwq[EPL], nwk[EPL];
+            uint16_t raw[2][EPL], nwq[EPL], nwk[EPL];
 #pragma unroll
             for (int e = 0; e < EPL; e++) {
                 const int i = lane + 64 * e;
-#pragma unroll
-                for (int r = 0; r < NQ; r++) raw[r][e] = nq ? a.prep.q_raw[(size_t)(h0 + r) * d + i] : (uint16_t)0;
-                raw[NQ][e] = has_k ? a.prep.k_raw[(size_t)kvh * d + i] : (uint16_t)0;
+                raw[0][e] = appender ? (uint16_t)0 : a.prep.q_raw[(size_t)h0 * d + i];
+                raw[1][e] = has_k ? a.prep.k_raw[(size_t)kvh * d + i] : (uint16_t)0;
                 nwq[e] = a.prep.q_norm[i];
                 nwk[e] = a.prep.k_norm[i];
             }
@@ -414,29 +388,29 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
             const uint16_t cv = lane < half ? a.prep.cos_t[trow + lane] : (uint16_t)0;
             const uint16_t sv = lane < half ? a.prep.sin_t[trow + lane] : (uint16_t)0;
             preload();   // (the appender too: no branch around loads)
-            // rows r < nq: q heads h0 + r; row NQ: the new key
+            // row 0: q head h0; row 1: the new key
 #pragma unroll
-            for (int r = 0; r <= NQ; r++)
+            for (int r = 0; r < 2; r++)
 #pragma unroll
                 for (int e = 0; e < EPL; e++) prow[r][lane + 64 * e] = raw[r][e];
             wave_lds_order();
-            // the NQ + 1 rows' statistics at once, one 16-lane row each (a
+            // the two rows' statistics at once, one 16-lane row each (a
             // row that is not prepared gets values that are never used)
-            float inv[NQ + 1];
-            uint16_t hinv[NQ + 1];
-            rms_stats_rows<D, NQ + 1>(&prow[0][0], D, a.prep.eps, inv, hinv);
+            float inv[2];
+            uint16_t hinv[2];
+            rms_stats_rows<D, 2>(&prow[0][0], D, a.prep.eps, inv, hinv);
 #pragma unroll
-            for (int r = 0; r <= NQ; r++)
+            for (int r = 0; r < 2; r++)
 #pragma unroll
                 for (int e = 0; e < EPL; e++) {
                     const int i = lane + 64 * e;
-                    pys[r][i] = rms_apply(raw[r][e], r < NQ ? nwq[e] : nwk[e], i, end8, inv[r], hinv[r]);
+                    pys[r][i] = rms_apply(raw[r][e], r == 0 ? nwq[e] : nwk[e], i, end8, inv[r], hinv[r]);
                 }
             wave_lds_order();
             // RoPE (kernel_attention.cpp:640-671): pair (i, i + d/2), lane i
 #pragma unroll
-            for (int r = 0; r <= NQ; r++) {
-                if (lane < half && ((r < nq) || (r == NQ && has_k))) {
+            for (int r = 0; r < 2; r++) {
+                if (lane < half && (r == 0 ? !appender : has_k)) {
                     const uint16_t x1 = pys[r][lane], x2 = pys[r][lane + half];
                     uint16_t o1, o2;
                     if (lane < vh) {
@@ -447,9 +421,9 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
                         o1 = f2h(fa * cf - fb * sf);
                         o2 = f2h(fb * cf + fa * sf);
                     }
-                    if (r < NQ) {
-                        qsh[r][lane] = tab_ok ? h2f(o1) : 0.0f;
-                        qsh[r][lane + half] = tab_ok ? h2f(o2) : 0.0f;
+                    if (r == 0) {
+                        qsh[lane] = tab_ok ? h2f(o1) : 0.0f;
+                        qsh[lane + half] = tab_ok ? h2f(o2) : 0.0f;
                     } else {
                         krot[lane] = o1;
                         krot[lane + half] = o2;
@@ -469,18 +443,16 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
                 }
                 return;
             }
-            // the new key's eight accumulators per query vector, lane
-            // 8 q + c running accumulator c of query q over dims 8 i + c in
-            // increasing i: the main loop's operands and order, one
-            // D/8-step chain per lane instead of the key lane's fp16 row read
-            // from LDS at every step of that loop
+            // the new key's eight accumulators, lane c running accumulator c
+            // over dims 8 i + c in increasing i: the main loop's operands and
+            // order, one D/8-step chain per lane instead of the key lane's
+            // fp16 row read from LDS at every step of that loop
             if (has_k) {
-                if (lane < 8 * NQ) {
-                    const int q = lane >> 3, c = lane & 7;
+                if (lane < 8) {
                     float s = 0.0f;
 #pragma unroll
-                    for (int i = 0; i < D / 8; i++) s = __builtin_fmaf(qsh[q][8 * i + c], h2f(krot[8 * i + c]), s);
-                    nk_acc[q][c] = s;
+                    for (int i = 0; i < D / 8; i++) s = __builtin_fmaf(qsh[8 * i + lane], h2f(krot[8 * i + lane]), s);
+                    nk_acc[lane] = s;
                 }
                 wave_lds_order();
                 nk_lane = kp == a.cache_len;
@@ -489,30 +461,22 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
     }
     if (!a.prep.q_raw) {
         preload();
-        for (int i = threadIdx.x; i < NQ * D; i += 64) {
-            const int v = i / D, dim = i % D;
-            const int qp = qp0 + v / gq;
-            qsh[v][dim] = qp < a.S ? h2f(a.q[((b * a.S + qp) * a.Hq + h0 + v % gq) * (size_t)d + dim]) : 0.0f;
-        }
+        for (int i = lane; i < D; i += 64) qsh[i] = h2f(a.q[((b * a.S + qp) * a.Hq + h0) * (size_t)d + i]);
     }
     __syncthreads();
-    if (wbase >= kv_end_max) return;                   // wave-uniform; no barrier follows
+    if (wbase >= kv_end) return;                   // wave-uniform; no barrier follows
 
-    // ---- dot products of this lane's key with every query vector
-    float acc[NQ][8];
+    // ---- dot product of this lane's key with the query vector
+    float acc[8];
 #pragma unroll
-    for (int q = 0; q < NQ; q++)
-#pragma unroll
-        for (int c = 0; c < 8; c++) acc[q][c] = 0.0f;
+    for (int c = 0; c < 8; c++) acc[c] = 0.0f;
     const int lr = lane & 15;
     // every step's query values in registers before the loop
     // (a read from LDS right before its step's FMAs would wait out the LDS
     // latency at each of the D/16 steps)
-    float qall[D / 16][NQ];
+    float qall[D / 16];
 #pragma unroll
-    for (int m = 0; m < D / 16; m++)
-#pragma unroll
-        for (int q = 0; q < NQ; q++) qall[m][q] = qsh[q][16 * m + lr];
+    for (int m = 0; m < D / 16; m++) qall[m] = qsh[16 * m + lr];
     auto conv_i8 = [](float (&kk)[16], const uint4 raw, const float s) {
         const float ns = -128.0f * s;
         const uint32_t w4[4] = {raw.x ^ 0x80808080u, raw.y ^ 0x80808080u, raw.z ^ 0x80808080u,
@@ -548,10 +512,7 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
                 for (int e = 0; e < 16; e++) kk[e] = 0.0f;
             }
         }
-        float qv[NQ];
-#pragma unroll
-        for (int q = 0; q < NQ; q++) qv[q] = qall[m][q];
-        sq_group16<NQ>(acc, qv, kk, std::make_integer_sequence<int, 16>{});
+        sq_group16(acc, qall[m], kk, std::make_integer_sequence<int, 16>{});
     };
     bool all_i8 = false;
     if constexpr (HYBRID) all_i8 = a.prep.q_raw != nullptr && a.qgs >= D;
@@ -562,42 +523,32 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
 #pragma unroll
         for (int m = 0; m < D / 16; m++) step(m, std::false_type{});
     }
-    {
-        if (__builtin_amdgcn_readfirstlane(__ballot(nk_lane) != 0ull ? 1 : 0)) {   // the new key's chunk only
-            typedef float f4v __attribute__((ext_vector_type(4)));
+    if (__builtin_amdgcn_readfirstlane(__ballot(nk_lane) != 0ull ? 1 : 0)) {   // the new key's chunk only
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(&nk_acc[0]);
+        const f32x4 hi = *reinterpret_cast<const f32x4*>(&nk_acc[4]);
 #pragma unroll
-            for (int q = 0; q < NQ; q++) {
-                const f4v lo = *reinterpret_cast<const f4v*>(&nk_acc[q][0]);
-                const f4v hi = *reinterpret_cast<const f4v*>(&nk_acc[q][4]);
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    acc[q][c] = nk_lane ? lo[c] : acc[q][c];
-                    acc[q][c + 4] = nk_lane ? hi[c] : acc[q][c + 4];
-                }
-            }
+        for (int c = 0; c < 4; c++) {
+            acc[c] = nk_lane ? lo[c] : acc[c];
+            acc[c + 4] = nk_lane ? hi[c] : acc[c + 4];
         }
     }
 
-    // ---- per query vector: mask, block max, weight, stores
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        const int qp = qp0 + q / gq;
-        const bool row_ok = qp < a.S;
-        const size_t aq = a.pos_off + qp;
-        size_t s0 = 0, kv_end = 0, blk_limit = 0;
-        if (row_ok) kv_range<HYBRID>(a, (size_t)qp, s0, kv_end, blk_limit);
-        const bool block_live = row_ok && bs0 < kv_end;
+    // ---- mask, block max, weight, stores
+    const size_t aq = a.pos_off + qp;
+    const bool is_decode = (!HYBRID) && (qp == a.S - 1) && a.S > 1;
+    const size_t row = (b * a.S + qp) * a.Hq + h0;
+    {
+        const bool block_live = bs0 < kv_end;
         const size_t be = block_live ? ((bs0 + ATT_BLOCK < blk_limit) ? bs0 + ATT_BLOCK : blk_limit) : bs0;
         const int bsz = (int)(be - bs0);
-        const bool is_decode = (!HYBRID) && (qp == a.S - 1) && a.S > 1;
         const bool block_skipped = !HYBRID && !is_decode && a.causal && bs0 > aq;
         const bool in_block = block_live && jl < bsz && !block_skipped;
         bool computed = in_block;
         if (computed && a.causal && kp > aq && (HYBRID || !is_decode)) computed = false;
         float sc = NEG_INF;
         if (computed) {
-            const float t0 = acc[q][0] + acc[q][4], t1 = acc[q][1] + acc[q][5];
-            const float t2 = acc[q][2] + acc[q][6], t3 = acc[q][3] + acc[q][7];
+            const float t0 = acc[0] + acc[4], t1 = acc[1] + acc[5];
+            const float t2 = acc[2] + acc[6], t3 = acc[3] + acc[7];
             sc = ((t0 + t1) + (t2 + t3)) * a.scale;
             if (!HYBRID) {
                 if (a.causal && kp > aq) sc = NEG_INF;
@@ -611,59 +562,45 @@ __global__ void __launch_bounds__(64) attn_scores_row_kernel(AttnArgs a_in) {
             if (jl < vs4) w = poly_exp_weight(sc, mx);
             else w = (sc != NEG_INF) ? cactus_expf(sc - mx) : 0.0f;
         }
-        const bool wlane = block_live && jl < bsz;
-        const size_t row = (b * a.S + (row_ok ? qp : 0)) * a.Hq + h0 + q % gq;
-        if (wlane) a.w[row * a.wstride + kp] = w;
-        wsh[q][lane] = w;
-        if (jl == 0) msh[q][lane >> 5] = mx;
+        if (block_live && jl < bsz) a.w[row * a.wstride + kp] = w;
+        wsh[lane] = w;
+        if (jl == 0) msh[lane >> 5] = mx;
     }
     wave_lds_order();
-    // ---- block sums, one lane per (query vector, block), reference order
-    if (lane < 2 * NQ) {
-        const int q = lane >> 1, half = lane & 1;
-        const int qp = qp0 + q / gq;
-        const size_t bs = wbase + 32 * half;
-        if (qp < a.S) {
-            const size_t aq = a.pos_off + qp;
-            size_t s0, kv_end, blk_limit;
-            kv_range<HYBRID>(a, (size_t)qp, s0, kv_end, blk_limit);
-            if (bs < kv_end) {
-                const size_t be = (bs + ATT_BLOCK < blk_limit) ? bs + ATT_BLOCK : blk_limit;
-                const int bsz = (int)(be - bs);
-                const bool is_decode = (!HYBRID) && (qp == a.S - 1) && a.S > 1;
-                const bool block_skipped = !HYBRID && !is_decode && a.causal && bs > aq;
-                // the block's 32 weights by eight 16-byte reads first (the slots
-                // past bsz hold other keys' weights or stale values; they are
-                // selected out), then the fold in the reference's order
-                typedef float f4v __attribute__((ext_vector_type(4)));
-                const f4v* x4 = reinterpret_cast<const f4v*>(&wsh[q][32 * half]);
-                float x[32];
+    // ---- block sums, one lane per block, reference order
+    const size_t bs = wbase + 32 * lane;
+    if (lane < 2 && bs < kv_end) {
+        const size_t be = (bs + ATT_BLOCK < blk_limit) ? bs + ATT_BLOCK : blk_limit;
+        const int bsz = (int)(be - bs);
+        const bool block_skipped = !HYBRID && !is_decode && a.causal && bs > aq;
+        // the block's 32 weights by eight 16-byte reads first (the slots
+        // past bsz hold other keys' weights or stale values; they are
+        // selected out), then the fold in the reference's order
+        const f32x4* x4 = reinterpret_cast<const f32x4*>(&wsh[32 * lane]);
+        float x[32];
 #pragma unroll
-                for (int t = 0; t < 8; t++) {
-                    const f4v v = x4[t];
-                    x[4 * t] = v.x; x[4 * t + 1] = v.y; x[4 * t + 2] = v.z; x[4 * t + 3] = v.w;
-                }
-                const int v4 = HYBRID ? 0 : (bsz / 4) * 4;
-                float sum = 0.0f;
-                bool has_zero = false;
-#pragma unroll
-                for (int j = 0; j < 32; j += 4) {
-                    if (!HYBRID && j < v4) {
-                        sum = sum + ((x[j] + x[j + 1]) + (x[j + 2] + x[j + 3]));
-                    } else {
-#pragma unroll
-                        for (int u = 0; u < 4; u++) sum = j + u < bsz ? sum + x[j + u] : sum;
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; u++) has_zero |= j + u < bsz && !(x[j + u] != 0.0f);
-                }
-                const size_t row = (b * a.S + qp) * a.Hq + h0 + q % gq;
-                const int blk = (int)(bs / ATT_BLOCK);
-                a.bmax[row * a.nbstride + blk] = block_skipped ? NEG_INF : msh[q][half];
-                const float bsv = block_skipped ? 0.0f : sum;
-                a.bsum[row * a.nbstride + blk] = has_zero ? set_sign(bsv) : bsv;
-            }
+        for (int t = 0; t < 8; t++) {
+            const f32x4 v = x4[t];
+            x[4 * t] = v.x; x[4 * t + 1] = v.y; x[4 * t + 2] = v.z; x[4 * t + 3] = v.w;
         }
+        const int v4 = HYBRID ? 0 : (bsz / 4) * 4;
+        float sum = 0.0f;
+        bool has_zero = false;
+#pragma unroll
+        for (int j = 0; j < 32; j += 4) {
+            if (!HYBRID && j < v4) {
+                sum = sum + ((x[j] + x[j + 1]) + (x[j + 2] + x[j + 3]));
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; u++) sum = j + u < bsz ? sum + x[j + u] : sum;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) has_zero |= j + u < bsz && !(x[j + u] != 0.0f);
+        }
+        const int blk = (int)(bs / ATT_BLOCK);
+        a.bmax[row * a.nbstride + blk] = block_skipped ? NEG_INF : msh[lane];
+        const float bsv = block_skipped ? 0.0f : sum;
+        a.bsum[row * a.nbstride + blk] = has_zero ? set_sign(bsv) : bsv;
     }
 }
 
@@ -2127,9 +2064,8 @@ static int launch_attention(AttnArgs a, void* stream) {
         // (consecutive, so on one XCD: all but the first read the key rows
         // from its L2), so a wave's dot and weight work is one head's (with
         // 8 heads per kv head in one wave the whole call took 35 us at 64 keys)
-        a.hsplit = a.gq;
-        a.xcd_chunks = (int)(chunks + (a.prep.q_raw ? 1 : 0)) * a.hsplit;
-        a.xcd_rest = a.B * a.S;                          // row groups of one row, one head
+        a.xcd_chunks = (int)(chunks + (a.prep.q_raw ? 1 : 0)) * a.gq;
+        a.xcd_rest = a.B * a.S;
         const size_t nwg = 8 * (size_t)((a.Hkv + 7) / 8) * a.xcd_chunks * a.xcd_rest;
         CH_REQUIRE(nwg < (1u << 31), "attention: decode key range too long");
         auto go = [&](auto kern, size_t n) { hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64), 0, as_stream(stream), a); };

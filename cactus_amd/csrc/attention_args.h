@@ -42,14 +42,10 @@ struct AttnArgs {
     // decode scores that also build those tiles from the cache (vsh is then
     // scratch of the launch): the first of the workgroups that do, 0 = none
     unsigned tile_first;
-    // decode score grid mapped onto the XCDs (0: plain 2-D grid): workgroup
-    // i runs on XCD i % 8, kv head h's workgroups on XCD h % 8; xcd_chunks
-    // workgroups per (row group, kv head), xcd_rest row groups
+    // decode score grid mapped onto the XCDs: workgroup i runs on XCD i % 8,
+    // kv head h's workgroups on XCD h % 8; xcd_chunks workgroups per (row, kv
+    // head), those of one key chunk's gq heads consecutive, xcd_rest rows
     int xcd_chunks, xcd_rest;
-    // decode scores: the query heads of a kv head split over this many
-    // workgroups per key chunk (0 or 1: one workgroup takes all gq heads);
-    // the workgroups of one chunk are consecutive within xcd_chunks
-    int hsplit;
     // decode step with the head preparation fused into the scores (null
     // q_raw: q and the new key row come prepared in q and k): raw q / k / v
     // rows of the step, head RMSNorm weights, RoPE tables, and the cache
