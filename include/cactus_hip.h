@@ -203,8 +203,9 @@ int cactus_hip_attention_f16(const uint16_t* q, const uint16_t* k, const uint16_
  * later positions read k_new/v_new [B][new_len][Hkv][d] fp16. expf weights.
  * Calls of one or two rows of one batch over a cache keep fp32 products of its
  * values in scratch of the stream, up to 256 MiB (4 bytes per cached value, and
- * a quarter more for growth) until the stream is destroyed; where that memory
- * cannot be had they convert the cache as they go, to the same results. */
+ * a quarter more for growth) until the stream is destroyed (the default
+ * stream: until the process ends); where that memory cannot be had they convert
+ * the cache as they go, to the same results. */
 int cactus_hip_attention_hybrid_int8_fp16(const uint16_t* q, const int8_t* k_cached,
                                           const int8_t* v_cached, const float* k_scales,
                                           const float* v_scales, const uint16_t* k_new,
