@@ -1023,6 +1023,17 @@ __global__ void __launch_bounds__(64 * W, 2) attn_prefill_mfma_kernel(PrefillArg
                 const h16x4 v1 = *reinterpret_cast<const h16x4*>(&vt[buf][16 * db + lr][16 + 4 * lg]);
                 va[db] = (h16x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
             }
+            if (W * 16 * VB != PF_BV && t * PF_T + PF_T > blk_end) {
+                // keys past the block's end are staged for a later block: zero
+                // values here, so that what a later row holds (an infinity)
+                // stays out of this block's rows
+                const int rem = blk_end - t * PF_T - 4 * lg;
+#pragma unroll
+                for (int db = 0; db < ND; db++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++)
+                        if (16 * (j >> 2) + (j & 3) >= rem) va[db][j] = (_Float16)0.0f;
+            }
             __builtin_amdgcn_sched_barrier(0);
             float sc[VB][8], mx[VB];
 #pragma unroll

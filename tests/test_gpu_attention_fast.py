@@ -266,6 +266,30 @@ def test_attention_hybrid_prefill_fast(dev, orc, B, cache, new, Hq, Hkv, d, qmul
     print(f"[prefill fast] max abs error {err:.2e}", flush=True)
 
 
+def test_attention_hybrid_prefill_fast_later_infinity(dev):
+    """An infinite value in the first row of a later block of 128 query
+    vectors (row 64 of two heads per KV head), which shares a workgroup and a
+    key tile with the block before it, leaves the earlier rows' bits alone."""
+    say("attention_hybrid_prefill_fast, later infinity")
+    S, C, Hq, Hkv, d = 333, 2667, 16, 8, 128
+    r = np.random.RandomState(1)
+    half = lambda *s: (r.randint(-512, 513, s) / 256).astype(np.float16)
+    q, kn, vn = half(S, Hq, d), half(S, Hkv, d), half(S, Hkv, d)
+    kc, vc = (r.randint(-127, 128, (C, Hkv, d)).astype(np.int8) for _ in range(2))
+    ks, vs = ((r.randint(64, 256, (C, Hkv, 1)) / 16384).astype(np.float32) for _ in range(2))
+    out = []
+    for inf in (False, True):
+        v = vn.copy()
+        if inf:
+            v[64] = np.inf
+        o = dev.put(np.full(q.shape, 9.0, np.float16))
+        dev.cm.call("cactus_hip_attention_hybrid_int8_fp16_fast", *map(dev.put, (q, kc, vc, ks, vs, kn, v)), o, 1, S, C, S,
+                    Hq, Hkv, d, ctypes.c_float(1 / math.sqrt(d)), C, 1, 128, None)
+        out.append(dev.get_ptr(o, np.uint16, q.shape))
+    assert (out[0][:64] == out[1][:64]).all()
+    assert not np.isfinite(out[1][64:].view(np.float16)).any()
+
+
 def test_attention_hybrid_fast_without_keys(dev):
     """No cached and no new keys: zero rows, as from the exact entry point."""
     say("attention_hybrid_fast, no keys")
