@@ -29,8 +29,8 @@ __device__ __forceinline__ float row_scale_from_max(float m) {
 // hold a float per wave in LDS.  NT: the workgroup's threads where the kernel
 // fixes them: blockDim.x is one more dependent scalar load, from a cache line
 // of its own behind a launch's arguments (GEMV, us at M=1: INT8 K=640 N=1024
-// 4.48 -> 4.14, INT4 K=1024 N=2048 4.33 -> 4.01; M=2 INT8 K=640 N=1024 5.72 ->
-// 5.25; the one that loses is M=2 INT8 K=3072 N=1024, 8.7 -> 9.0).
+// 4.48 -> 4.14, INT4 K=1024 N=2048 4.33 -> 4.01; at M=2: INT8 K=640 N=1024
+// 5.72 -> 5.25, K=3072 8.62 -> 8.14).
 template <int NT = 0>
 __device__ __forceinline__ float block_max_abs_f16(const uint16_t* __restrict__ x, int K,
                                                    float* red) {
@@ -41,6 +41,8 @@ __device__ __forceinline__ float block_max_abs_f16(const uint16_t* __restrict__ 
     if ((((uintptr_t)x) & 15) == 0) {
         const int K8 = K / 8;
         const uint4* x4 = reinterpret_cast<const uint4*>(x);
+        // two loads in flight (K = 3072: one and a half per thread)
+#pragma unroll 2
         for (int i = tid; i < K8; i += nt) {
             uint4 u = x4[i];
             uint32_t w[4] = {u.x, u.y, u.z, u.w};
